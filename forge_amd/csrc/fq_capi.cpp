@@ -1067,11 +1067,8 @@ int fq_dequant_rows(uint32_t dtype, const void* w, float* out, int N, int K, voi
     if (e != hipSuccess) return hip_fail(e);
     const DevInfo di = device_info(dev);
     const int nblk = (K + g.be - 1) / g.be;
-    const int U = nblk * (g.be / 32);
-    const size_t total = (size_t)N * U;
-    int grid = (int)std::min<size_t>((total + 255) / 256, (size_t)di.cus * 16);
-    e = fq::launch_dequant((int)dtype, static_cast<const uint8_t*>(w), out, N, K, U,
-                           nblk * g.bb, grid, static_cast<hipStream_t>(stream));
+    e = fq::launch_dequant((int)dtype, static_cast<const uint8_t*>(w), out, N, K, nblk * g.bb,
+                           di.cus, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? FQ_OK : hip_fail(e);
 }
 

@@ -133,33 +133,6 @@ __device__ __forceinline__ float f16_ref(uint32_t h) {
     }
     return __builtin_bit_cast(float, (s << 31) | ((e + 112u) << 23) | (m << 13));
 }
-template <bool EXACT>
-__device__ __forceinline__ float f16(uint32_t h) {
-    if constexpr (EXACT) return f16_ref(h);
-    else return f16_hw(h);
-}
-
-__device__ __forceinline__ float ubyte(uint32_t w, int b) {
-    return (float)((w >> (8 * b)) & 0xFFu);
-}
-
-// Nibble unpack of 4 bytes: low nibbles to slots [lo, lo+4), high to [hi, hi+4).
-// The masks go through an opaque v_and so the compiler keeps the byte
-// extracts as v_cvt_f32_ubyte{0..3} instead of folding them into bfe + cvt.
-__device__ __forceinline__ uint32_t opaque_and(uint32_t a, uint32_t m) {
-    uint32_t r;
-    asm volatile("v_and_b32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(m));
-    return r;
-}
-__device__ __forceinline__ void nibbles(uint32_t w, float* q, int lo, int hi) {
-    uint32_t l = opaque_and(w, 0x0F0F0F0Fu), h = opaque_and(w >> 4, 0x0F0F0F0Fu);
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        q[lo + b] = ubyte(l, b);
-        q[hi + b] = ubyte(h, b);
-    }
-}
-
 template <int F>
 struct Fmt;
 
@@ -177,18 +150,6 @@ struct Fmt<Q4_0> {
         const uint8_t* p = row + 18 * u;
         return Raw{ldg16<NT>(p), ldg128<NT>(p + 2)};
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int, float* q, float* A, float* B) {
-        float d = f16<EXACT>(r.d);
-        nibbles(r.qs.x, q, 0, 16);
-        nibbles(r.qs.y, q, 4, 20);
-        nibbles(r.qs.z, q, 8, 24);
-        nibbles(r.qs.w, q, 12, 28);
-        A[0] = d;
-        B[0] = -8.0f * d;
-    }
-    // Bit-exact dequantized value of a slot (reference expression order).
-    __device__ static float value(float q, float A, float) { return (q - 8.0f) * A; }
 };
 
 // ---------------------------------------------------------------- Q4_1 (20 B)
@@ -205,17 +166,6 @@ struct Fmt<Q4_1> {
         const uint8_t* p = row + 20 * u;
         return Raw{ldg32<NT>(p), ldg128<NT>(p + 4)};
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int, float* q, float* A, float* B) {
-        nibbles(r.qs.x, q, 0, 16);
-        nibbles(r.qs.y, q, 4, 20);
-        nibbles(r.qs.z, q, 8, 24);
-        nibbles(r.qs.w, q, 12, 28);
-        A[0] = f16<EXACT>(r.dm & 0xFFFFu);
-        B[0] = f16<EXACT>(r.dm >> 16);
-    }
-    // q*d is exact, so the fused form rounds exactly like q*d + m.
-    __device__ static float value(float q, float A, float B) { return __builtin_fmaf(q, A, B); }
 };
 
 // ---------------------------------------------------------------- Q8_0 (34 B)
@@ -232,20 +182,6 @@ struct Fmt<Q8_0> {
         const uint8_t* p = row + 34 * u;
         return Raw{ldg16<NT>(p), ldg128<NT>(p + 2), ldg128<NT>(p + 18)};
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int, float* q, float* A, float* B) {
-        const uint32_t v[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            uint32_t b = v[i] ^ 0x80808080u;  // int8 q -> unsigned q + 128
-#pragma unroll
-            for (int j = 0; j < 4; ++j) q[4 * i + j] = ubyte(b, j);
-        }
-        float d = f16<EXACT>(r.d);
-        A[0] = d;
-        B[0] = -128.0f * d;
-    }
-    __device__ static float value(float q, float A, float) { return (q - 128.0f) * A; }
 };
 
 // --------------------------------------------------------------- Q4_K (144 B)
@@ -288,22 +224,6 @@ struct Fmt<Q4_K> {
             mb = ((a8 >> 12) & 0xFu) | (((a4 >> 14) & 3u) << 4);
         }
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int u, float* q, float* A, float* B) {
-        nibbles(r.qs.x, q, 0, 16);
-        nibbles(r.qs.y, q, 4, 20);
-        nibbles(r.qs.z, q, 8, 24);
-        nibbles(r.qs.w, q, 12, 28);
-        float d = f16<EXACT>(r.hdr.x & 0xFFFFu), dmin = f16<EXACT>(r.hdr.x >> 16);
-        uint32_t sa, ma, sb, mb;
-        scale_min(r.hdr, (u & 7) >> 1, sa, ma, sb, mb);
-        A[0] = d * (float)sa;
-        B[0] = -(dmin * (float)ma);
-        A[1] = d * (float)sb;
-        B[1] = -(dmin * (float)mb);
-    }
-    // (d*sc)*q is exact, so fma(A, q, -dmin*m) rounds like d1*q - m1.
-    __device__ static float value(float q, float A, float B) { return __builtin_fmaf(A, q, B); }
 };
 
 // --------------------------------------------------------------- Q6_K (210 B)
@@ -329,37 +249,6 @@ struct Fmt<Q6_K> {
                    ldg64<NT>(p + 128 + 32 * n + l0), ldg64<NT>(p + 192 + 8 * n),
                    ldg16<NT>(p + 208)};
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int u, float* q, float* A, float* B) {
-        const uint32_t a[2] = {r.ql_lo.x, r.ql_lo.y}, b[2] = {r.ql_hi.x, r.ql_hi.y},
-                       h[2] = {r.qh.x, r.qh.y};
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            uint32_t q1 = (a[i] & 0x0F0F0F0Fu) | ((h[i] & 0x03030303u) << 4);
-            uint32_t q2 = (b[i] & 0x0F0F0F0Fu) | ((h[i] & 0x0C0C0C0Cu) << 2);
-            uint32_t q3 = ((a[i] >> 4) & 0x0F0F0F0Fu) | (h[i] & 0x30303030u);
-            uint32_t q4 = ((b[i] >> 4) & 0x0F0F0F0Fu) | ((h[i] >> 2) & 0x30303030u);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                q[0 + 4 * i + e] = ubyte(q1, e);
-                q[8 + 4 * i + e] = ubyte(q2, e);
-                q[16 + 4 * i + e] = ubyte(q3, e);
-                q[24 + 4 * i + e] = ubyte(q4, e);
-            }
-        }
-        float d = f16<EXACT>(r.d);
-        int is = (u & 3) >> 1;  // l/16 for l in [8c, 8c+8)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            int t = is + 2 * g;  // sc[8n + is + 2g]
-            uint32_t word = t < 4 ? r.sc.x : r.sc.y;
-            int sc = (int)(int8_t)((word >> (8 * (t & 3))) & 0xFFu);
-            A[g] = d * (float)sc;
-            B[g] = -32.0f * A[g];
-        }
-    }
-    // (d*sc) exact; one rounding of (d*sc)*(q-32), as the reference.
-    __device__ static float value(float q, float A, float) { return A * (q - 32.0f); }
 };
 
 
@@ -411,24 +300,6 @@ struct Fmt<Q5_0> {
         lo = five_bit(w & 0x0F0F0F0Fu, qh >> (4 * i));
         hi = five_bit((w >> 4) & 0x0F0F0F0Fu, qh >> (16 + 4 * i));
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int, float* q, float* A, float* B) {
-        const uint32_t w[4] = {r.qs.x, r.qs.y, r.qs.z, r.qs.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t lo, hi;
-            codes(w[i], r.qh, i, lo, hi);
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                q[4 * i + b] = ubyte(lo, b);
-                q[16 + 4 * i + b] = ubyte(hi, b);
-            }
-        }
-        const float d = f16<EXACT>(r.d);
-        A[0] = d;
-        B[0] = -16.0f * d;
-    }
-    __device__ static float value(float q, float A, float) { return (q - 16.0f) * A; }
 };
 
 // ---------------------------------------------------------------- Q5_1 (24 B)
@@ -446,24 +317,6 @@ struct Fmt<Q5_1> {
         const uint8_t* p = row + 24 * u;
         return Raw{ldg32<NT>(p), ldg32<NT>(p + 4), ldg128<NT>(p + 8)};
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int, float* q, float* A, float* B) {
-        const uint32_t w[4] = {r.qs.x, r.qs.y, r.qs.z, r.qs.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t lo, hi;
-            Fmt<Q5_0>::codes(w[i], r.qh, i, lo, hi);
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                q[4 * i + b] = ubyte(lo, b);
-                q[16 + 4 * i + b] = ubyte(hi, b);
-            }
-        }
-        A[0] = f16<EXACT>(r.dm & 0xFFFFu);
-        B[0] = f16<EXACT>(r.dm >> 16);
-    }
-    // q*d is exact (5 x 11 bits), so the fused form rounds like q*d + m.
-    __device__ static float value(float q, float A, float B) { return __builtin_fmaf(q, A, B); }
 };
 
 // -------------------------------------------------------------- IQ4_NL (18 B)
@@ -481,22 +334,6 @@ struct Fmt<IQ4_NL> {
         const uint8_t* p = row + 18 * u;
         return Raw{ldg16<NT>(p), ldg128<NT>(p + 2)};
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int, float* q, float* A, float* B) {
-        const uint32_t w[4] = {r.qs.x, r.qs.y, r.qs.z, r.qs.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t lo = iq4_lookup(w[i]), hi = iq4_lookup(w[i] >> 4);
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                q[4 * i + b] = (float)(int8_t)(lo >> (8 * b));
-                q[16 + 4 * i + b] = (float)(int8_t)(hi >> (8 * b));
-            }
-        }
-        A[0] = f16<EXACT>(r.d);
-        B[0] = 0.0f;
-    }
-    __device__ static float value(float q, float A, float) { return A * q; }
 };
 
 // --------------------------------------------------------------- Q3_K (110 B)
@@ -540,26 +377,6 @@ struct Fmt<Q3_K> {
         const uint32_t q = i ? r.qs.y : r.qs.x, h = i ? r.hm.y : r.hm.x;
         return ((q >> (2 * g)) & 0x03030303u) | (((h >> (4 * n + g)) & 0x01010101u) << 2);
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int u, float* q, float* A, float* B) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const uint32_t c = codes(r, u, g, i);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) q[8 * g + 4 * i + e] = ubyte(c, e);
-            }
-        int sc[4];
-        scales(r, u, sc);
-        const float d = f16<EXACT>(r.d);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            A[g] = d * (float)sc[g];
-            B[g] = -4.0f * A[g];
-        }
-    }
-    __device__ static float value(float q, float A, float) { return A * (q - 4.0f); }
 };
 
 // --------------------------------------------------------------- Q5_K (176 B)
@@ -588,28 +405,6 @@ struct Fmt<Q5_K> {
         lo = (w & 0x0F0F0F0Fu) | (((h >> (2 * g)) & 0x01010101u) << 4);
         hi = ((w >> 4) & 0x0F0F0F0Fu) | (((h >> (2 * g + 1)) & 0x01010101u) << 4);
     }
-    template <bool EXACT>
-    __device__ static void decode(const Raw& r, int u, float* q, float* A, float* B) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t lo, hi;
-            codes(r, u, i, lo, hi);
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                q[4 * i + b] = ubyte(lo, b);
-                q[16 + 4 * i + b] = ubyte(hi, b);
-            }
-        }
-        const float d = f16<EXACT>(r.hdr.x & 0xFFFFu), dmin = f16<EXACT>(r.hdr.x >> 16);
-        uint32_t sa, ma, sb, mb;
-        Fmt<Q4_K>::scale_min(r.hdr, (u & 7) >> 1, sa, ma, sb, mb);
-        A[0] = d * (float)sa;
-        B[0] = -(dmin * (float)ma);
-        A[1] = d * (float)sb;
-        B[1] = -(dmin * (float)mb);
-    }
-    // (d*sc)*q is exact (11 + 6 + 5 bits), so fma rounds like d1*q - m1.
-    __device__ static float value(float q, float A, float B) { return __builtin_fmaf(A, q, B); }
 };
 
 // ---------------------------------------------------------------- int8 limbs

@@ -134,7 +134,7 @@ hipError_t launch_q6c(const uint8_t* w, int N, int K, int64_t row_bytes, uint8_t
                       hipStream_t st);
 hipError_t launch_mmqp(int dtype, const MmqArgs& a, int splits, hipStream_t st);
 hipError_t launch_reduce(const MmqArgs& a, int splits, hipStream_t st);
-hipError_t launch_dequant(int dtype, const uint8_t* w, float* out, int N, int K, int U,
-                          int row_bytes, int grid, hipStream_t st);
+hipError_t launch_dequant(int dtype, const uint8_t* w, float* out, int N, int K, int row_bytes,
+                          int cus, hipStream_t st);
 
 }  // namespace fq
