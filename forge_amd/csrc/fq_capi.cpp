@@ -242,7 +242,8 @@ MmqpPlan plan_mmqp(int M, int K, int N, int cus, bool q6k = false) {
     }
     p.xop_b = (size_t)Tn * K * 64 * 2;
     p.ex_b = (size_t)M * 4;
-    p.sum_b = (size_t)Tn * 32 * K / 32 * 4;  // sub-block sums (formats with a min term)
+    // sub-block sums (formats with a min term): floats, or mmqk's hi + lo
+    p.sum_b = (size_t)Tn * std::max<size_t>((size_t)K * 4, fq::mmqk_sum_bytes(K));
     p.part_b = p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
     p.q6c_b = q6k ? (size_t)fq::mmqp_q6c_bytes(N, K) : 0;  // Q6_K rows as 36-byte blocks
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
@@ -670,7 +671,13 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
     }
 
     const bool q6k = dtype == FQ_DTYPE_Q6_K;
-    if (fq::mmqp_supported((int)dtype) && M > 32 && K > 0 && K % 256 == 0 &&
+    const bool mmqk = fq::mmqk_supported((int)dtype);
+    // (Q5_K in a fixed workspace that its K-splits here do not fit, 2040 x
+    // 256 x 4096 for instance, runs on the fp16 MFMA kernel below, whose
+    // plan may)
+    const bool fits = !(fixed && dtype == FQ_DTYPE_Q5_K && K % 256 == 0) ||
+                      plan_mmqp(M, K, N, di.cus).total <= fixed_cap;
+    if (fits && (mmqk || fq::mmqp_supported((int)dtype)) && M > 32 && K > 0 && K % 256 == 0 &&
         (q6k || (reinterpret_cast<uintptr_t>(w) & 15) == 0) &&
         (int64_t)N * (q6k ? fq::mmqp_q6c_bytes(1, K) : (K / g.be) * g.bb) < ((int64_t)1 << 32)) {
         // prefill, rows that are whole 16-byte chunks (K a multiple of 256,
@@ -704,7 +711,7 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
         }
         a.xop = buf;
         a.ex = reinterpret_cast<const int*>(buf + al(xop_b));
-        a.xsum = dtype == FQ_DTYPE_Q4_K || dtype == FQ_DTYPE_Q4_1 || dtype == FQ_DTYPE_Q5_1
+        a.xsum = mmqk || dtype == FQ_DTYPE_Q4_1 || dtype == FQ_DTYPE_Q5_1
                      ? reinterpret_cast<const float*>(buf + al(xop_b) + al(ex_b))
                                : nullptr;
         a.part = splits > 1 ? reinterpret_cast<float*>(buf + al(xop_b) + al(ex_b) + al(sum_b))
@@ -716,10 +723,13 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
         a.M = M;
         a.N = N;
         a.K = K;
+        float* const sums = const_cast<float*>(a.xsum);
         e = fq::launch_xprep32(x, M, K, reinterpret_cast<_Float16*>(buf),
-                               const_cast<int*>(a.ex), const_cast<float*>(a.xsum), q6k, st);
+                               const_cast<int*>(a.ex), mmqk ? nullptr : sums,
+                               mmqk ? reinterpret_cast<_Float16*>(sums) : nullptr, q6k, st);
         if (e != hipSuccess) return hip_fail(e);
-        e = fq::launch_mmqp((int)dtype, a, splits, st);
+        e = mmqk ? fq::launch_mmqk((int)dtype, a, splits, st)
+                 : fq::launch_mmqp((int)dtype, a, splits, st);
         if (e == hipSuccess && splits > 1) e = fq::launch_reduce(a, splits, st);
         return e == hipSuccess ? FQ_OK : hip_fail(e);
     }

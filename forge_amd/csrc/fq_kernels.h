@@ -125,8 +125,15 @@ int mmqp_tile_rows();    // rows per work-group tile
 int mmqp_tile_tokens();  // tokens per work-group tile
 // sub16: the operand order of the Q6_K kernel (each 16-element quarter one
 // sub-block)
+// xsum / xsum2 (either may be null): the sub-block sums as floats, or in
+// mmqk's fp16 hi + lo
 hipError_t launch_xprep32(const float* x, int M, int K, _Float16* xop, int* ex, float* xsum,
-                          bool sub16, hipStream_t st);
+                          _Float16* xsum2, bool sub16, hipStream_t st);
+// the same for Q4_K and Q5_K with the sub-block scales in the weight operand
+// (fq_mmqk.hip): a.xsum holds the hi + lo sums (mmqk_sum_bytes per 32 tokens)
+bool mmqk_supported(int dtype);
+size_t mmqk_sum_bytes(int K);
+hipError_t launch_mmqk(int dtype, const MmqArgs& a, int splits, hipStream_t st);
 // Q6_K: the kernel reads 36-byte blocks that launch_q6c writes from the GGUF
 // rows (mmqp_q6c_bytes(N, K) bytes, 16-byte aligned)
 int64_t mmqp_q6c_bytes(int N, int K);

@@ -1,10 +1,10 @@
-// fq_mmqp.hip -- prefill (M > 32 tokens) for Q8_0, Q4_0, Q4_1, Q5_0, Q5_1,
-// Q4_K and Q6_K on v_mfma_f32_32x32x16_f16.
+// fq_mmqp.hip -- prefill (M > 32 tokens) for Q8_0, Q4_0, Q4_1, Q5_0, Q5_1
+// and Q6_K on v_mfma_f32_32x32x16_f16 (Q4_K and Q5_K: fq_mmqk.hip).
 //
 //   D[token][n] = X[token][k] . W[n][k]^T on the fp16 matrix cores, with the
 // tokens as x 2^-e(token) in fp16 hi + lo and the weights' integer codes
 // exact in fp16; one FMA per output and 32-element block folds in the block
-// scale, and the formats with a per-block minimum (Q4_1, Q4_K) add it as an
+// scale, and the formats with a per-block minimum (Q4_1, Q5_1) add it as an
 // fp32 outer product (mmqp_kernel below).
 //
 // Token prep is one launch (xprep4_kernel): the per-token exponent, then the
@@ -54,7 +54,8 @@ template <bool SUB16>
 __global__ __launch_bounds__(1024) void xprep4_kernel(const float* __restrict__ x, int M, int K,
                                                       int* __restrict__ ex,
                                                       _Float16* __restrict__ xop,
-                                                      float* __restrict__ xsum) {
+                                                      float* __restrict__ xsum,
+                                                      _Float16* __restrict__ xsum2) {
     __shared__ float wmax[16][4];
     __shared__ int es[4];
     const int tid = threadIdx.x, t = tid & 3;
@@ -123,13 +124,25 @@ __global__ __launch_bounds__(1024) void xprep4_kernel(const float* __restrict__ 
         _Float16* dst = xop + ((size_t)T * KQ + kq) * XT + (lm + 32 * g) * 8;
         *reinterpret_cast<h8*>(dst) = hi;
         *reinterpret_cast<h8*>(dst + 512) = lo;
-        if (xsum) {
+        if (xsum || xsum2) {
             // the token's sum of x 2^-e over its 32-element sub-block kq / 2:
             // pieces p, p ^ 4, p ^ 8, p ^ 12 of one wave, added in a fixed tree
             float t8 = ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
             t8 += __shfl_xor(t8, 4, 64);
             t8 += __shfl_xor(t8, 8, 64);
-            if ((p & 12) == 0) xsum[((size_t)T * (K / 32) + (kq >> 1)) * 32 + lm] = t8;
+            if ((p & 12) == 0) {
+                const int b = kq >> 1;  // sub-block
+                if (xsum) xsum[((size_t)T * (K / 32) + b) * 32 + lm] = t8;
+                if (xsum2) {
+                    // times 2^-5 (below 2^15) as fp16 hi + lo:
+                    // [super-block][hi, lo][token][sub-block of the super-block]
+                    const float v = t8 * 0x1p-5f;
+                    const _Float16 hi = (_Float16)v;
+                    _Float16* d = xsum2 + ((size_t)T * (K / 256) + (b >> 3)) * 512 + lm * 8 + (b & 7);
+                    d[0] = hi;
+                    d[256] = (_Float16)(v - (float)hi);
+                }
+            }
         }
     };
     // P is a multiple of 64: whole waves take part in each piece's shuffles
@@ -228,26 +241,6 @@ struct PB<Q5_1> {
     }
 };
 
-// Q4_K super-block (144 B, matmul.cpp:340-377): d @0, dmin @2, scales[12]
-// @4 (6-bit scale and min per 32-element sub-block), qs[128] @16.  A step
-// (64 elements) is sub-block pair p = s mod 4 of super-block s / 4: the
-// low nibbles of qs[32 p, 32 p + 32) are sub-block 2 p (block b = 0), the
-// high nibbles sub-block 2 p + 1 (b = 1).  Per row and step three 16-byte
-// chunks are copied, all aligned: the header and the pair's 32 code bytes.
-// Lane group g: bytes 16 g .. 16 g + 15 of the pair, nibble b; half h =
-// bytes 8 h .. 8 h + 7.  w = d sc q - dmin m: the min term goes through
-// the per-token sub-block sums of xprep4_kernel.
-template <>
-struct PB<Q4_K> {
-    static constexpr int CH = 3;
-    static constexpr bool MIN = true;
-    template <int B>
-    __device__ static void ops(const uint32_t (&q)[4], int, h8& b0, h8& b1) {
-        b0 = nib8(q[0], q[1], 4 * B, (_Float16)1024.0f);
-        b1 = nib8(q[2], q[3], 4 * B, (_Float16)1024.0f);
-    }
-};
-
 // Q6_K as converted by q6c_kernel (36-byte blocks of 32 elements): d @0,
 // the two sub-block scales int8 @2, @3, then the 32 six-bit codes q (0..63)
 // @4, stored so that lane group g's 16 bytes are elements 8 g .. 8 g + 7 of
@@ -277,35 +270,26 @@ struct Chunks {
     // step s0 + u starts (u SB) mod 16 bytes into its first chunk (s0 a
     // multiple of 4 and rows 16-byte aligned)
     static constexpr int o4(int u) { return u * PB<F>::SB & 15; }
-    __device__ static size_t off(int s, int) { return (size_t)s * PB<F>::SB & ~(size_t)15; }
+    __device__ static size_t off(int s) { return (size_t)s * PB<F>::SB & ~(size_t)15; }
 };
 template <>
 struct Chunks<Q6_K> {  // a step (72 bytes) starts 0 or 8 bytes into a chunk
     static constexpr int CH = 5;
     static constexpr int o4(int u) { return u * 72 & 15; }
-    __device__ static size_t off(int s, int) { return (size_t)s * 72 & ~(size_t)15; }
+    __device__ static size_t off(int s) { return (size_t)s * 72 & ~(size_t)15; }
 };
 template <>
 struct Chunks<Q5_1> {  // a step (48 bytes) starts on a chunk
     static constexpr int CH = 3;
     static constexpr int o4(int) { return 0; }
-    __device__ static size_t off(int s, int) { return (size_t)s * 48; }
+    __device__ static size_t off(int s) { return (size_t)s * 48; }
 };
 template <>
 struct Chunks<Q4_1> {  // a step (40 bytes) starts 0 or 8 bytes into a chunk
     static constexpr int CH = 3;
     static constexpr int o4(int u) { return u * 40 & 15; }
-    __device__ static size_t off(int s, int) { return (size_t)s * 40 & ~(size_t)15; }
+    __device__ static size_t off(int s) { return (size_t)s * 40 & ~(size_t)15; }
 };
-template <>
-struct Chunks<Q4_K> {
-    static constexpr int CH = 3;
-    static constexpr int o4(int u) { return 4 * u; }  // the pair index, as 4 p
-    __device__ static size_t off(int s, int p) {
-        return (size_t)144 * (s >> 2) + (p ? 32 * (s & 3) : 0);
-    }
-};
-
 // The 16 code bytes of lane group g of block b, for a row whose step starts
 // O4 bytes into its LDS slot (the slot holds the step's 16-byte chunks, so
 // O4 = (s SB) mod 16, a multiple of 4).  One or two aligned 16-byte reads
@@ -330,19 +314,11 @@ __device__ __forceinline__ void codes16(const uint8_t* row, int g, uint32_t (&q)
 }
 
 // The 16 code bytes of lane group g of block B and the block's scale and
-// minimum coefficient (d sc, dmin m; the minimum is 0 without a min term),
+// minimum coefficient (0 without a min term),
 // for a row slot whose step starts O4 bytes into its first chunk.
 template <int F, int O4, int B>
 __device__ __forceinline__ void codes(const uint8_t* row, int g, uint32_t (&q)[4]) {
-    if constexpr (F == Q4_K) {  // planes of BNT x 16 bytes: header, codes 0..15, codes 16..31
-        typedef const __attribute__((address_space(3))) fq_u32x4* lds_v4;
-        const fq_u32x4 v =
-            *reinterpret_cast<lds_v4>(reinterpret_cast<uintptr_t>(row + BNT * 16 * (1 + g)));
-        q[0] = v[0];
-        q[1] = v[1];
-        q[2] = v[2];
-        q[3] = v[3];
-    } else if constexpr (F == Q5_0 || F == Q5_1) {
+    if constexpr (F == Q5_0 || F == Q5_1) {
         uint32_t n[4];
         codes16<F, O4, B>(row, g, n);  // the 16 qs bytes
         const uint32_t qh = lds4_a2(row + O4 + PB<F>::BB * B + PB<F>::HOFF) >> (16 * g);
@@ -358,14 +334,7 @@ __device__ __forceinline__ void codes(const uint8_t* row, int g, uint32_t (&q)[4
 }
 template <int F, int O4, int B>
 __device__ __forceinline__ void scales(const uint8_t* row, float& db, float& mn) {
-    if constexpr (F == Q4_K) {
-        typedef const __attribute__((address_space(3))) fq_u32x4* lds_v4;
-        const fq_u32x4 h = *reinterpret_cast<lds_v4>(reinterpret_cast<uintptr_t>(row));
-        uint32_t sa, ma, sb, mb;
-        Fmt<Q4_K>::scale_min(uint4{h[0], h[1], h[2], h[3]}, O4 / 4, sa, ma, sb, mb);
-        db = f16_hw(h[0] & 0xFFFFu) * (float)(B ? sb : sa);
-        mn = f16_hw(h[0] >> 16) * (float)(B ? mb : ma);
-    } else if constexpr (F == Q6_K) {  // db = d sc1 and mn = sc0 / sc1 (sc1 = 0: d sc0, 1)
+    if constexpr (F == Q6_K) {  // db = d sc1 and mn = sc0 / sc1 (sc1 = 0: d sc0, 1)
         const uint32_t h = lds4_a2(row + O4 + PB<F>::BB * B);
         const float d = f16_hw(h & 0xFFFFu);
         const float s0 = (float)(int8_t)(h >> 16), s1 = (float)(int8_t)(h >> 24);
@@ -384,9 +353,7 @@ __device__ __forceinline__ void scales(const uint8_t* row, float& db, float& mn)
 template <int F>
 struct Tile {
     static constexpr int CH = Chunks<F>::CH;            // chunks per row and step
-    // Q8_0 / Q4_0: rows of CH chunks; Q4_K: CH planes of one chunk per row
-    static constexpr bool PLANES = F == Q4_K;
-    static constexpr int WROW = PLANES ? 16 : 16 * CH;  // LDS bytes between rows
+    static constexpr int WROW = 16 * CH;                // LDS bytes between rows
     static constexpr int WCH = BNT * CH;                // chunks of a step's weight tile
     static constexpr int WIN = WCH / 64;                // copy instructions per step (whole)
     static_assert(WCH % 64 == 0, "whole copy instructions");
@@ -411,7 +378,7 @@ struct Tile {
 //   B (16 k x 32 rows):   the block's integer codes, exact in fp16,
 //   D_b = A_hi B + A_lo B  (two MFMAs per 16 k, one fp32 result per block),
 //   acc += d_b(n) D_b      (one FMA per output and block),
-//   acc -= S_b(token) m_b(n) (Q4_1, Q4_K: v_mfma_f32_32x32x2_f32 over a
+//   acc -= S_b(token) m_b(n) (Q4_1, Q5_1: v_mfma_f32_32x32x2_f32 over a
 //                          step's two blocks, S_b the token's scaled sum),
 // y = 2^e(token) acc at the end.  Weights are the B operand so that a lane's
 // 16 results all belong to one row n: the block scale d_b(n) is one value
@@ -451,10 +418,7 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
 #pragma unroll
     for (int q = 0; q < TL::WI_HI; ++q) {
         const int L = min(64 * (NW * q + wave) + lane, TL::WCH - 1);
-        // row-major [row][CH] slots, or (PLANES) chunk-major [CH][row]: copy
-        // instruction k = NW q + wave is plane k / 4, wave-uniform
-        const int r = TL::PLANES ? L % BNT : L / TL::CH;
-        const int p = TL::PLANES ? L / BNT : L - r * TL::CH;
+        const int r = L / TL::CH, p = L - r * TL::CH;  // [row][CH] slots
         woff[q] = (uint32_t)min(n0 + r, a.N - 1) * (uint32_t)a.row_bytes + 16 * p;
     }
     // sub-block sums (min term): tile T, block wave & 1, lanes 0..7
@@ -481,8 +445,7 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
 #pragma unroll
         for (int q = 0; q < TL::WI_HI; ++q)
             if (q < nwi) {
-                const uint32_t so =
-                    (uint32_t)Chunks<F>::off(s, TL::PLANES ? (NW * q + wave) >> 2 : 0);
+                const uint32_t so = (uint32_t)Chunks<F>::off(s);
                 const uint32_t vo = F == Q5_0 ? min(woff[q], wend - so) : woff[q];
                 dma16s(vo, a.w + so, wl + NW * 1024 * q);
             }
@@ -749,7 +712,7 @@ __global__ __launch_bounds__(256) void q6c_kernel(const uint8_t* __restrict__ w,
 
 bool mmqp_supported(int dtype) {
     return dtype == Q8_0 || dtype == Q4_0 || dtype == Q4_1 || dtype == Q5_0 || dtype == Q5_1 ||
-           dtype == Q4_K || dtype == Q6_K;
+           dtype == Q6_K;
 }
 
 int64_t mmqp_q6c_bytes(int N, int K) { return (int64_t)N * (K / 32) * 36; }
@@ -765,14 +728,14 @@ int mmqp_tile_rows() { return BNT; }
 int mmqp_tile_tokens() { return BMT; }
 
 hipError_t launch_xprep32(const float* x, int M, int K, _Float16* xop, int* ex, float* xsum,
-                          bool sub16, hipStream_t st) {
+                          _Float16* xsum2, bool sub16, hipStream_t st) {
     if (K % 256 != 0) return hipErrorInvalidValue;
     if (sub16)
         hipLaunchKernelGGL(xprep4_kernel<true>, dim3(8 * ((M + 31) / 32)), dim3(1024), 0, st, x, M,
-                           K, ex, xop, xsum);
+                           K, ex, xop, xsum, xsum2);
     else
         hipLaunchKernelGGL(xprep4_kernel<false>, dim3(8 * ((M + 31) / 32)), dim3(1024), 0, st, x,
-                           M, K, ex, xop, xsum);
+                           M, K, ex, xop, xsum, xsum2);
     return hipGetLastError();
 }
 
@@ -791,8 +754,6 @@ hipError_t launch_mmqp(int dtype, const MmqArgs& a, int splits, hipStream_t st) 
         hipLaunchKernelGGL(mmqp_kernel<Q5_0>, grid, dim3(64 * NW), 0, st, a, sps);
     else if (dtype == Q5_1)
         hipLaunchKernelGGL(mmqp_kernel<Q5_1>, grid, dim3(64 * NW), 0, st, a, sps);
-    else if (dtype == Q4_K)
-        hipLaunchKernelGGL(mmqp_kernel<Q4_K>, grid, dim3(64 * NW), 0, st, a, sps);
     else if (dtype == Q6_K)
         hipLaunchKernelGGL(mmqp_kernel<Q6_K>, grid, dim3(64 * NW), 0, st, a, sps);
     else
