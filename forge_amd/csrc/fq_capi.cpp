@@ -209,45 +209,52 @@ size_t mmqs_need(int M, int K, int N, int cus, int mt) {
     return 256 + al(pl.xop_b) + al(pl.xsum_b) + al(pl.ex_b) + al(part_b);
 }
 
-// Workspace bytes and K-splits of the prefill kernel (M > 32, K a multiple
-// of 256): one work-group per CU and tile, K split when that
-// shortens the busiest CU's work, each split a multiple of four 64-element
-// steps.
+// Workspace bytes and K-splits of the prefill kernels (M > 32, K a multiple
+// of 256): one work-group per CU and tile, each split a multiple of four
+// 64-element steps.
 struct MmqpPlan {
     int splits;
     size_t xop_b, ex_b, sum_b, part_b, q6c_b, total;
 };
 
-MmqpPlan plan_mmqp(int M, int K, int N, int cus, bool q6k = false) {
+// tiles_n: work-groups along the rows, cols: columns of a partial slab,
+// q6_rows: Q6_K rows to rewrite (0: another format); cap: bytes the plan has
+// to fit where a smaller split count can (0: no limit).
+MmqpPlan plan_mmqp(int M, int K, long tiles_n, int cols, int q6_rows, int cus, size_t cap = 0) {
     MmqpPlan p{};
     const int Tn = (M + 31) / 32, nsteps = K / 64;
-    const int tn = fq::mmqp_tile_rows(), tm = fq::mmqp_tile_tokens();
-    const long tiles = (long)((N + tn - 1) / tn) * ((M + tm - 1) / tm);
-    // the split count with the fewest steps on the busiest CU (rounds of
-    // work-groups x steps per split), taken only when it saves at least a
-    // quarter of the unsplit count: every split adds a partial slab and its
-    // share of the reduce (14336 x 4096 x 512: 224 tiles run fastest
-    // unsplit, 4096 x 4096 x 512: 64 tiles with 4 splits)
-    const long cost1 = ((tiles + cus - 1) / cus) * nsteps;
-    long best = cost1;
-    p.splits = 1;
-    for (int sp = 2; sp <= std::min(16, nsteps / 4); ++sp) {
-        const int sps = ((nsteps + sp - 1) / sp + 3) & ~3;
-        const int eff = (nsteps + sps - 1) / sps;  // non-empty splits
-        const long cost = ((tiles * eff + cus - 1) / cus) * sps;
-        if (4 * cost <= 3 * cost1 && cost < best) {
-            best = cost;
-            p.splits = eff;
-        }
-    }
+    const int tm = fq::mmqp_tile_tokens();
+    const long tiles = tiles_n * ((M + tm - 1) / tm);
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     p.xop_b = (size_t)Tn * K * 64 * 2;
     p.ex_b = (size_t)M * 4;
     // sub-block sums (formats with a min term): floats, or mmqk's hi + lo
     p.sum_b = (size_t)Tn * std::max<size_t>((size_t)K * 4, fq::mmqk_sum_bytes(K));
-    p.part_b = p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
-    p.q6c_b = q6k ? (size_t)fq::mmqp_q6c_bytes(N, K) : 0;  // Q6_K rows as 36-byte blocks
-    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    p.total = 256 + al(p.xop_b) + al(p.ex_b) + al(p.sum_b) + al(p.part_b) + al(p.q6c_b);
+    p.q6c_b = (size_t)fq::mmqp_q6c_bytes(q6_rows, K);  // Q6_K rows as 36-byte blocks
+    const size_t fixed_b = 256 + al(p.xop_b) + al(p.ex_b) + al(p.sum_b) + al(p.q6c_b);
+    // The split count of the smallest estimated time: rounds of work-groups x
+    // (steps per split at 2.1 us, 3 us to fill the pipeline and store), and
+    // for a split the slab sum, a launch of 4 us and each slab written and
+    // read at 4 TB/s.  (Counting steps alone took 16 splits for a 14336-row
+    // gate/up pair at K = 4096, M = 77: 117 + 23 us against 80 + 7 with 2, and
+    // 8 for a 6144-row QKV at M = 512: 82 + 19 us against 72 + 8.)
+    double best = 0.0;
+    p.splits = 1;
+    for (int sp = 1; sp <= std::max(1, std::min(16, nsteps / 4)); ++sp) {
+        const int sps = ((nsteps + sp - 1) / sp + 3) & ~3;
+        const int eff = (nsteps + sps - 1) / sps;  // non-empty splits
+        if (eff != sp) continue;
+        const size_t part_b = sp > 1 ? (size_t)sp * M * cols * 4 : 0;
+        if (sp > 1 && cap && fixed_b + al(part_b) > cap) continue;
+        const double t = (double)((tiles * sp + cus - 1) / cus) * (2.1 * sps + 3.0) +
+                         (sp > 1 ? 4.0 + ((double)sp + 1.0) * M * cols * 4.0 / 4e6 : 0.0);
+        if (sp == 1 || t < best) {
+            best = t;
+            p.splits = sp;
+            p.part_b = part_b;
+        }
+    }
+    p.total = fixed_b + al(p.part_b);
     return p;
 }
 
@@ -292,6 +299,104 @@ int run_mmq(uint32_t dtype, const Geometry& g, const float* x, const void* w, co
         if (e != hipSuccess) return hip_fail(e);
     }
     e = fq::launch_mmq((int)dtype, a, pl.shape, pl.gx, pl.gy, pl.splits, st);
+    return e == hipSuccess ? FQ_OK : hip_fail(e);
+}
+
+// The matrices of one prefill call: fq::MM_ONE w[0]; fq::MM_PAIR the gate and
+// up matrices w[0], w[1] of n[0] rows each; fq::MM_CAT up to three whose
+// results are concatenated (empty ones last).
+struct Mats {
+    int mm;
+    const void* w[3];
+    int n[3];
+};
+
+// Prefill on v_mfma_f32_32x32x16_f16 (fq_mmqk.hip for Q4_K and Q5_K,
+// fq_mmqp.hip for the other formats): rows that are whole 16-byte chunks (K a
+// multiple of 256, 16-byte aligned weights, under 4 GiB of them: the copies
+// take 32-bit offsets): per-token operands, then one work-group per CU and
+// tile (K-split while the tiles leave CUs idle).  Q6_K rows are first
+// rewritten into 36-byte blocks in the workspace.  kNotTaken: another kernel
+// runs the call (several matrices: one call each, also where the workspace
+// cannot grow to this call's size under graph capture).
+constexpr int kNotTaken = -1;
+int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms,
+                const float* bias, int bias_mode, int64_t bias_len, float* y, int M, int K, int N,
+                int dev, const DevInfo& di, hipStream_t st, uint8_t* fixed, size_t fixed_cap) {
+    const bool q6k = dtype == FQ_DTYPE_Q6_K, mmqk = fq::mmqk_supported((int)dtype);
+    if (!(mmqk || fq::mmqp_supported((int)dtype)) || M <= 32 || K <= 0 || K % 256 != 0)
+        return kNotTaken;
+    const int64_t rb = q6k ? fq::mmqp_q6c_bytes(1, K) : (int64_t)(K / g.be) * g.bb;
+    int rows = 0;  // of all matrices
+    for (int i = 0; i < 3; ++i) {
+        const int n = ms.mm == fq::MM_PAIR && i < 2 ? ms.n[0] : ms.n[i];
+        if (n == 0) continue;
+        if ((!q6k && (reinterpret_cast<uintptr_t>(ms.w[i]) & 15) != 0) || n * rb >= ((int64_t)1 << 32))
+            return kNotTaken;
+        rows += n;
+    }
+    fq::MmqArgs a{};
+    a.mm = ms.mm;
+    a.w = static_cast<const uint8_t*>(ms.w[0]);
+    a.w2 = static_cast<const uint8_t*>(ms.w[1]);
+    a.w3 = static_cast<const uint8_t*>(ms.w[2]);
+    a.n1 = ms.n[0];
+    a.n2 = ms.n[1];
+    a.n3 = ms.n[2];
+    a.row_bytes = (K / g.be) * g.bb;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    const MmqpPlan pl = plan_mmqp(M, K, fq::mmqp_row_tiles(a), fq::mm_cols(a), q6k ? rows : 0, di.cus,
+                                  fixed_cap);
+    const int splits = pl.splits;
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    const size_t xop_b = pl.xop_b, ex_b = pl.ex_b, sum_b = pl.sum_b, need = pl.total;
+    std::unique_ptr<StreamScratch::Lease> lease;
+    uint8_t* buf = fixed;
+    if (fixed) {
+        // (Q5_K in a fixed workspace that its K-splits here do not fit, 2040 x
+        // 256 x 4096 for instance, runs on the fp16 MFMA kernel, whose plan
+        // may)
+        if (need > fixed_cap) return dtype == FQ_DTYPE_Q5_K ? kNotTaken : FQ_ERR_WORKSPACE;
+    } else {
+        lease.reset(new StreamScratch::Lease(stream_scratch(dev, st, 0)));
+        const int rc = lease->get(need, st, &buf);
+        if (rc == FQ_ERR_WORKSPACE && ms.mm != fq::MM_ONE) return kNotTaken;
+        if (rc != FQ_OK) return rc;
+    }
+    hipError_t e = hipSuccess;
+    if (q6k) {
+        uint8_t* conv = buf + al(xop_b) + al(ex_b) + al(sum_b) + al(pl.part_b);
+        const uint8_t** w[3] = {&a.w, &a.w2, &a.w3};
+        for (int i = 0; i < 3; ++i) {
+            const int n = ms.mm == fq::MM_PAIR && i < 2 ? ms.n[0] : ms.n[i];
+            if (n == 0) continue;
+            e = fq::launch_q6c(*w[i], n, K, a.row_bytes, conv, st);
+            if (e != hipSuccess) return hip_fail(e);
+            *w[i] = conv;
+            conv += n * rb;
+        }
+        a.row_bytes = (int)rb;
+    }
+    a.xop = buf;
+    a.ex = reinterpret_cast<const int*>(buf + al(xop_b));
+    float* const sums = mmqk || dtype == FQ_DTYPE_Q4_1 || dtype == FQ_DTYPE_Q5_1
+                            ? reinterpret_cast<float*>(buf + al(xop_b) + al(ex_b))
+                            : nullptr;
+    a.xsum = sums;
+    a.part = splits > 1 ? reinterpret_cast<float*>(buf + al(xop_b) + al(ex_b) + al(sum_b))
+                        : nullptr;
+    a.y = y;
+    a.bias = bias;
+    a.bias_len = bias_mode ? bias_len : 0;
+    a.bias_mode = bias_mode;
+    e = fq::launch_xprep32(x, M, K, reinterpret_cast<_Float16*>(buf), const_cast<int*>(a.ex),
+                           mmqk ? nullptr : sums, mmqk ? reinterpret_cast<_Float16*>(sums) : nullptr,
+                           q6k, st);
+    if (e != hipSuccess) return hip_fail(e);
+    e = mmqk ? fq::launch_mmqk((int)dtype, a, splits, st) : fq::launch_mmqp((int)dtype, a, splits, st);
+    if (e == hipSuccess && splits > 1) e = fq::launch_reduce(a, splits, st);
     return e == hipSuccess ? FQ_OK : hip_fail(e);
 }
 
@@ -670,68 +775,10 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
         }
     }
 
-    const bool q6k = dtype == FQ_DTYPE_Q6_K;
-    const bool mmqk = fq::mmqk_supported((int)dtype);
-    // (Q5_K in a fixed workspace that its K-splits here do not fit, 2040 x
-    // 256 x 4096 for instance, runs on the fp16 MFMA kernel below, whose
-    // plan may)
-    const bool fits = !(fixed && dtype == FQ_DTYPE_Q5_K && K % 256 == 0) ||
-                      plan_mmqp(M, K, N, di.cus).total <= fixed_cap;
-    if (fits && (mmqk || fq::mmqp_supported((int)dtype)) && M > 32 && K > 0 && K % 256 == 0 &&
-        (q6k || (reinterpret_cast<uintptr_t>(w) & 15) == 0) &&
-        (int64_t)N * (q6k ? fq::mmqp_q6c_bytes(1, K) : (K / g.be) * g.bb) < ((int64_t)1 << 32)) {
-        // prefill, rows that are whole 16-byte chunks (K a multiple of 256,
-        // 16-byte aligned weights, under 4 GiB of them: the copies take
-        // 32-bit offsets): per-token operands, then one work-group per CU and
-        // tile on v_mfma_f32_32x32x16_f16 (K-split while the tiles leave CUs
-        // idle).  Q6_K rows are first rewritten into 36-byte blocks in the
-        // workspace
-        const MmqpPlan pl = plan_mmqp(M, K, N, di.cus, q6k);
-        const int splits = pl.splits;
-        auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-        const size_t xop_b = pl.xop_b, ex_b = pl.ex_b, sum_b = pl.sum_b, need = pl.total;
-        std::unique_ptr<StreamScratch::Lease> lease;
-        uint8_t* buf = fixed;
-        if (fixed) {
-            if (need > fixed_cap) return FQ_ERR_WORKSPACE;
-        } else {
-            lease.reset(new StreamScratch::Lease(stream_scratch(dev, st, 0)));
-            const int rc = lease->get(need, st, &buf);
-            if (rc != FQ_OK) return rc;
-        }
-        fq::MmqArgs a{};
-        a.w = static_cast<const uint8_t*>(w);
-        a.row_bytes = (K / g.be) * g.bb;
-        if (q6k) {
-            uint8_t* conv = buf + al(xop_b) + al(ex_b) + al(sum_b) + al(pl.part_b);
-            e = fq::launch_q6c(static_cast<const uint8_t*>(w), N, K, a.row_bytes, conv, st);
-            if (e != hipSuccess) return hip_fail(e);
-            a.w = conv;
-            a.row_bytes = (int)fq::mmqp_q6c_bytes(1, K);
-        }
-        a.xop = buf;
-        a.ex = reinterpret_cast<const int*>(buf + al(xop_b));
-        a.xsum = mmqk || dtype == FQ_DTYPE_Q4_1 || dtype == FQ_DTYPE_Q5_1
-                     ? reinterpret_cast<const float*>(buf + al(xop_b) + al(ex_b))
-                               : nullptr;
-        a.part = splits > 1 ? reinterpret_cast<float*>(buf + al(xop_b) + al(ex_b) + al(sum_b))
-                            : nullptr;
-        a.y = y;
-        a.bias = bias;
-        a.bias_len = bias_mode ? bias_len : 0;
-        a.bias_mode = bias_mode;
-        a.M = M;
-        a.N = N;
-        a.K = K;
-        float* const sums = const_cast<float*>(a.xsum);
-        e = fq::launch_xprep32(x, M, K, reinterpret_cast<_Float16*>(buf),
-                               const_cast<int*>(a.ex), mmqk ? nullptr : sums,
-                               mmqk ? reinterpret_cast<_Float16*>(sums) : nullptr, q6k, st);
-        if (e != hipSuccess) return hip_fail(e);
-        e = mmqk ? fq::launch_mmqk((int)dtype, a, splits, st)
-                 : fq::launch_mmqp((int)dtype, a, splits, st);
-        if (e == hipSuccess && splits > 1) e = fq::launch_reduce(a, splits, st);
-        return e == hipSuccess ? FQ_OK : hip_fail(e);
+    if (M > 32) {
+        const int rc = run_prefill(dtype, g, x, Mats{fq::MM_ONE, {w}, {N}}, bias, bias_mode,
+                                   bias_len, y, M, K, N, dev, di, st, fixed, fixed_cap);
+        if (rc != kNotTaken) return rc;
     }
 
     // M > 4, and rows too long for the batch-1 kernels' LDS
@@ -1177,6 +1224,17 @@ int fq_fused_qkv(uint32_t dtype, const float* x, const void* wq, const void* wk,
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e);
     const DevInfo di = device_info(dev);
+    if (M > 32) {  // one prefill launch over the three matrices
+        Mats ms{fq::MM_CAT, {}, {}};
+        int n = 0;
+        for (int i = 0; i < 3; ++i)
+            if (ns[i] > 0) {
+                ms.w[n] = ws[i];
+                ms.n[n++] = ns[i];
+            }
+        const int rc = run_prefill(dtype, g, x, ms, nullptr, 0, 0, y, M, K, Nt, dev, di, st, nullptr, 0);
+        if (rc != kNotTaken) return rc;
+    }
     uint8_t* buf = nullptr;
     const int nmax = std::max(Nq, std::max(Nk, Nv));
     StreamScratch::Lease lease(stream_scratch(dev, st, 1));
@@ -1248,6 +1306,11 @@ int fq_ffn_up_fused(uint32_t dtype, const float* x, const void* w_gate, const vo
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e);
     const DevInfo di = device_info(dev);
+    if (M > 32) {  // one prefill launch, gate and up rows in each tile
+        const int rc = run_prefill(dtype, g, x, Mats{fq::MM_PAIR, {w_gate, w_up}, {N}}, nullptr, 0, 0,
+                                   y, M, K, N, dev, di, st, nullptr, 0);
+        if (rc != kNotTaken) return rc;
+    }
     uint8_t* buf = nullptr;
     StreamScratch::Lease lease(stream_scratch(dev, st, 1));
     const int rs = lease.get(2 * (size_t)M * N * sizeof(float), st, &buf);
@@ -1284,7 +1347,11 @@ int fq_reserve_workspace(int M_max, int K_max, int N_max, void* stream) {
             need0 = std::max(need0, plan_mmq(m, K_max, n, di.cus).total);
             if (m <= 16 && Kp > 0)  // band kernel (from M = 2), four- and two-tile bands
                 for (int mt : {4, 3, 2}) need0 = std::max(need0, mmqs_need(m, Kp, n, di.cus, mt));
-            if (m > 32 && Kp > 0) need0 = std::max(need0, plan_mmqp(m, Kp, n, di.cus, true).total);
+            if (m > 32 && Kp > 0) {  // one matrix, and a gate/up pair
+                const int tn = fq::mmqp_tile_rows();
+                need0 = std::max(need0, plan_mmqp(m, Kp, (n + tn - 1) / tn, n, n, di.cus).total);
+                need0 = std::max(need0, plan_mmqp(m, Kp, (2L * n + tn - 1) / tn, 2 * n, 2 * n, di.cus).total);
+            }
             // the batch-1 kernel's K-split slabs for 2..4 tokens (at most 8)
             if (m <= 4) need0 = std::max(need0, (size_t)8 * m * n * sizeof(float));
         }

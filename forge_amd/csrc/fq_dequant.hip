@@ -8,6 +8,7 @@
 
 #include "fq_formats.h"
 #include "fq_kernels.h"
+#include "fq_mmtile.h"
 
 namespace fq {
 
@@ -214,8 +215,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__
                                                        const float* __restrict__ up,
                                                        float* __restrict__ y, size_t n) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        const float g = gate[i];
-        y[i] = g / (1.0f + expf(-g)) * up[i];
+        y[i] = silu_mul(gate[i], up[i]);
     }
 }
 

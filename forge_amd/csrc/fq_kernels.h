@@ -101,7 +101,18 @@ struct MmqArgs {
     int64_t bias_len;
     int bias_mode;
     int M, N, K, NC, row_bytes;
+    // several matrices over the same tokens (MM_PAIR, MM_CAT; the prefill
+    // kernels): w, w2, w3 with n1, n2, n3 rows.  MM_PAIR: y = silu(x w) (x w2),
+    // both of n1 = N rows.  MM_CAT: y = [x w | x w2 | x w3], N = n1 + n2 + n3
+    // (empty matrices last).  MM_ONE: w alone, n1 = N.
+    int mm;
+    const uint8_t *w2, *w3;
+    int n1, n2, n3;
 };
+enum { MM_ONE = 0, MM_PAIR = 1, MM_CAT = 2 };
+// Columns of a call's partial slabs: an MM_PAIR slab holds the gate columns,
+// then the up columns.
+inline int mm_cols(const MmqArgs& a) { return a.mm == MM_PAIR ? 2 * a.N : a.N; }
 enum { MMQ_SMALL1 = 0, MMQ_SMALL2 = 1, MMQ_MID = 2, MMQ_BIG = 3 };
 void mmq_shape(int shape, int* bn, int* bm);
 hipError_t launch_xprep(int dtype, const float* x, int M, int K, int NC, _Float16* xop,
@@ -123,6 +134,7 @@ hipError_t launch_mmqs(int dtype, const MmqArgs& a, int rows_per_wg, int wg, int
 bool mmqp_supported(int dtype);
 int mmqp_tile_rows();    // rows per work-group tile
 int mmqp_tile_tokens();  // tokens per work-group tile
+int mmqp_row_tiles(const MmqArgs& a);  // work-groups along the rows of a's matrices
 // sub16: the operand order of the Q6_K kernel (each 16-element quarter one
 // sub-block)
 // xsum / xsum2 (either may be null): the sub-block sums as floats, or in

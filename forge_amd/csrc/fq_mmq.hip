@@ -28,6 +28,7 @@
 #include "fq_formats.h"
 #include "fq_kernels.h"
 #include "fq_mfma16.h"
+#include "fq_mmtile.h"
 
 namespace fq {
 namespace {
@@ -698,7 +699,41 @@ hipError_t launch_xprep(int dtype, const float* x, int M, int K, int NC, _Float1
     return hipGetLastError();
 }
 
+// The slab sum of an MM_PAIR call: slabs of [M][2 N] (gate columns, then up),
+// y = silu(gate) * up, each summed in split order.  V: values per thread (4:
+// N a multiple of 4 and 16-byte aligned buffers).
+template <int V>
+__global__ __launch_bounds__(256) void reduce_pair_kernel(MmqArgs a, int splits) {
+    typedef float fv __attribute__((ext_vector_type(V)));
+    const int nv = a.N / V;
+    const size_t total = (size_t)a.M * nv, slab = (size_t)a.M * 2 * a.N;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total;
+         i += (size_t)gridDim.x * 256) {
+        const size_t m = i / nv, n = (i - m * nv) * V;
+        const float* p = a.part + m * 2 * a.N + n;
+        fv g = *reinterpret_cast<const fv*>(p), u = *reinterpret_cast<const fv*>(p + a.N);
+#pragma unroll 4
+        for (int z = 1; z < splits; ++z) {
+            g += *reinterpret_cast<const fv*>(p + z * slab);
+            u += *reinterpret_cast<const fv*>(p + z * slab + a.N);
+        }
+        fv y;
+#pragma unroll
+        for (int k = 0; k < V; ++k) y[k] = silu_mul(g[k], u[k]);
+        *reinterpret_cast<fv*>(a.y + m * a.N + n) = y;
+    }
+}
+
 hipError_t launch_reduce(const MmqArgs& a, int splits, hipStream_t st) {
+    if (a.mm == MM_PAIR) {
+        const bool v4 = a.N % 4 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 &&
+                        (reinterpret_cast<uintptr_t>(a.part) & 15) == 0;
+        const size_t n = (size_t)a.M * a.N / (v4 ? 4 : 1);
+        const dim3 grid((unsigned)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096));
+        if (v4) hipLaunchKernelGGL(reduce_pair_kernel<4>, grid, dim3(256), 0, st, a, splits);
+        else hipLaunchKernelGGL(reduce_pair_kernel<1>, grid, dim3(256), 0, st, a, splits);
+        return hipGetLastError();
+    }
     const size_t total = (size_t)a.M * a.N;
     if (a.N % 4 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 &&
         (reinterpret_cast<uintptr_t>(a.part) & 15) == 0) {

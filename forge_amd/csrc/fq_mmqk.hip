@@ -40,6 +40,7 @@
 #include "fq_formats.h"
 #include "fq_kernels.h"
 #include "fq_mfma16.h"
+#include "fq_mmtile.h"
 
 namespace fq {
 namespace {
@@ -71,7 +72,7 @@ struct KQ {
     static constexpr int LDS = NBUF * (XBUF + QBUF) + 2 * (HBUF + SBUF);
     // copy instructions per wave: every step, and more with a super-block's first
     static constexpr int CS = 4 + 1;
-    static constexpr int CB = (HBUF / NW + 1023) / 1024 + 1;
+    static constexpr int CB = (HP + 1) / 2 + 1;
     static_assert(LDS <= 160 * 1024, "LDS");
 };
 
@@ -114,9 +115,10 @@ __device__ __forceinline__ fq_u32x4 lds16(const uint8_t* p) {
 // lane.  All operands reach LDS by direct copies, three buffers deep for a
 // step's, two for a super-block's; one barrier per step publishes step s and
 // frees the buffers that step s + 2 refills.
-template <int F>
+template <int F, bool PAIR>
 __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_split) {
     using Q = KQ<F>;
+    constexpr int RJ = PAIR ? BNT / 2 : 32;  // tile rows between a wave's two row tiles
     __shared__ __attribute__((aligned(16))) uint8_t lds[Q::LDS];
     uint8_t* const xs0 = lds;
     uint8_t* const qs0 = xs0 + NBUF * Q::XBUF;
@@ -125,30 +127,39 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 2, wn = wave & 3;  // 64-token / 64-row quadrant
-    const int n0 = blockIdx.x * BNT, m0 = blockIdx.y * BMT;
+    const RowTile rt = row_tile<PAIR>(a, blockIdx.x, BNT);
+    const int m0 = blockIdx.y * BMT;
     const int nsteps = a.K / KS;
     const int s0 = blockIdx.z * steps_per_split, s1 = min(nsteps, s0 + steps_per_split);
     const int Tn = (a.M + 31) / 32;
     const int KQ16 = a.K / 16, NSB = a.K / 256;
 
     // copy sources: token run (tile wave / 2, half wave & 1 of its 8 KiB per
-    // step), 64 rows of code plane wave / 4, 768 bytes of the sums of tile
-    // wave / 2; the super-block planes of a wave are HBUF / NW bytes = HP / 2
-    // runs of 64 chunks, run L of all in plane L / 4, rows 64 (L % 4)
+    // step), 64 rows of code plane wave / 4, half the sums of tile wave / 2
     const int T = min(m0 / 32 + (wave >> 1), Tn - 1);
     const uint8_t* const xbase =
         reinterpret_cast<const uint8_t*>(a.xop) + ((size_t)T * KQ16 * XT) * 2 + (wave & 1) * 4096;
     const uint8_t* const sbase =
         reinterpret_cast<const uint8_t*>(a.xsum) + (size_t)T * NSB * STILE + (wave & 1) * (STILE / 2);
-    const uint32_t qoff = (uint32_t)min(n0 + 64 * (wave & 3) + lane, a.N - 1) * (uint32_t)a.row_bytes +
-                          Q::QOFF + 16 * (wave >> 2);
-    // super-block chunk 32 L + lane (L-th half run of this wave's share)
-    constexpr int HL = Q::HP;  // 32-chunk half runs per wave
-    uint32_t hoff[(HL + 1) / 2];
+    // tile row r is row r % 128 of the gate (r < 128) or up matrix of a pair
+    auto row_off = [&](int r) {
+        return (uint32_t)min(rt.n0 + (PAIR ? r & (BNT / 2 - 1) : r), rt.rows - 1) *
+               (uint32_t)a.row_bytes;
+    };
+    auto row_base = [&](int r) { return PAIR && r >= BNT / 2 ? a.w2 : rt.w; };  // wave-uniform r
+    const uint32_t qoff = row_off(64 * (wave & 3) + lane) + Q::QOFF + 16 * (wave >> 2);
+    const uint8_t* const qbase = row_base(64 * (wave & 3));
+    // super-block planes: 64 rows of planes 2 q and 2 q + 1 each (all eight
+    // waves), 32 rows of an odd last plane
+    constexpr int HR = (Q::HP + 1) / 2;
+    uint32_t hoff[HR];
+    const uint8_t* hbase[HR];
 #pragma unroll
-    for (int q = 0; q < (HL + 1) / 2; ++q) {
-        const int ch = min(32 * HL * wave + 64 * q + lane, Q::HP * BNT - 1);
-        hoff[q] = (uint32_t)min(n0 + (ch & (BNT - 1)), a.N - 1) * (uint32_t)a.row_bytes + 16 * (ch / BNT);
+    for (int q = 0; q < HR; ++q) {
+        const bool half = 2 * q + 1 == Q::HP;
+        const int r0 = half ? 32 * wave : 64 * (wave & 3), pl = half ? 2 * q : 2 * q + (wave >> 2);
+        hoff[q] = row_off(min(r0 + lane, BNT - 1)) + 16 * pl;
+        hbase[q] = row_base(r0);
     }
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds);
@@ -158,14 +169,15 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
         const uint8_t* xg = xbase + (size_t)s * 4 * XT * 2;
 #pragma unroll
         for (int i = 0; i < 4; ++i) dma16s(16 * lane + 1024 * i, xg, xl + 1024 * i);
-        const uint8_t* wsb = a.w + (size_t)sb * Q::BB;
-        dma16s(qoff, wsb + 32 * (s & 3), lds_base + NBUF * Q::XBUF + buf * Q::QBUF + wave * 1024);
+        const size_t wsb = (size_t)sb * Q::BB;
+        dma16s(qoff, qbase + wsb + 32 * (s & 3), lds_base + NBUF * Q::XBUF + buf * Q::QBUF + wave * 1024);
         if (first) {
-            const uint32_t hl =
-                lds_base + NBUF * (Q::XBUF + Q::QBUF) + (sb & 1) * Q::HBUF + wave * (Q::HBUF / NW);
+            const uint32_t hl = lds_base + NBUF * (Q::XBUF + Q::QBUF) + (sb & 1) * Q::HBUF;
 #pragma unroll
-            for (int q = 0; q < (HL + 1) / 2; ++q)
-                if (2 * q + 1 < HL || lane < 32) dma16s(hoff[q], wsb, hl + 1024 * q);
+            for (int q = 0; q < HR; ++q) {
+                if (2 * q + 1 < Q::HP) dma16s(hoff[q], hbase[q] + wsb, hl + 8192 * q + 1024 * wave);
+                else if (lane < 32) dma16s(hoff[q], hbase[q] + wsb, hl + 8192 * q + 512 * wave);
+            }
             if (lane < STILE / 32)
                 dma16s(16 * lane, sbase + (size_t)sb * STILE,
                        lds_base + NBUF * (Q::XBUF + Q::QBUF) + 2 * Q::HBUF + (sb & 1) * Q::SBUF +
@@ -196,13 +208,13 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
         constexpr int U = decltype(u)::value;
         h8 A[2][4];
         read_a(xs, 0, 0, A[0]);
-        const int rl = 64 * wn + c;
+        const int rl = PAIR ? 32 * wn + c : 64 * wn + c;
         fq_u32x4 hdr[2], qh[2], qv[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            hdr[j] = lds16(hs + (rl + 32 * j) * 16);
-            qv[j] = lds16(qs + (g * BNT + rl + 32 * j) * 16);
-            if constexpr (F == Q5_K) qh[j] = lds16(hs + ((1 + g) * BNT + rl + 32 * j) * 16);
+            hdr[j] = lds16(hs + (rl + RJ * j) * 16);
+            qv[j] = lds16(qs + (g * BNT + rl + RJ * j) * 16);
+            if constexpr (F == Q5_K) qh[j] = lds16(hs + ((1 + g) * BNT + rl + RJ * j) * 16);
         }
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
@@ -312,32 +324,10 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
         run(std::integral_constant<int, 2>{}, s + 2);
         run(std::integral_constant<int, 3>{}, s + 3);
     }
-    // lane (c, g): column n = 32 j + c of its quadrant, rows 8 (e / 4) + 4 g + e % 4
-    const bool split = gridDim.z > 1;
-    float* out = split ? a.part + (size_t)blockIdx.z * a.M * a.N : a.y;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        int ei[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-            ei[e] = a.ex[min(m0 + 64 * wm + 32 * i + 8 * (e >> 2) + 4 * g + (e & 3), a.M - 1)];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + 64 * wn + 32 * j + c;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int m = m0 + 64 * wm + 32 * i + 8 * (e >> 2) + 4 * g + (e & 3);
-                if (m < a.M && n < a.N) {
-                    float v = __builtin_amdgcn_ldexpf(acc[i][j][e], ei[e]);
-                    if (!split) {
-                        if (a.bias_mode == 1) v += n < a.bias_len ? a.bias[n] : 0.0f;
-                        else if (a.bias_mode == 2) v += a.bias[(size_t)m * a.N + n];
-                    }
-                    out[(size_t)m * a.N + n] = v;
-                }
-            }
-        }
-    }
+    for (int i = 0; i < 2; ++i)
+        store_tiles<PAIR>(a, rt, m0 + 64 * wm + 32 * i, rt.n0 + (PAIR ? 32 : 64) * wn + c, g, acc[i],
+                          gridDim.z > 1, blockIdx.z);
 }
 
 }  // namespace
@@ -351,11 +341,16 @@ hipError_t launch_mmqk(int dtype, const MmqArgs& a, int splits, hipStream_t st) 
     const int nsteps = a.K / KS;
     const int sps = ((nsteps + splits - 1) / splits + 3) & ~3;  // whole super-blocks
     if (a.K % 256 != 0 || (long)sps * (splits - 1) >= nsteps) return hipErrorInvalidValue;
-    const dim3 grid((a.N + BNT - 1) / BNT, (a.M + BMT - 1) / BMT, splits);
-    if (dtype == Q4_K)
-        hipLaunchKernelGGL(mmqk_kernel<Q4_K>, grid, dim3(64 * NW), 0, st, a, sps);
+    const dim3 grid(row_tiles(a, BNT), (a.M + BMT - 1) / BMT, splits), wg(64 * NW);
+    const bool pair = a.mm == MM_PAIR;
+    if (dtype == Q4_K && pair)
+        hipLaunchKernelGGL((mmqk_kernel<Q4_K, true>), grid, wg, 0, st, a, sps);
+    else if (dtype == Q4_K)
+        hipLaunchKernelGGL((mmqk_kernel<Q4_K, false>), grid, wg, 0, st, a, sps);
+    else if (dtype == Q5_K && pair)
+        hipLaunchKernelGGL((mmqk_kernel<Q5_K, true>), grid, wg, 0, st, a, sps);
     else if (dtype == Q5_K)
-        hipLaunchKernelGGL(mmqk_kernel<Q5_K>, grid, dim3(64 * NW), 0, st, a, sps);
+        hipLaunchKernelGGL((mmqk_kernel<Q5_K, false>), grid, wg, 0, st, a, sps);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

@@ -22,6 +22,7 @@
 #include "fq_kernels.h"
 #include "fq_limbs.h"
 #include "fq_mfma16.h"
+#include "fq_mmtile.h"
 
 namespace fq {
 namespace {
@@ -387,18 +388,20 @@ struct Tile {
 // Both operands reach LDS by direct copies into three buffers: while step s
 // is computed, the copies of steps s + 1 and s + 2 are in flight, and one
 // barrier per step publishes the next step's buffers.
-template <int F>
+template <int F, bool PAIR>
 __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_split) {
     using P = PB<F>;
     using TL = Tile<F>;
     constexpr int WROW = TL::WROW;
+    constexpr int RJ = PAIR ? BNT / 2 : 32;  // tile rows between a wave's two row tiles
     __shared__ __attribute__((aligned(16))) uint8_t lds[TL::LDS];
     uint8_t* const xs0 = lds;                       // NBUF token buffers
     uint8_t* const ws0 = lds + NBUF * TL::XBUF;     // NBUF weight buffers
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 2, wn = wave & 3;  // 64-token / 64-row quadrant
-    const int n0 = blockIdx.x * BNT, m0 = blockIdx.y * BMT;
+    const RowTile rt = row_tile<PAIR>(a, blockIdx.x, BNT);
+    const int m0 = blockIdx.y * BMT;
     const int nsteps = a.K / KS;
     const int s0 = blockIdx.z * steps_per_split, s1 = min(nsteps, s0 + steps_per_split);
     const int Tn = (a.M + 31) / 32;         // token tiles in the operand buffer
@@ -415,11 +418,17 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
         reinterpret_cast<const uint8_t*>(a.xop) + ((size_t)T * KQ * XT) * 2 + (wave & 1) * 4096;
     const int nwi = wave < TL::W_HI ? TL::WI_HI : TL::WI_LO;  // wave-uniform
     uint32_t woff[TL::WI_HI];
+    const uint8_t* wbase[TL::WI_HI];
 #pragma unroll
     for (int q = 0; q < TL::WI_HI; ++q) {
         const int L = min(64 * (NW * q + wave) + lane, TL::WCH - 1);
         const int r = L / TL::CH, p = L - r * TL::CH;  // [row][CH] slots
-        woff[q] = (uint32_t)min(n0 + r, a.N - 1) * (uint32_t)a.row_bytes + 16 * p;
+        // tile row r is row r % 128 of the gate (r < 128) or up matrix of a
+        // pair; 128 rows are whole copy instructions, so each has one base
+        woff[q] = (uint32_t)min(rt.n0 + (PAIR ? r & (BNT / 2 - 1) : r), rt.rows - 1) *
+                      (uint32_t)a.row_bytes +
+                  16 * p;
+        wbase[q] = PAIR && 64 * (NW * q + wave) >= BNT / 2 * TL::CH ? a.w2 : rt.w;
     }
     // sub-block sums (min term): tile T, block wave & 1, lanes 0..7
     const float* const sbase =
@@ -427,7 +436,7 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
     // Q5_0: a 44-byte step that starts 4 bytes into its first chunk ends 16
     // bytes before the last of its four: on the matrix's last row that chunk
     // lies past the end (its bytes are never read)
-    const uint32_t wend = (uint32_t)a.N * (uint32_t)a.row_bytes - 16;
+    const uint32_t wend = (uint32_t)rt.rows * (uint32_t)a.row_bytes - 16;
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds);
     auto issue = [&](int s) {
@@ -447,7 +456,7 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
             if (q < nwi) {
                 const uint32_t so = (uint32_t)Chunks<F>::off(s);
                 const uint32_t vo = F == Q5_0 ? min(woff[q], wend - so) : woff[q];
-                dma16s(vo, a.w + so, wl + NW * 1024 * q);
+                dma16s(vo, wbase[q] + so, wl + NW * 1024 * q);
             }
     };
     // this wave's copies of step s are complete (those of step s + 1 may
@@ -494,7 +503,7 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
             float db[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const uint8_t* row = ws + (64 * wn + 32 * j + c) * WROW;
+                const uint8_t* row = ws + ((PAIR ? 32 : 64) * wn + RJ * j + c) * WROW;
                 uint32_t q[4];
                 if (b == 0) {
                     codes<F, O4, 0>(row, g, q);
@@ -629,32 +638,10 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[1][j][e] = __builtin_fmaf(dbp[j], dp[j][e], acc[1][j][e]);
     }
-    // lane (c, g): column n = 32 j + c of its quadrant, rows 8 (e / 4) + 4 g + e % 4
-    const bool split = gridDim.z > 1;
-    float* out = split ? a.part + (size_t)blockIdx.z * a.M * a.N : a.y;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        int ei[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-            ei[e] = a.ex[min(m0 + 64 * wm + 32 * i + 8 * (e >> 2) + 4 * g + (e & 3), a.M - 1)];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + 64 * wn + 32 * j + c;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int m = m0 + 64 * wm + 32 * i + 8 * (e >> 2) + 4 * g + (e & 3);
-                if (m < a.M && n < a.N) {
-                    float v = __builtin_amdgcn_ldexpf(acc[i][j][e], ei[e]);
-                    if (!split) {
-                        if (a.bias_mode == 1) v += n < a.bias_len ? a.bias[n] : 0.0f;
-                        else if (a.bias_mode == 2) v += a.bias[(size_t)m * a.N + n];
-                    }
-                    out[(size_t)m * a.N + n] = v;
-                }
-            }
-        }
-    }
+    for (int i = 0; i < 2; ++i)
+        store_tiles<PAIR>(a, rt, m0 + 64 * wm + 32 * i, rt.n0 + (PAIR ? 32 : 64) * wn + c, g, acc[i],
+                          gridDim.z > 1, blockIdx.z);
 }
 
 // ------------------------------------------------------ Q6_K conversion
@@ -726,6 +713,7 @@ hipError_t launch_q6c(const uint8_t* w, int N, int K, int64_t row_bytes, uint8_t
 }
 int mmqp_tile_rows() { return BNT; }
 int mmqp_tile_tokens() { return BMT; }
+int mmqp_row_tiles(const MmqArgs& a) { return row_tiles(a, BNT); }
 
 hipError_t launch_xprep32(const float* x, int M, int K, _Float16* xop, int* ex, float* xsum,
                           _Float16* xsum2, bool sub16, hipStream_t st) {
@@ -743,21 +731,21 @@ hipError_t launch_mmqp(int dtype, const MmqArgs& a, int splits, hipStream_t st) 
     const int nsteps = a.K / KS;
     const int sps = ((nsteps + splits - 1) / splits + 3) & ~3;  // a multiple of 4 steps
     if ((long)sps * (splits - 1) >= nsteps) return hipErrorInvalidValue;
-    const dim3 grid((a.N + BNT - 1) / BNT, (a.M + BMT - 1) / BMT, splits);
-    if (dtype == Q8_0)
-        hipLaunchKernelGGL(mmqp_kernel<Q8_0>, grid, dim3(64 * NW), 0, st, a, sps);
-    else if (dtype == Q4_0)
-        hipLaunchKernelGGL(mmqp_kernel<Q4_0>, grid, dim3(64 * NW), 0, st, a, sps);
-    else if (dtype == Q4_1)
-        hipLaunchKernelGGL(mmqp_kernel<Q4_1>, grid, dim3(64 * NW), 0, st, a, sps);
-    else if (dtype == Q5_0)
-        hipLaunchKernelGGL(mmqp_kernel<Q5_0>, grid, dim3(64 * NW), 0, st, a, sps);
-    else if (dtype == Q5_1)
-        hipLaunchKernelGGL(mmqp_kernel<Q5_1>, grid, dim3(64 * NW), 0, st, a, sps);
-    else if (dtype == Q6_K)
-        hipLaunchKernelGGL(mmqp_kernel<Q6_K>, grid, dim3(64 * NW), 0, st, a, sps);
-    else
-        return hipErrorInvalidValue;
+    const dim3 grid(row_tiles(a, BNT), (a.M + BMT - 1) / BMT, splits), wg(64 * NW);
+    auto go = [&](auto f) {
+        constexpr int F = decltype(f)::value;
+        if (a.mm == MM_PAIR)
+            hipLaunchKernelGGL((mmqp_kernel<F, true>), grid, wg, 0, st, a, sps);
+        else
+            hipLaunchKernelGGL((mmqp_kernel<F, false>), grid, wg, 0, st, a, sps);
+    };
+    if (dtype == Q8_0) go(FmtTag<Q8_0>{});
+    else if (dtype == Q4_0) go(FmtTag<Q4_0>{});
+    else if (dtype == Q4_1) go(FmtTag<Q4_1>{});
+    else if (dtype == Q5_0) go(FmtTag<Q5_0>{});
+    else if (dtype == Q5_1) go(FmtTag<Q5_1>{});
+    else if (dtype == Q6_K) go(FmtTag<Q6_K>{});
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
