@@ -22,7 +22,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 SOURCES = ["fq_dequant.hip", "fq_gemv1.hip", "fq_gemvp.hip", "fq_gemvt.hip", "fq_pack.hip", "fq_mmq.hip",
-           "fq_mmqi.hip", "fq_mmqs.hip", "fq_mmqp.hip", "fq_mmqk.hip",
+           "fq_mmqi.hip", "fq_mmqs.hip", "fq_mmqp.hip", "fq_mmqk.hip", "fq_mmqt.hip",
            "fq_capi.cpp"]
 
 COMMON = [
@@ -36,7 +36,7 @@ COMMON = [
 # MFMA results per lane: with the results in AGPRs (the compiler's default
 # under that register pressure) every FMA needs a v_accvgpr_read first, so
 # the MFMA results are kept in VGPRs.
-EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("fq_mmqp.hip", "fq_mmqk.hip")}
+EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("fq_mmqp.hip", "fq_mmqk.hip", "fq_mmqt.hip")}
 
 
 def _compile(src: str) -> str:

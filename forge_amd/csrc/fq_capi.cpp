@@ -7,9 +7,10 @@
 // of fq_gemv1.hip under about 4 MB of weights); M = 2..4
 // the same batch-1 kernels with each weight unit dotted with every token;
 // M = 2..16 (by format and shape) the band kernel of fq_mmqs.hip
-// (Q6_K M = 4 on wide matrices: three tokens, then the fourth); M > 32 the
-// prefill kernel
-// of fq_mmqp.hip (rows in 16-byte chunks, K a multiple of 256); the rest --
+// (Q6_K M = 4 on wide matrices: three tokens, then the fourth); M = 4..16 of
+// Q4_K, Q5_K and Q6_K on 24 MB and more and M = 17..32 the kernel of
+// fq_mmqt.hip; M > 32 the prefill kernels
+// of fq_mmqk.hip and fq_mmqp.hip (rows in 16-byte chunks, K a multiple of 256); the rest --
 // the reference's batched GEMV (1 < M <= 32) and dequant + GEMM prefill
 // (M > 32), matmul.cpp:1150-1286 -- the int8 and fp16 MFMA kernels of
 // fq_mmqi.hip and fq_mmq.hip.
@@ -400,6 +401,123 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
     return e == hipSuccess ? FQ_OK : hip_fail(e);
 }
 
+// Small batches of Q4_K, Q5_K and Q6_K with the token operands shared by the
+// rows of a work-group (fq_mmqt.hip).
+struct MmqtPlan {
+    int rows, splits;
+    size_t xop_b, sum_b, part_b, total;
+};
+
+// Rows per work-group and K-splits of the smallest estimated time: rounds of
+// work-groups x (iterations of one or two super-blocks + 1.5 us to fill the
+// pipeline), and for a split the slab sum (3.5 us and each slab written and
+// read at 4 TB/s).  us per iteration measured at 14336 x 4096 on 224
+// work-groups.
+MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
+    struct Shape {
+        int rows, kg;
+        double t;
+    };
+    const bool q6 = dtype == FQ_DTYPE_Q6_K, wide = a.M > 16;
+    const Shape shapes[3] = {{256, 1, q6 ? 2.7 : wide ? 2.6 : 2.0},
+                             {128, q6 || wide ? 1 : 2, q6 ? (wide ? 2.2 : 1.7) : wide ? 1.6 : 1.7},
+                             {64, 2, q6 ? 1.8 : 1.3}};
+    MmqtPlan p{};
+    const int nsb = a.K / 256;
+    double best = 0.0;
+    for (const Shape& s : shapes) {
+        if (!fq::mmqt_has_rows((int)dtype, a.M, s.rows)) continue;
+        const long tiles = fq::mmqt_row_tiles(a, s.rows);
+        for (int sp = 1; sp <= std::min(16, nsb); ++sp) {
+            const int sps = (nsb + sp - 1) / sp;
+            if (sps * (sp - 1) >= nsb) continue;  // an empty split
+            const double t = (double)((tiles * sp + cus - 1) / cus) *
+                                 (1.5 + s.t * ((sps + s.kg - 1) / s.kg)) +
+                             (sp > 1 ? 3.5 + (sp + 1.0) * a.M * fq::mm_cols(a) * 4.0 / 4e6 : 0.0);
+            if (p.rows == 0 || t < best) {
+                best = t;
+                p.rows = s.rows;
+                p.splits = sp;
+            }
+        }
+    }
+    if (p.rows == 0) return p;
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    p.xop_b = fq::mmqt_xop_bytes(a.M, a.K);
+    p.sum_b = fq::mmqt_sum_bytes(a.M, a.K);
+    p.part_b = p.splits > 1 ? (size_t)p.splits * a.M * fq::mm_cols(a) * 4 : 0;
+    p.total = 256 + al(p.xop_b) + al(p.sum_b) + al(p.part_b);
+    return p;
+}
+
+// Whether 2..32 tokens on one matrix of this size (or on a gate/up pair of two)
+// go there.  17..32 tokens always (the fp16 MFMA path: Q4_K 4096 x 4096 at M =
+// 32 20.8 -> 14.7 us, 14336 x 4096 40.2 -> 23.2, Q6_K 4096 x 14336 56.4 ->
+// 29.0).  Up to 16 from 24 MB (Q6_K: 32 MB) of weights: below, the band
+// kernel's bands fill the chip without a K split and its slab sum (Q4_K 8192 x
+// 4096, 19 MB, M = 8: 12.6 us there, 13.5 here; 14336 x 4096, 33 MB: 18.7 and
+// 16.3; Q6_K 8192 x 4096, 28 MB: 16.5 and 16.8; 14336 x 4096: 27.6 and 20.9;
+// 152064 x 3584 at M = 16 216 and 139).
+bool thin_takes(uint32_t dtype, int M, int64_t bytes) {
+    if (!fq::mmqt_supported((int)dtype) || M < 2 || M > 32) return false;
+    return M > 16 || bytes >= (dtype == FQ_DTYPE_Q6_K ? 32LL << 20 : 24LL << 20);
+}
+
+// kNotTaken: another kernel runs the call (also where the workspace cannot
+// hold this one's operands: capture, the fixed array).
+int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, const float* bias,
+             int bias_mode, int64_t bias_len, float* y, int M, int K, int N, int dev,
+             const DevInfo& di, hipStream_t st, uint8_t* fixed, size_t fixed_cap) {
+    if (K <= 0 || K % 256 != 0) return kNotTaken;
+    const bool q6k = dtype == FQ_DTYPE_Q6_K;
+    const int64_t rb = (int64_t)(K / g.be) * g.bb;
+    for (int i = 0; i < 3; ++i) {
+        const int n = ms.mm == fq::MM_PAIR && i < 2 ? ms.n[0] : ms.n[i];
+        if (n == 0) continue;
+        if ((reinterpret_cast<uintptr_t>(ms.w[i]) & (q6k ? 1 : 15)) != 0 ||
+            n * rb + 16 >= ((int64_t)1 << 32))
+            return kNotTaken;
+    }
+    fq::MmqArgs a{};
+    a.mm = ms.mm;
+    a.w = static_cast<const uint8_t*>(ms.w[0]);
+    a.w2 = static_cast<const uint8_t*>(ms.w[1]);
+    a.w3 = static_cast<const uint8_t*>(ms.w[2]);
+    a.n1 = ms.n[0];
+    a.n2 = ms.n[1];
+    a.n3 = ms.n[2];
+    a.row_bytes = (int)rb;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    const MmqtPlan pl = plan_mmqt(a, dtype, di.cus);
+    if (pl.rows == 0) return kNotTaken;
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    std::unique_ptr<StreamScratch::Lease> lease;
+    uint8_t* buf = fixed;
+    if (fixed) {
+        if (pl.total > fixed_cap) return kNotTaken;
+    } else {
+        lease.reset(new StreamScratch::Lease(stream_scratch(dev, st, 0)));
+        const int rc = lease->get(pl.total, st, &buf);
+        if (rc == FQ_ERR_WORKSPACE) return kNotTaken;
+        if (rc != FQ_OK) return rc;
+    }
+    a.xop = buf;
+    uint8_t* const sums = buf + al(pl.xop_b);
+    a.xsum = reinterpret_cast<const float*>(sums);
+    a.part = pl.splits > 1 ? reinterpret_cast<float*>(sums + al(pl.sum_b)) : nullptr;
+    a.y = y;
+    a.bias = bias;
+    a.bias_len = bias_mode ? bias_len : 0;
+    a.bias_mode = bias_mode;
+    hipError_t e = fq::launch_xprept((int)dtype, x, M, K, buf, sums, st);
+    if (e != hipSuccess) return hip_fail(e);
+    e = fq::launch_mmqt((int)dtype, a, pl.rows, pl.splits, st);
+    if (e == hipSuccess && pl.splits > 1) e = fq::launch_reduce(a, pl.splits, st);
+    return e == hipSuccess ? FQ_OK : hip_fail(e);
+}
+
 // band_x (optional): in, true when the stream's slot-0 workspace already
 // holds the band kernel's token operands of this x, M, K and format (a call
 // just before with the same x, M, K, N and format took the band kernel:
@@ -496,6 +614,12 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
             if (rc != FQ_OK) return rc;
         }
         return FQ_OK;
+    }
+
+    if (M >= 4 && thin_takes(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {
+        const int rc = run_thin(dtype, g, x, Mats{fq::MM_ONE, {w}, {N}}, bias, bias_mode, bias_len, y, M,
+                                K, N, dev, di, st, fixed, fixed_cap);
+        if (rc != kNotTaken) return rc;
     }
 
     // Q4_0 and Q8_0 on the band kernel below: rows that start 16-byte aligned
@@ -1224,15 +1348,18 @@ int fq_fused_qkv(uint32_t dtype, const float* x, const void* wq, const void* wk,
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e);
     const DevInfo di = device_info(dev);
-    if (M > 32) {  // one prefill launch over the three matrices
-        Mats ms{fq::MM_CAT, {}, {}};
-        int n = 0;
-        for (int i = 0; i < 3; ++i)
-            if (ns[i] > 0) {
-                ms.w[n] = ws[i];
-                ms.n[n++] = ns[i];
-            }
-        const int rc = run_prefill(dtype, g, x, ms, nullptr, 0, 0, y, M, K, Nt, dev, di, st, nullptr, 0);
+    Mats ms{fq::MM_CAT, {}, {}};
+    for (int i = 0, n = 0; i < 3; ++i)
+        if (ns[i] > 0) {
+            ms.w[n] = ws[i];
+            ms.n[n++] = ns[i];
+        }
+    if (M > 16) {  // one launch over the three matrices
+        int rc = kNotTaken;
+        if (M > 32)
+            rc = run_prefill(dtype, g, x, ms, nullptr, 0, 0, y, M, K, Nt, dev, di, st, nullptr, 0);
+        else if (thin_takes(dtype, M, 0))
+            rc = run_thin(dtype, g, x, ms, nullptr, 0, 0, y, M, K, Nt, dev, di, st, nullptr, 0);
         if (rc != kNotTaken) return rc;
     }
     uint8_t* buf = nullptr;
@@ -1306,6 +1433,11 @@ int fq_ffn_up_fused(uint32_t dtype, const float* x, const void* w_gate, const vo
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e);
     const DevInfo di = device_info(dev);
+    if (thin_takes(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {  // gate and up rows in one launch
+        const int rc = run_thin(dtype, g, x, Mats{fq::MM_PAIR, {w_gate, w_up}, {N}}, nullptr, 0, 0, y, M,
+                                K, N, dev, di, st, nullptr, 0);
+        if (rc != kNotTaken) return rc;
+    }
     if (M > 32) {  // one prefill launch, gate and up rows in each tile
         const int rc = run_prefill(dtype, g, x, Mats{fq::MM_PAIR, {w_gate, w_up}, {N}}, nullptr, 0, 0,
                                    y, M, K, N, dev, di, st, nullptr, 0);
@@ -1351,6 +1483,17 @@ int fq_reserve_workspace(int M_max, int K_max, int N_max, void* stream) {
                 const int tn = fq::mmqp_tile_rows();
                 need0 = std::max(need0, plan_mmqp(m, Kp, (n + tn - 1) / tn, n, n, di.cus).total);
                 need0 = std::max(need0, plan_mmqp(m, Kp, (2L * n + tn - 1) / tn, 2 * n, 2 * n, di.cus).total);
+            }
+            if (m <= 32 && Kp > 0) {  // one matrix, and a gate/up pair
+                fq::MmqArgs t{};
+                t.M = m;
+                t.K = Kp;
+                t.N = t.n1 = n;
+                for (uint32_t dt : {FQ_DTYPE_Q4_K, FQ_DTYPE_Q6_K})
+                    for (int mm : {fq::MM_ONE, fq::MM_PAIR}) {
+                        t.mm = mm;
+                        need0 = std::max(need0, plan_mmqt(t, dt, di.cus).total);
+                    }
             }
             // the batch-1 kernel's K-split slabs for 2..4 tokens (at most 8)
             if (m <= 4) need0 = std::max(need0, (size_t)8 * m * n * sizeof(float));

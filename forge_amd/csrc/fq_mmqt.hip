@@ -1,0 +1,542 @@
+// fq_mmqt.hip -- small batches (M <= 32 tokens) of Q4_K, Q5_K and Q6_K on the
+// fp16 matrix cores, the token operands shared by 128 or 256 rows.
+//
+// A work-group owns a tile of 64, 128 or 256 rows and a range of super-blocks
+// (256 elements of K).  Per super-block it copies into LDS, two or three
+// buffers deep and with no registers in between,
+//
+//   the rows' super-blocks as they lie in memory (16-byte pieces along each
+//   row: contiguous runs of 144 / 176 / 210 bytes), each wave its own 16 rows,
+//   the tokens' operands (16 KiB per 16 tokens), an equal share per wave,
+//   the tokens' sub-block sums and scales,
+//
+// and one barrier per super-block publishes them.  In the band kernel of
+// fq_mmqs.hip every wave reads the token operands of its own super-blocks from
+// L2, for 32 or 64 rows: 3.5 times the weight bytes for a Q6_K head at 16
+// tokens (1.1 GB).  Here the operands of a super-block serve all rows of the
+// work-group.  152064 x 3584 Q6_K, M = 16: 216 -> 139 us; Q4_K, M = 8 131 ->
+// 98; 14336 x 4096 Q4_K, M = 8 18.7 -> 16.3, M = 32 (fp16 MFMA kernel) 40.2 ->
+// 23.2, gate and up of that size in one launch 37.7 -> 22.0 and 82.5 -> 36.0.
+// What bounds it: vector and matrix issue with the LDS reads of the token
+// operands, about equal (without the copies the head's time is 117 us, without
+// the arithmetic 105), so the waves per SIMD count: 256 rows on eight waves of
+// two tiles each ran the head in 152 us, on sixteen waves 139.
+//
+// Tokens are the A operand of v_mfma_f32_16x16x32_f16 (lane 16 q + c: token c,
+// eight elements of k group q) and weights the B operand (lane 16 q + c: row
+// c), so that a lane's results belong to one row.  Lane group q takes the
+// q-th quarter of the super-block: Q4_K / Q5_K sub-block pair q (its 32 qs
+// bytes, two scales), Q6_K unit q (16 l positions of a half, four scales), and
+// decodes no scale but its own.  The scale goes into the weight operand:
+//
+//   Q4_K, Q5_K: sc (q - c) as in fq_mmqk.hip, exact in fp16 (at most 1008);
+//   Q6_K: sc (q - 32) has up to 13 bits: W = W_hi + W_lo, W_hi its fp16
+//   rounding and W_lo the exact rest; x W = x_hi W_hi + x_lo W_hi + x_hi W_lo
+//   (the dropped x_lo W_lo is 2^-23 of the product).
+//
+// One MFMA chain per super-block, then acc += 2^e (d D - dmin Dm), e the
+// token's exponent for this super-block (x 2^-e below 2^15, split into fp16
+// hi + lo: 22 significant bits).
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "fq_dma.h"
+#include "fq_formats.h"
+#include "fq_kernels.h"
+#include "fq_mfma16.h"
+#include "fq_mmtile.h"
+
+namespace fq {
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int XSB = 16384;  // operand bytes of a (16-token tile, super-block): [ks][hi, lo][lane][8]
+// sums and scales of a (tile, super-block): eight groups of 144 bytes, group
+// w: the sums operand of lanes 8 w .. 8 w + 7, then (w < 4) the floats 2^e of
+// tokens 4 w .. 4 w + 3
+constexpr int SG = 144, SSB = 8 * SG;
+
+// ------------------------------------------------------------- token prep
+// One work-group per super-block and 16-token tile; thread 16 c + p holds
+// elements 16 p .. 16 p + 15 of token c.  Eight elements 8 e8 .. + 7 are slots
+// (slot_elem order) of lane group q in MFMA ks: Q4_K / Q5_K q = e8 / 8, ks =
+// e8 % 8; Q6_K (U6) element 128 n + 32 u + 16 h + 8 i: q = 2 n + h, ks = 2 u +
+// i.  The sums operand of lane (c, q) holds token c's sums (times 2^-5) over
+// sub-blocks 2 q, 2 q + 1 in three fp16 parts: hi, hi, mid, mid, lo, lo, 0, 0.
+template <bool U6>
+__global__ __launch_bounds__(256) void xprept_kernel(const float* __restrict__ x, int M, int K,
+                                                     uint8_t* __restrict__ xop,
+                                                     uint8_t* __restrict__ xs) {
+    const int tid = threadIdx.x, c = tid >> 4, p = tid & 15;
+    const int sb = blockIdx.x, T = blockIdx.y, m = 16 * T + c, nsb = K / 256;
+    float v[16] = {};
+    if (m < M) {
+        const float4* s = reinterpret_cast<const float4*>(x + (size_t)m * K + 256 * sb + 16 * p);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 t = s[i];
+            v[4 * i] = t.x;
+            v[4 * i + 1] = t.y;
+            v[4 * i + 2] = t.z;
+            v[4 * i + 3] = t.w;
+        }
+    }
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(v[i]));
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    const int e = (mx > 0.0f && mx <= 3.0e38f) ? ilogbf(mx) - 14 : 0;
+    float sum = 0.0f;
+    uint8_t* const ob = xop + ((size_t)T * nsb + sb) * XSB;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int e8 = 2 * p + i;
+        const int q = U6 ? 2 * (e8 >> 4) + ((e8 >> 1) & 1) : e8 >> 3;
+        const int ks = U6 ? 2 * ((e8 >> 2) & 3) + (e8 & 1) : e8 & 7;
+        float w[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w[j] = __builtin_amdgcn_ldexpf(v[8 * i + j], -e);
+        h8 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float u = w[slot_elem(j)];
+            hi[j] = (_Float16)u;
+            lo[j] = (_Float16)(u - (float)hi[j]);
+        }
+        h8* o = reinterpret_cast<h8*>(ob + ks * 2048 + (16 * q + c) * 16);
+        o[0] = hi;
+        o[64] = lo;
+        sum += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+    }
+    uint8_t* const sbk = xs + ((size_t)T * nsb + sb) * SSB;
+    if (p == 0) *reinterpret_cast<float*>(sbk + (c >> 2) * SG + 128 + 4 * (c & 3)) =
+        __builtin_amdgcn_ldexpf(1.0f, e);
+    if constexpr (!U6) {
+        sum += __shfl_xor(sum, 1, 64);
+        if ((p & 1) == 0) {
+            const int b = p >> 1, l = 16 * (b >> 1) + c;
+            const float s = sum * 0x1p-5f;
+            const _Float16 s0 = (_Float16)s;
+            const float r = s - (float)s0;
+            const _Float16 s1 = (_Float16)r;
+            _Float16* d = reinterpret_cast<_Float16*>(sbk + (l >> 3) * SG + (l & 7) * 16) + (b & 1);
+            d[0] = s0;
+            d[2] = s1;
+            d[4] = (_Float16)(r - (float)s1);
+            d[6] = (_Float16)0.0f;
+        }
+    }
+}
+
+// ------------------------------------------------------------- weights
+// PPR: 16-byte pieces of a row's super-block in LDS; SHIFT: rows start at even
+// addresses only, each super-block copied from its aligned-down start and read
+// at its shift (Q6_K: 14 pieces always hold some of its 210 bytes; a 15th,
+// a repeat, keeps 16 rows' 16-byte units on distinct banks).
+template <int F>
+struct TQ;
+
+__device__ __forceinline__ fq_u32x4 lds16(const uint8_t* p) {
+    typedef const __attribute__((address_space(3))) fq_u32x4* lds_v4;
+    return *reinterpret_cast<lds_v4>(reinterpret_cast<uintptr_t>(p));
+}
+__device__ __forceinline__ uint32_t lds4(const uint8_t* p) {
+    typedef const __attribute__((address_space(3))) uint32_t* lds_v1;
+    return *reinterpret_cast<lds_v1>(reinterpret_cast<uintptr_t>(p));
+}
+
+template <int F>
+struct TQK {
+    static constexpr int SBB = F == Q5_K ? 176 : 144, PPR = SBB / 16, LAST = PPR - 1;
+    static constexpr bool SHIFT = false, MIN = true, SPLITW = false;
+    static constexpr float UNIT = F == Q5_K ? 8.0f : 16.0f, MID = F == Q5_K ? 16.0f : 8.0f;
+    uint32_t w[8], h[8];
+    h2 s[2], off[2];
+    h8 mb, cb;
+    float d, dn;
+    // row's super-block at p (LDS), lane group q
+    __device__ void load(const uint8_t* p, int, int q) {
+        const fq_u32x4 hd = lds16(p);
+        const uint8_t* qs = p + (F == Q5_K ? 48 : 16) + 32 * q;
+        const fq_u32x4 a = lds16(qs), b = lds16(qs + 16);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            w[k] = a[k];
+            w[4 + k] = b[k];
+        }
+        if constexpr (F == Q5_K) {  // bits 2 q, 2 q + 1 of each qh byte to bits 6, 7
+            const fq_u32x4 ha = lds16(p + 16), hb = lds16(p + 32);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                h[k] = ha[k] << (6 - 2 * q);
+                h[4 + k] = hb[k] << (6 - 2 * q);
+            }
+        }
+        uint32_t sa, ma, sb, mi;
+        Fmt<Q4_K>::scale_min(uint4{hd.x, hd.y, hd.z, hd.w}, q, sa, ma, sb, mi);
+        const float f0 = (float)sa, f1 = (float)sb;
+        const _Float16 u0 = (_Float16)(f0 * (1.0f / UNIT)), u1 = (_Float16)(f1 * (1.0f / UNIT));
+        s[0] = h2{u0, u0};
+        s[1] = h2{u1, u1};
+        off[0] = s[0] * h2{(_Float16)-1152.0f, (_Float16)-1152.0f};
+        off[1] = s[1] * h2{(_Float16)-1152.0f, (_Float16)-1152.0f};
+        const _Float16 m0 = (_Float16)(float)ma, m1 = (_Float16)(float)mi, z = (_Float16)0.0f;
+        mb = h8{m0, m1, m0, m1, m0, m1, z, z};
+        const _Float16 c0 = (_Float16)(f0 * (32.0f * MID)), c1 = (_Float16)(f1 * (32.0f * MID));
+        cb = h8{c0, c1, c0, c1, c0, c1, z, z};
+        d = f16_hw(hd.x & 0xFFFFu);
+        dn = -32.0f * f16_hw(hd.x >> 16);
+    }
+    template <int KSI>
+    __device__ uint32_t code(int k) const {
+        if constexpr (F == Q5_K) {
+            const uint32_t n = (KSI < 4 ? w[k] << 3 : w[k] >> 1) & 0x78787878u;
+            return n | ((KSI < 4 ? h[k] << 1 : h[k]) & 0x80808080u);
+        } else {
+            return (KSI < 4 ? w[k] << 4 : w[k]) & 0xF0F0F0F0u;
+        }
+    }
+    // the weight operand of MFMA KSI
+    template <int KSI>
+    __device__ void ops(h8& whi, h8&) const {
+        constexpr int k = 2 * (KSI & 3), t = KSI >> 2;
+        const uint32_t c0 = code<KSI>(k), c1 = code<KSI>(k + 1);
+        auto pr = [&](uint32_t c, uint32_t sel) {
+            return __builtin_elementwise_fma(
+                __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, c, sel)), s[t], off[t]);
+        };
+        const h2 a = pr(c0, 0x04020400u), b = pr(c0, 0x04030401u), e = pr(c1, 0x04020400u),
+                 f = pr(c1, 0x04030401u);
+        whi = h8{a[0], a[1], b[0], b[1], e[0], e[1], f[0], f[1]};
+    }
+};
+template <>
+struct TQ<Q4_K> : TQK<Q4_K> {};
+template <>
+struct TQ<Q5_K> : TQK<Q5_K> {};
+
+// Q6_K (210 B: ql[128] qh[64] sc[16] d), unit q = 2 n + h: 16 bytes each of
+// ql[64 n + 16 h], ql[64 n + 32 + 16 h] and qh[32 n + 16 h]; u = 0..3: nibble
+// u / 2 of the first (u even) or second run, bits 2 u of the third, scale
+// sc[8 n + 2 u + h]; MFMA ks = 2 u + i takes its bytes 8 i .. 8 i + 7.
+template <>
+struct TQ<Q6_K> {
+    static constexpr int SBB = 210, PPR = 15, LAST = 13;
+    static constexpr bool SHIFT = true, MIN = false, SPLITW = true;
+    uint32_t lo[4], hi[4], qh[4];
+    h2 s[4];
+    float d;
+    __device__ static void run16(const uint8_t* p, uint32_t sh, uint32_t (&o)[4]) {
+        uint32_t t[5];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) t[k] = lds4(p + 4 * k);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] = __builtin_amdgcn_alignbyte(t[k + 1], t[k], sh);
+    }
+    // the row's pieces at p, its super-block sh bytes in
+    __device__ void load(const uint8_t* p, int sh, int q) {
+        const uint32_t r = sh & 3;  // 0 or 2
+        const uint8_t* a = p + (sh & ~3);
+        const int n = q >> 1, h = q & 1;
+        run16(a + 64 * n + 16 * h, r, lo);
+        run16(a + 64 * n + 32 + 16 * h, r, hi);
+        run16(a + 128 + 32 * n + 16 * h, r, qh);
+        const uint32_t s0 = lds4(a + 192 + 8 * n), s1 = lds4(a + 196 + 8 * n), s2 = lds4(a + 200 + 8 * n);
+        const uint32_t sa = __builtin_amdgcn_alignbyte(s1, s0, r) >> (8 * h);
+        const uint32_t sb = __builtin_amdgcn_alignbyte(s2, s1, r) >> (8 * h);
+        const uint32_t sv[4] = {sa, sa >> 16, sb, sb >> 16};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const _Float16 f = (_Float16)(float)(int8_t)(sv[u] & 0xFFu);
+            s[u] = h2{f, f};
+        }
+        d = f16_hw((lds4(a + 208) >> (8 * r)) & 0xFFFFu);
+    }
+    template <int KSI>
+    __device__ void ops(h8& whi, h8& wlo) const {
+        constexpr int u = KSI >> 1, k = 2 * (KSI & 1);
+        h2 vh[4], vl[4];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const uint32_t l = u & 1 ? hi[k + t] : lo[k + t];
+            const uint32_t hb = u < 2 ? qh[k + t] << (4 - 2 * u) : qh[k + t] >> (2 * u - 4);
+            const uint32_t c = ((u < 2 ? l : l >> 4) & 0x0F0F0F0Fu) | (hb & 0x30303030u);
+            h2 p0, p1;
+            byte_pairs(c, (_Float16)1056.0f, p0, p1);  // q - 32
+            vh[2 * t] = p0 * s[u];
+            vh[2 * t + 1] = p1 * s[u];
+            vl[2 * t] = __builtin_elementwise_fma(p0, s[u], -vh[2 * t]);
+            vl[2 * t + 1] = __builtin_elementwise_fma(p1, s[u], -vh[2 * t + 1]);
+        }
+        whi = h8{vh[0][0], vh[0][1], vh[1][0], vh[1][1], vh[2][0], vh[2][1], vh[3][0], vh[3][1]};
+        wlo = h8{vl[0][0], vl[0][1], vl[1][0], vl[1][1], vl[2][0], vl[2][1], vl[3][0], vl[3][1]};
+    }
+};
+
+// TT 16-token tiles; RW waves along the rows, 16 each (PAIR: the first half
+// gate, the second half up rows), in KG groups: group k takes super-blocks
+// b0 + k, b0 + KG + k, ...
+template <int F, int TT, int RW, int KG>
+struct Thin {
+    using Q = TQ<F>;
+    static constexpr int NW = RW * KG, BN = 16 * RW;      // waves; rows of a work-group
+    static constexpr int PI = (16 * Q::PPR + 63) / 64;    // copies per 16-row tile
+    static constexpr int PANEL = BN * Q::PPR * 16;
+    static constexpr int GBUF = PANEL + TT * (XSB + SSB), BUF = KG * GBUF;
+    static constexpr int NB = 3 * BUF <= 160 * 1024 ? 3 : 2;
+    static constexpr int LDS = NB * BUF;
+    static constexpr int XC = 16 / RW;                    // 1 KiB token copies per wave and tile
+    static constexpr int SW = RW < 8 ? RW : 8;            // waves that copy a tile's sums
+    static_assert(LDS <= 160 * 1024, "LDS");
+    static_assert(NW * TT * 1024 <= LDS, "the sums exchanged at the end");
+};
+
+template <int F, bool PAIR, int TT, int RW, int KG>
+__global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int sb_per_split) {
+    using Q = TQ<F>;
+    using TH = Thin<F, TT, RW, KG>;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[TH::LDS];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int rw = wave % RW, kg = wave / RW;
+    const int c = lane & 15, q = lane >> 4;
+    const RowTile rt = row_tile<PAIR>(a, blockIdx.x, TH::BN);
+    const int nsb = a.K / 256;
+    const int b0 = blockIdx.z * sb_per_split, b1 = min(nsb, b0 + sb_per_split);
+    // this wave's 16 rows: tile_row .. of base
+    const bool up = PAIR && rw >= RW / 2;
+    const int tile_row = rt.n0 + 16 * (PAIR ? rw % (RW / 2) : rw);
+    const uint8_t* const base = up ? a.w2 : rt.w;
+
+    // copy sources.  SHIFT: offsets from the matrix's aligned-down base, not
+    // yet aligned themselves (the super-block's start is added first)
+    const uint32_t mis = Q::SHIFT ? (uint32_t)(reinterpret_cast<uintptr_t>(base) & 15) : 0u;
+    const uint8_t* const wb = base - mis;
+    uint32_t woff[TH::PI], wp[TH::PI];
+#pragma unroll
+    for (int i = 0; i < TH::PI; ++i) {
+        const int L = min(64 * i + lane, 16 * Q::PPR - 1), r = L / Q::PPR;
+        wp[i] = 16u * (uint32_t)min(L - r * Q::PPR, Q::LAST);
+        woff[i] = (uint32_t)min(tile_row + r, rt.rows - 1) * (uint32_t)a.row_bytes + mis +
+                  (Q::SHIFT ? 0u : wp[i]);
+    }
+    constexpr int XB = XSB / RW, SB = SSB / TH::SW;  // this wave's share of a tile's operands
+    const uint8_t* const xb = reinterpret_cast<const uint8_t*>(a.xop) + XB * rw;
+    const uint8_t* const sbase = reinterpret_cast<const uint8_t*>(a.xsum) + SB * rw;
+    const uint32_t l0 = __builtin_amdgcn_readfirstlane(lds_addr(lds)) + kg * TH::GBUF;
+    const bool sums = rw < TH::SW;  // wave-uniform
+    // super-block sb, the it-th of this wave's group
+    auto issue = [&](int sb, int it) {
+        const uint32_t lb = l0 + (uint32_t)(it % TH::NB) * TH::BUF;
+        const uint32_t lp = lb + (uint32_t)(16 * rw) * (Q::PPR * 16), so = (uint32_t)sb * Q::SBB;
+#pragma unroll
+        for (int i = 0; i < TH::PI; ++i) {
+            if (64 * (i + 1) > 16 * Q::PPR && lane >= 16 * Q::PPR - 64 * i) continue;
+            if constexpr (Q::SHIFT) dma16s(((woff[i] + so) & ~15u) + wp[i], wb, lp + 1024 * i);
+            else dma16s(woff[i], wb + so, lp + 1024 * i);
+        }
+#pragma unroll
+        for (int T = 0; T < TT; ++T) {
+            const size_t blk = (size_t)T * nsb + sb;
+            const uint32_t lx = lb + TH::PANEL + T * XSB + XB * rw;
+#pragma unroll
+            for (int i = 0; i < TH::XC; ++i)
+                dma16s(16 * lane + 1024 * i, xb + blk * XSB, lx + 1024 * i);
+            if (sums && lane < SB / 16)
+                dma16s(16 * lane, sbase + blk * SSB, lb + TH::PANEL + TT * XSB + T * SSB + SB * rw);
+        }
+    };
+    // wait until this wave's copies of all but its newest `later` super-blocks
+    // are complete
+    auto wait = [&](bool later) {
+        constexpr int C = TH::PI + TH::XC * TT;
+        if (TH::NB == 2 || !later) wait_vm<0>();
+        else if (sums) wait_vm<C + TT>();
+        else wait_vm<C>();
+    };
+    // byte shift of lane row c's super-block in its pieces, before sb's
+    const uint32_t rsh = (uint32_t)(reinterpret_cast<uintptr_t>(base) & 15) +
+                         (uint32_t)min(tile_row + c, rt.rows - 1) * (uint32_t)a.row_bytes;
+
+    f32x4 acc[TT];
+#pragma unroll
+    for (int T = 0; T < TT; ++T) acc[T] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+#pragma unroll
+    for (int i = 0; i < TH::NB - 1; ++i)
+        if (b0 + KG * i + kg < b1) issue(b0 + KG * i + kg, i);
+    for (int it = 0; b0 + KG * it < b1; ++it) {
+        const int sb = b0 + KG * it + kg;  // (past b1: this group has none left)
+        wait(sb + KG < b1);
+        __syncthreads();
+        if (sb >= b1) continue;
+        if (sb + KG * (TH::NB - 1) < b1) issue(sb + KG * (TH::NB - 1), it + TH::NB - 1);
+        const uint8_t* buf = lds + kg * TH::GBUF + (it % TH::NB) * TH::BUF;
+        const uint8_t* xs = buf + TH::PANEL;
+        const uint8_t* ss = xs + TT * XSB;
+        Q w;
+        w.load(buf + (16 * rw + c) * (Q::PPR * 16),
+               Q::SHIFT ? (int)((rsh + (uint32_t)sb * Q::SBB) & 15u) : 0, q);
+        // The matrix cores' additions round toward zero, so a chain's error
+        // grows with its length times its magnitude: four chains of two for
+        // the large products (x_hi W_hi), one for the small ones
+        f32x4 D[4][TT], Dl[TT];
+        const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+        auto ks = [&](auto ki) {
+            constexpr int KSI = decltype(ki)::value;
+            h8 whi, wlo;
+            w.template ops<KSI>(whi, wlo);
+#pragma unroll
+            for (int T = 0; T < TT; ++T) {
+                const uint8_t* xp = xs + T * XSB + KSI * 2048 + 16 * lane;
+                const h8 xh = *reinterpret_cast<const h8*>(xp);
+                const h8 xl = *reinterpret_cast<const h8*>(xp + 1024);
+                f32x4& d = D[KSI >> 1][T];
+                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, whi, KSI & 1 ? d : z, 0, 0, 0);
+                Dl[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, whi, KSI ? Dl[T] : z, 0, 0, 0);
+                if constexpr (Q::SPLITW)
+                    Dl[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, wlo, Dl[T], 0, 0, 0);
+            }
+        };
+        ks(std::integral_constant<int, 0>{});
+        ks(std::integral_constant<int, 1>{});
+        ks(std::integral_constant<int, 2>{});
+        ks(std::integral_constant<int, 3>{});
+        ks(std::integral_constant<int, 4>{});
+        ks(std::integral_constant<int, 5>{});
+        ks(std::integral_constant<int, 6>{});
+        ks(std::integral_constant<int, 7>{});
+#pragma unroll
+        for (int T = 0; T < TT; ++T) {
+            const uint8_t* st = ss + T * SSB;
+            const float4 f = *reinterpret_cast<const float4*>(st + q * SG + 128);
+            const float fv[4] = {f.x, f.y, f.z, f.w};
+            f32x4 Dc = z, Dm = z;
+            if constexpr (Q::MIN) {
+                const h8 S = *reinterpret_cast<const h8*>(st + (lane >> 3) * SG + (lane & 7) * 16);
+                Dc = __builtin_amdgcn_mfma_f32_16x16x32_f16(S, w.cb, z, 0, 0, 0);
+                Dm = __builtin_amdgcn_mfma_f32_16x16x32_f16(S, w.mb, z, 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float v = ((D[0][T][i] + D[1][T][i]) + (D[2][T][i] + D[3][T][i])) + Dl[T][i];
+                if constexpr (Q::MIN) v = w.d * (v + Dc[i]) + w.dn * Dm[i];
+                else v *= w.d;
+                acc[T][i] = __builtin_fmaf(v, fv[i], acc[T][i]);
+            }
+        }
+    }
+    f32x4* const gs = reinterpret_cast<f32x4*>(lds);
+    if constexpr (KG > 1) {  // the groups' sums, added in group order
+        __syncthreads();
+#pragma unroll
+        for (int T = 0; T < TT; ++T)
+            if (kg > 0) gs[(wave * TT + T) * 64 + lane] = acc[T];
+        __syncthreads();
+        if (kg == 0) {
+#pragma unroll
+            for (int k = 1; k < KG; ++k)
+#pragma unroll
+                for (int T = 0; T < TT; ++T) acc[T] += gs[((k * RW + rw) * TT + T) * 64 + lane];
+        }
+    }
+    const bool split = gridDim.z > 1;
+    if constexpr (PAIR) {  // the up waves hand their sums to the gate waves
+        __syncthreads();
+#pragma unroll
+        for (int T = 0; T < TT; ++T)
+            if (kg == 0 && up && !split) gs[(wave * TT + T) * 64 + lane] = acc[T];
+        __syncthreads();
+    }
+    if (kg > 0 || (PAIR && up && !split)) return;
+    // lane (c, q): row c of the wave's tile, tokens 16 T + 4 q + i
+    const int cols = PAIR ? 2 * a.N : a.N, n = tile_row + c;
+    if (n >= rt.rows) return;
+    float* const out = split ? a.part + (size_t)blockIdx.z * a.M * cols : a.y;
+#pragma unroll
+    for (int T = 0; T < TT; ++T) {
+        f32x4 u = acc[T];
+        if constexpr (PAIR) {
+            if (!split) u = gs[((rw + RW / 2) * TT + T) * 64 + lane];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = 16 * T + 4 * q + i;
+            if (m >= a.M) continue;
+            if (split) {
+                out[(size_t)m * cols + rt.col + (up ? a.N : 0) + n] = acc[T][i];
+            } else if constexpr (PAIR) {
+                out[(size_t)m * a.N + n] = silu_mul(acc[T][i], u[i]);
+            } else {
+                float v = acc[T][i];
+                if (a.bias_mode == 1) v += n < a.bias_len ? a.bias[n] : 0.0f;
+                else if (a.bias_mode == 2) v += a.bias[(size_t)m * a.N + n];
+                out[(size_t)m * cols + rt.col + n] = v;
+            }
+        }
+    }
+}
+
+template <int F, int TT, int RW, int KG>
+hipError_t go(const MmqArgs& a, int splits, hipStream_t st) {
+    const int nsb = a.K / 256, sps = (nsb + splits - 1) / splits;
+    if (sps * (splits - 1) >= nsb) return hipErrorInvalidValue;  // an empty split
+    const dim3 grid(row_tiles(a, 16 * RW), 1, splits), wg(64 * RW * KG);
+    if (a.mm == MM_PAIR)
+        hipLaunchKernelGGL((mmqt_kernel<F, true, TT, RW, KG>), grid, wg, 0, st, a, sps);
+    else
+        hipLaunchKernelGGL((mmqt_kernel<F, false, TT, RW, KG>), grid, wg, 0, st, a, sps);
+    return hipGetLastError();
+}
+// Work-groups of 256, 128 or 64 rows; what does not fit LDS: Q6_K at 17..32
+// tokens in 256 rows, two groups of Q6_K in 128, 64 rows at 17..32 tokens.
+template <int F, int TT>
+hipError_t go_f(const MmqArgs& a, int rows, int splits, hipStream_t st) {
+    if constexpr (TT == 1 || F != Q6_K) {
+        if (rows == 256) return go<F, TT, 16, 1>(a, splits, st);
+    }
+    if (rows == 128) return go<F, TT, 8, TT == 1 && F != Q6_K ? 2 : 1>(a, splits, st);
+    if constexpr (TT == 1) {
+        if (rows == 64) return go<F, TT, 4, 2>(a, splits, st);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+bool mmqt_supported(int dtype) { return dtype == Q4_K || dtype == Q5_K || dtype == Q6_K; }
+bool mmqt_has_rows(int dtype, int M, int rows) {
+    if (rows == 128) return true;
+    return M <= 16 ? rows == 256 || rows == 64 : rows == 256 && dtype != Q6_K;
+}
+int mmqt_row_tiles(const MmqArgs& a, int rows) { return row_tiles(a, rows); }
+size_t mmqt_xop_bytes(int M, int K) { return (size_t)((M + 15) / 16) * (K / 256) * XSB; }
+size_t mmqt_sum_bytes(int M, int K) { return (size_t)((M + 15) / 16) * (K / 256) * SSB; }
+
+hipError_t launch_xprept(int dtype, const float* x, int M, int K, uint8_t* xop, uint8_t* xs,
+                         hipStream_t st) {
+    const dim3 grid(K / 256, (M + 15) / 16);
+    if (dtype == Q6_K) hipLaunchKernelGGL(xprept_kernel<true>, grid, dim3(256), 0, st, x, M, K, xop, xs);
+    else hipLaunchKernelGGL(xprept_kernel<false>, grid, dim3(256), 0, st, x, M, K, xop, xs);
+    return hipGetLastError();
+}
+
+hipError_t launch_mmqt(int dtype, const MmqArgs& a, int rows, int splits, hipStream_t st) {
+    if (a.M > 32 || a.K % 256 != 0 || splits < 1) return hipErrorInvalidValue;
+    auto tt = [&](auto f) {
+        constexpr int F = decltype(f)::value;
+        return a.M <= 16 ? go_f<F, 1>(a, rows, splits, st) : go_f<F, 2>(a, rows, splits, st);
+    };
+    switch (dtype) {
+        case Q4_K: return tt(FmtTag<Q4_K>{});
+        case Q5_K: return tt(FmtTag<Q5_K>{});
+        case Q6_K: return tt(FmtTag<Q6_K>{});
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace fq
