@@ -518,6 +518,172 @@ int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, 
     return e == hipSuccess ? FQ_OK : hip_fail(e);
 }
 
+// Whether the band kernel (fq_mmqs.hip) takes a call of 2..16 tokens; block:
+// a 32-element-block format there, ahead of the batch-1 kernel with several
+// tokens.
+struct BandRule {
+    bool block, takes;
+};
+BandRule band_rule(uint32_t dtype, const Geometry& g, int M, int K, int N, const void* w, int cus) {
+    // Q4_0 and Q8_0: rows that start 16-byte aligned
+    // (K a multiple of 256), 5..16 tokens, or 4 from 16 MB (below, other
+    // kernels take M = 4 0.4-0.7 us faster for Q4_0; Q8_0 only
+    // while the bands number at most one per CU: lm_head 157 us on the
+    // batch-1 kernel against 173), or, Q4_0 only, 3 from 16 MB with K of
+    // 14336 and more (3584 x 18944: 26.4 us on the batch-1 kernel).  At 3
+    // and 4 tokens Q4_0 needs at most one band per CU or at least eight
+    // (152064 rows at M = 4 129 against 151 us); from 5 tokens any count
+    // (18944 rows in three-tile bands, below: 24.5 against 27.5 us at M =
+    // 8).  Q8_0 takes any count (the fp16 MFMA path is slower at every one
+    // measured: 14336 x 4096 at M = 8 24.1 against 37.6 us)
+    const int bmt = fq::mmqs_max_tiles((int)dtype);
+    const long bands = ((long)N + 16 * bmt - 1) / (16 * bmt);
+    // (Q4_1 as Q4_0)
+    const bool q4x = dtype == FQ_DTYPE_Q4_0 || dtype == FQ_DTYPE_Q4_1;
+    const bool blk_band = (q4x || dtype == FQ_DTYPE_Q8_0) && K % 256 == 0 &&
+                          (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
+                          (M >= 5 ||
+                           ((M == 4 ? q4x || bands <= cus : M == 3 && q4x && K >= 14336) &&
+                            (int64_t)N * (K / g.be) * g.bb >= (16 << 20))) &&
+                          (dtype == FQ_DTYPE_Q8_0 || M >= 5 || bands <= cus ||
+                           bands >= 8L * cus);
+    // Q5_K (rows 16-byte aligned): 5..16 tokens; 4 while the bands number at
+    // most one per CU or at least eight per CU (18944 x 3584: 33.4 against
+    // 31.7 us on the fp16 MFMA path); 3 at K >= 14336 or eight bands per CU
+    // and more (3584 x 18944 54.1 -> 27.0 us at M = 4, lm_head at M = 3 166
+    // against about 150; 18944 x 3584 at M = 3 26.0 against 33); 2 at K >=
+    // 14336 (3584 x 18944: 53.9 on the fp16 MFMA path; lm_head at M = 2
+    // 111.5 against about 150 stays there)
+    const bool al16 = K % 256 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+    // Q5_0 and IQ4_NL: K >= 14336 from 2 tokens (3584 x 18944 at M = 2..8:
+    // 55.3 -> 27.9 and 47.4 -> 28.3 us), or 4..16 tokens in one round of
+    // bands (14336 x 4096 at M = 8: 33.2 -> 21.3, 29.2 -> 21.6); 18944 rows
+    // at M = 8 measured slower (35.5 against 32.7, 36.1 against 28.4).
+    // Q5_1 (160 KB of LDS per work-group): K >= 14336 only (43.8 -> 37.5;
+    // lm_head at M = 8 216 against 159)
+    const bool q5x_band =
+        al16 && M >= 2 &&
+        (((dtype == FQ_DTYPE_Q5_0 || dtype == FQ_DTYPE_IQ4_NL) &&
+          (K >= 14336 || (M >= 4 && bands <= cus))) ||
+         (dtype == FQ_DTYPE_Q5_1 && K >= 14336));
+    // Q3_K (rows at even addresses): K >= 14336 from two tokens (3584 x 18944
+    // 61 -> 28.7 us), 4..16 tokens for any row count (152064 x 3584 at M = 8
+    // 262 -> 184, 14336 x 4096 41.9 -> 32.0; equal at M = 4)
+    const bool q3k_band = dtype == FQ_DTYPE_Q3_K && K % 256 == 0 &&
+                          (reinterpret_cast<uintptr_t>(w) & 1) == 0 && M >= 2 &&
+                          (K >= 14336 || M >= 4);
+    const bool q5k_band =
+        q3k_band || (dtype == FQ_DTYPE_Q5_K && al16 &&
+         (M >= 5 || (M == 4 && (bands <= cus || bands >= 8L * cus)) ||
+          (M == 3 && (K >= 14336 || bands >= 8L * cus)) || (M == 2 && K >= 14336))) ||
+        q5x_band;
+    // Q4_K beyond one band per CU only above 8 tokens, which the int8 kernel
+    // does not take (18944 x 3584 at M = 16 31.2 against 34.4 us on the fp16
+    // MFMA path, 152064 x 3584 143.5 against 170.4; at M = 4..8 the int8
+    // kernel is faster, 21.1-27.5 against 30.2-30.4 and 108-130 against
+    // 137-139); Q4_K at M = 2, 3 is faster on the batch-1 and int8 kernels
+    const bool takes =
+        fq::mmqs_supported((int)dtype) && M >= (q5k_band ? 2 : blk_band ? 3 : 4) && M <= 16 && K > 0 &&
+        (dtype == FQ_DTYPE_Q4_K   ? N <= 16 * bmt * cus || M > 8
+         : dtype == FQ_DTYPE_Q6_K ? (reinterpret_cast<uintptr_t>(w) & 1) == 0
+         : (q4x || dtype == FQ_DTYPE_Q8_0) ? blk_band
+                                           : q5k_band);
+    return {blk_band, takes};
+}
+
+// Tiles of the band kernel's bands over N rows.
+int band_tiles(uint32_t dtype, int K, int N, int cus) {
+    const int bmt = fq::mmqs_max_tiles((int)dtype);
+    // Q8_0: two- or three-tile bands, whichever the estimate (rounds of
+    // work-groups x tiles x super-blocks per split) puts lower, three
+    // within 5 % (14336 x 4096 at M = 8: 24.2 us on two, 30.1 on three;
+    // 152064 x 3584: 175.4 / 170.0; 18944 x 3584: 31.3 / 29.6)
+    int tiles = bmt;
+    if (bmt == 4 && K / 256 < 32) {
+        // four-tile bands whose last round of work-groups is mostly idle
+        // (18944 rows: 296 bands on 256 CUs) take three tiles when those
+        // fill their rounds better (395 bands: Q4_0 at M = 8 27.5 ->
+        // 24.5 us, Q4_K at M = 16 31.3 -> 26.4, Q5_K 33.2 -> 27.7; at
+        // 14336 and 152064 rows four tiles measured faster)
+        auto fill = [&](int t) {
+            const long b = ((long)N + 16 * t - 1) / (16 * t);
+            return (double)b / (double)(((b + cus - 1) / cus) * cus);
+        };
+        if (N > 64L * cus && fill(4) < 0.6 && fill(3) > fill(4)) tiles = 3;
+    } else if (dtype == FQ_DTYPE_Q8_0) {
+        auto est = [&](int mt) {
+            int r = 0;
+            const long sp = mmqs_plan(N, K, cus, &r, mt);
+            const long wgs = ((long)N + r - 1) / r * sp;
+            return (double)((wgs + cus - 1) / cus) * (r / 16) *
+                   (double)((K / 256 + sp - 1) / sp);
+        };
+        tiles = est(3) <= 1.05 * est(2) ? 3 : 2;
+    }
+    return tiles;
+}
+
+// 2..16 tokens (by format and shape): token operands, then one pass over the
+// weights on the fp16 matrix cores, one band of rows per work-group (Q4_K at
+// 14336 x 4096: 19.2-19.7 us for every M in 4..16, against 21-30 us on the
+// int8 matrix-core and fp16 MFMA paths).  Several matrices (unsplit K only):
+// one token preparation and one launch, the same bits as one call per matrix.
+int run_band(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, const float* bias,
+             int bias_mode, int64_t bias_len, float* y, int M, int K, int N, int dev,
+             const DevInfo& di, hipStream_t st, uint8_t* fixed, size_t fixed_cap, bool x_ready) {
+    const int NC = K / 64;
+    const MmqPlan pl = plan_mmq(M, K, N, di.cus);
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    hipError_t e = hipSuccess;
+    const bool pair = ms.mm == fq::MM_PAIR;
+    int tiles = band_tiles(dtype, K, N, di.cus);
+    if (pair) tiles = tiles >= 4 ? 4 : 2;
+    int rpw = 0;
+    const int splits = mmqs_plan(pair ? 2 * N : N, K, di.cus, &rpw, tiles);
+    if (pair) rpw = 16 * ((rpw / 16 + 1) / 2);  // gate rows of a band, as many up rows
+    const size_t need = mmqs_need(M, K, N, di.cus, tiles);
+    std::unique_ptr<StreamScratch::Lease> lease;
+    uint8_t* buf = fixed;
+    if (fixed) {
+        if (need > fixed_cap) return FQ_ERR_WORKSPACE;
+    } else {
+        lease.reset(new StreamScratch::Lease(stream_scratch(dev, st, 0)));
+        const int rc = lease->get(need, st, &buf);
+        if (rc != FQ_OK) return rc;
+    }
+    fq::MmqArgs a{};
+    a.mm = ms.mm;
+    a.w = static_cast<const uint8_t*>(ms.w[0]);
+    a.w2 = static_cast<const uint8_t*>(ms.w[1]);
+    a.w3 = static_cast<const uint8_t*>(ms.w[2]);
+    a.n1 = ms.n[0];
+    a.n2 = ms.n[1];
+    a.n3 = ms.n[2];
+    a.xop = buf;
+    a.xsum = reinterpret_cast<const float*>(buf + al(pl.xop_b));
+    a.ex = reinterpret_cast<const int*>(buf + al(pl.xop_b) + al(pl.xsum_b));
+    a.part = splits > 1 ? reinterpret_cast<float*>(buf + al(pl.xop_b) + al(pl.xsum_b) +
+                                                   al(pl.ex_b))
+                        : nullptr;
+    a.y = y;
+    a.bias = bias;
+    a.bias_len = bias_mode ? bias_len : 0;
+    a.bias_mode = bias_mode;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.NC = NC;
+    a.row_bytes = (K / g.be) * g.bb;
+    if (!x_ready) {
+        e = fq::launch_xprep((int)dtype, x, M, K, NC, reinterpret_cast<_Float16*>(buf),
+                             const_cast<float*>(a.xsum), const_cast<int*>(a.ex), st);
+        if (e != hipSuccess) return hip_fail(e);
+    }
+    e = fq::launch_mmqs((int)dtype, a, rpw, 512, splits, st);
+    if (e != hipSuccess) return hip_fail(e);
+    return FQ_OK;
+}
+
 // band_x (optional): in, true when the stream's slot-0 workspace already
 // holds the band kernel's token operands of this x, M, K and format (a call
 // just before with the same x, M, K, N and format took the band kernel:
@@ -622,29 +788,8 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
         if (rc != kNotTaken) return rc;
     }
 
-    // Q4_0 and Q8_0 on the band kernel below: rows that start 16-byte aligned
-    // (K a multiple of 256), 5..16 tokens, or 4 from 16 MB (below, the
-    // kernels further down take M = 4 0.4-0.7 us faster for Q4_0; Q8_0 only
-    // while the bands number at most one per CU: lm_head 157 us on the
-    // batch-1 kernel against 173), or, Q4_0 only, 3 from 16 MB with K of
-    // 14336 and more (3584 x 18944: 26.4 us on the batch-1 kernel).  At 3
-    // and 4 tokens Q4_0 needs at most one band per CU or at least eight
-    // (152064 rows at M = 4 129 against 151 us); from 5 tokens any count
-    // (18944 rows in three-tile bands, below: 24.5 against 27.5 us at M =
-    // 8).  Q8_0 takes any count (the fp16 MFMA path is slower at every one
-    // measured: 14336 x 4096 at M = 8 24.1 against 37.6 us)
-    const int bmt = fq::mmqs_max_tiles((int)dtype);
-    const long bands = ((long)N + 16 * bmt - 1) / (16 * bmt);
-    // (Q4_1 as Q4_0)
-    const bool q4x = dtype == FQ_DTYPE_Q4_0 || dtype == FQ_DTYPE_Q4_1;
-    const bool blk_band = (q4x || dtype == FQ_DTYPE_Q8_0) && K % 256 == 0 &&
-                          (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
-                          (M >= 5 ||
-                           ((M == 4 ? q4x || bands <= di.cus : M == 3 && q4x && K >= 14336) &&
-                            (int64_t)N * (K / g.be) * g.bb >= (16 << 20))) &&
-                          (dtype == FQ_DTYPE_Q8_0 || M >= 5 || bands <= di.cus ||
-                           bands >= 8L * di.cus);
-    if (M >= 2 && M <= 4 && !blk_band && K > 0 && packable(dtype) &&
+    const BandRule rule = band_rule(dtype, g, M, K, N, w, di.cus);
+    if (M >= 2 && M <= 4 && !rule.block && K > 0 && packable(dtype) &&
         (dtype == FQ_DTYPE_Q6_K || (int64_t)N * (K / g.be) * g.bb >= (8 << 20))) {
         // two to four tokens: the same kernel dots each weight unit it reads
         // with every token's limbs, K split into slabs where the tokens'
@@ -656,121 +801,11 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
         if (rc != FQ_ERR_SHAPE) return rc;
     }
 
-    // Q5_K (rows 16-byte aligned): 5..16 tokens; 4 while the bands number at
-    // most one per CU or at least eight per CU (18944 x 3584: 33.4 against
-    // 31.7 us on the fp16 MFMA path); 3 at K >= 14336 or eight bands per CU
-    // and more (3584 x 18944 54.1 -> 27.0 us at M = 4, lm_head at M = 3 166
-    // against about 150; 18944 x 3584 at M = 3 26.0 against 33); 2 at K >=
-    // 14336 (3584 x 18944: 53.9 on the fp16 MFMA path; lm_head at M = 2
-    // 111.5 against about 150 stays there)
-    const bool al16 = K % 256 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
-    // Q5_0 and IQ4_NL: K >= 14336 from 2 tokens (3584 x 18944 at M = 2..8:
-    // 55.3 -> 27.9 and 47.4 -> 28.3 us), or 4..16 tokens in one round of
-    // bands (14336 x 4096 at M = 8: 33.2 -> 21.3, 29.2 -> 21.6); 18944 rows
-    // at M = 8 measured slower (35.5 against 32.7, 36.1 against 28.4).
-    // Q5_1 (160 KB of LDS per work-group): K >= 14336 only (43.8 -> 37.5;
-    // lm_head at M = 8 216 against 159)
-    const bool q5x_band =
-        al16 && M >= 2 &&
-        (((dtype == FQ_DTYPE_Q5_0 || dtype == FQ_DTYPE_IQ4_NL) &&
-          (K >= 14336 || (M >= 4 && bands <= di.cus))) ||
-         (dtype == FQ_DTYPE_Q5_1 && K >= 14336));
-    // Q3_K (rows at even addresses): K >= 14336 from two tokens (3584 x 18944
-    // 61 -> 28.7 us), 4..16 tokens for any row count (152064 x 3584 at M = 8
-    // 262 -> 184, 14336 x 4096 41.9 -> 32.0; equal at M = 4)
-    const bool q3k_band = dtype == FQ_DTYPE_Q3_K && K % 256 == 0 &&
-                          (reinterpret_cast<uintptr_t>(w) & 1) == 0 && M >= 2 &&
-                          (K >= 14336 || M >= 4);
-    const bool q5k_band =
-        q3k_band || (dtype == FQ_DTYPE_Q5_K && al16 &&
-         (M >= 5 || (M == 4 && (bands <= di.cus || bands >= 8L * di.cus)) ||
-          (M == 3 && (K >= 14336 || bands >= 8L * di.cus)) || (M == 2 && K >= 14336))) ||
-        q5x_band;
-    if (fq::mmqs_supported((int)dtype) && M >= (q5k_band ? 2 : blk_band ? 3 : 4) && M <= 16 &&
-        K > 0 &&
-        (dtype == FQ_DTYPE_Q4_K   ? N <= 16 * bmt * di.cus || M > 8
-         : dtype == FQ_DTYPE_Q6_K ? (reinterpret_cast<uintptr_t>(w) & 1) == 0
-         : (dtype == FQ_DTYPE_Q4_0 || dtype == FQ_DTYPE_Q4_1 || dtype == FQ_DTYPE_Q8_0)
-             ? blk_band
-             : q5k_band)) {
-        // (Q4_0, Q8_0: see blk_band.  Q4_K beyond one band per CU only above
-        // 8 tokens, which the int8 kernel does not take: 18944 x 3584 at M =
-        // 16 31.2 against 34.4 us on the fp16 MFMA path, 152064 x 3584 143.5
-        // against 170.4; at M = 4..8 the int8 kernel is faster, 21.1-27.5
-        // against 30.2-30.4 and 108-130 against 137-139)
-        // 2..16 tokens (by format and shape, above): token operands, then one
-        // pass over the weights on the fp16 matrix cores, one band of rows per
-        // work-group (Q4_K at 14336 x 4096: 19.2-19.7 us for every M in 4..16,
-        // against 21-30 us on the int8 matrix-core and fp16 MFMA paths; Q4_K
-        // at M = 2, 3 is faster on the batch-1 and int8 kernels, and at M =
-        // 4..8 on rows beyond one band per CU on the int8 kernel)
-        const int NC = K / 64;
-        const MmqPlan pl = plan_mmq(M, K, N, di.cus);
-        auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-        // Q8_0: two- or three-tile bands, whichever the estimate (rounds of
-        // work-groups x tiles x super-blocks per split) puts lower, three
-        // within 5 % (14336 x 4096 at M = 8: 24.2 us on two, 30.1 on three;
-        // 152064 x 3584: 175.4 / 170.0; 18944 x 3584: 31.3 / 29.6)
-        int tiles = bmt;
-        if (bmt == 4 && K / 256 < 32) {
-            // four-tile bands whose last round of work-groups is mostly idle
-            // (18944 rows: 296 bands on 256 CUs) take three tiles when those
-            // fill their rounds better (395 bands: Q4_0 at M = 8 27.5 ->
-            // 24.5 us, Q4_K at M = 16 31.3 -> 26.4, Q5_K 33.2 -> 27.7; at
-            // 14336 and 152064 rows four tiles measured faster)
-            auto fill = [&](int t) {
-                const long b = ((long)N + 16 * t - 1) / (16 * t);
-                return (double)b / (double)(((b + di.cus - 1) / di.cus) * di.cus);
-            };
-            if (N > 64L * di.cus && fill(4) < 0.6 && fill(3) > fill(4)) tiles = 3;
-        } else if (dtype == FQ_DTYPE_Q8_0) {
-            auto est = [&](int mt) {
-                int r = 0;
-                const long sp = mmqs_plan(N, K, di.cus, &r, mt);
-                const long wgs = ((long)N + r - 1) / r * sp;
-                return (double)((wgs + di.cus - 1) / di.cus) * (r / 16) *
-                       (double)((K / 256 + sp - 1) / sp);
-            };
-            tiles = est(3) <= 1.05 * est(2) ? 3 : 2;
-        }
-        int rpw = 0;
-        const int splits = mmqs_plan(N, K, di.cus, &rpw, tiles);
-        const size_t need = mmqs_need(M, K, N, di.cus, tiles);
-        std::unique_ptr<StreamScratch::Lease> lease;
-        uint8_t* buf = fixed;
-        if (fixed) {
-            if (need > fixed_cap) return FQ_ERR_WORKSPACE;
-        } else {
-            lease.reset(new StreamScratch::Lease(stream_scratch(dev, st, 0)));
-            const int rc = lease->get(need, st, &buf);
-            if (rc != FQ_OK) return rc;
-        }
-        fq::MmqArgs a{};
-        a.w = static_cast<const uint8_t*>(w);
-        a.xop = buf;
-        a.xsum = reinterpret_cast<const float*>(buf + al(pl.xop_b));
-        a.ex = reinterpret_cast<const int*>(buf + al(pl.xop_b) + al(pl.xsum_b));
-        a.part = splits > 1 ? reinterpret_cast<float*>(buf + al(pl.xop_b) + al(pl.xsum_b) +
-                                                       al(pl.ex_b))
-                            : nullptr;
-        a.y = y;
-        a.bias = bias;
-        a.bias_len = bias_mode ? bias_len : 0;
-        a.bias_mode = bias_mode;
-        a.M = M;
-        a.N = N;
-        a.K = K;
-        a.NC = NC;
-        a.row_bytes = (K / g.be) * g.bb;
-        if (!x_ready) {
-            e = fq::launch_xprep((int)dtype, x, M, K, NC, reinterpret_cast<_Float16*>(buf),
-                                 const_cast<float*>(a.xsum), const_cast<int*>(a.ex), st);
-            if (e != hipSuccess) return hip_fail(e);
-        }
-        e = fq::launch_mmqs((int)dtype, a, rpw, 512, splits, st);
-        if (e != hipSuccess) return hip_fail(e);
-        if (band_x) *band_x = true;
-        return FQ_OK;
+    if (rule.takes) {
+        const int rc = run_band(dtype, g, x, Mats{fq::MM_ONE, {w}, {N}}, bias, bias_mode, bias_len, y, M,
+                                K, N, dev, di, st, fixed, fixed_cap, x_ready);
+        if (rc == FQ_OK && band_x) *band_x = true;
+        return rc;
     }
 
     if ((M == 1 || M == 2) && K > 0) {
@@ -1362,6 +1397,21 @@ int fq_fused_qkv(uint32_t dtype, const float* x, const void* wq, const void* wk,
             rc = run_thin(dtype, g, x, ms, nullptr, 0, 0, y, M, K, Nt, dev, di, st, nullptr, 0);
         if (rc != kNotTaken) return rc;
     }
+    if (M >= 5 && M <= 16 && K < 32 * 256) {
+        // where each matrix would run on the band kernel (K unsplit): one
+        // launch over the three (Q4_K 4096 -> 4096 + 1024 + 1024 at M = 8: 33
+        // -> 12 us against a preparation, three bands and three copies)
+        bool band = true;
+        for (int i = 0; i < 3; ++i)
+            band = band && (ns[i] == 0 ||
+                            (band_rule(dtype, g, M, K, ns[i], ws[i], di.cus).takes &&
+                             !thin_takes(dtype, M, (int64_t)ns[i] * (K / g.be) * g.bb)));
+        if (band) {
+            const int rc = run_band(dtype, g, x, ms, nullptr, 0, 0, y, M, K, Nt, dev, di, st, nullptr,
+                                    0, false);
+            if (rc != FQ_ERR_WORKSPACE) return rc;
+        }
+    }
     uint8_t* buf = nullptr;
     const int nmax = std::max(Nq, std::max(Nk, Nv));
     StreamScratch::Lease lease(stream_scratch(dev, st, 1));
@@ -1442,6 +1492,13 @@ int fq_ffn_up_fused(uint32_t dtype, const float* x, const void* w_gate, const vo
         const int rc = run_prefill(dtype, g, x, Mats{fq::MM_PAIR, {w_gate, w_up}, {N}}, nullptr, 0, 0,
                                    y, M, K, N, dev, di, st, nullptr, 0);
         if (rc != kNotTaken) return rc;
+    }
+    if (M >= 5 && M <= 16 && K < 32 * 256 &&
+        band_rule(dtype, g, M, K, N, w_gate, di.cus).takes &&
+        band_rule(dtype, g, M, K, N, w_up, di.cus).takes) {  // one band launch, K unsplit
+        const int rc = run_band(dtype, g, x, Mats{fq::MM_PAIR, {w_gate, w_up}, {N}}, nullptr, 0, 0, y,
+                                M, K, N, dev, di, st, nullptr, 0, false);
+        if (rc != FQ_ERR_WORKSPACE) return rc;
     }
     uint8_t* buf = nullptr;
     StreamScratch::Lease lease(stream_scratch(dev, st, 1));

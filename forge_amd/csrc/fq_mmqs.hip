@@ -41,6 +41,7 @@
 #include "fq_formats.h"
 #include "fq_kernels.h"
 #include "fq_mfma16.h"
+#include "fq_mmtile.h"
 
 namespace fq {
 namespace {
@@ -347,7 +348,12 @@ struct Band<Q3_K> {
     }
 };
 
-template <int F, int TW, int WG, bool BIAS>
+// MODE 0: plain; 1: with a bias; 2: a gate/up pair, the band's first TW / 2
+// tiles gate and the others the same up rows (rows_per_wg gate rows).  Several
+// matrices side by side (MM_CAT): a band belongs to one of them.  A row's sum
+// does not depend on its band, so these forms give the bits of one call per
+// matrix.
+template <int F, int TW, int WG, int MODE>
 __global__ __launch_bounds__(WG) void mmqs_kernel(MmqArgs a, int rows_per_wg, int sb_per_split) {
     using B = Band<F>;
     constexpr int W = WG / 64;
@@ -361,9 +367,16 @@ __global__ __launch_bounds__(WG) void mmqs_kernel(MmqArgs a, int rows_per_wg, in
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4;  // A operand: row r, element group q
     const int c = lane & 15;                 // D and B operands: token column c
-    const int lo = blockIdx.x * rows_per_wg;
-    const int hi = min(a.N, lo + rows_per_wg);
+    constexpr bool PAIR = MODE == 2;
+    constexpr int HT = PAIR ? TW / 2 : TW;  // tiles per matrix
+    static_assert(!PAIR || TW % 2 == 0, "a pair's tiles");
+    const RowTile rt = row_tile<PAIR>(a, blockIdx.x, PAIR ? 2 * rows_per_wg : rows_per_wg);
+    const int lo = rt.n0;
+    const int hi = min(rt.rows, lo + rows_per_wg);
     const int ntl = (hi - lo + 15) >> 4;
+    // first row of tile t (its matrix: tile_w)
+    auto tile_lo = [&](int t) { return min(lo + 16 * (t % HT), rt.rows - 1); };
+    auto tile_w = [&](int t) { return PAIR && t >= HT ? a.w2 : rt.w; };
     // this work-group's super-blocks: all of K, or split blockIdx.y of a K
     // split whose partial sums go to slab blockIdx.y of a.part
     const int sb0 = blockIdx.y * sb_per_split;
@@ -372,14 +385,14 @@ __global__ __launch_bounds__(WG) void mmqs_kernel(MmqArgs a, int rows_per_wg, in
     // piece p of a tile's panel (rows clamped into the matrix)
     const uint8_t* prow[TW];
 #pragma unroll
-    for (int t = 0; t < TW; ++t) prow[t] = a.w + (size_t)min(lo + 16 * t, a.N - 1) * a.row_bytes;
+    for (int t = 0; t < TW; ++t) prow[t] = tile_w(t) + (size_t)tile_lo(t) * a.row_bytes;
     // pieces per lane, per panel row
     constexpr int NPL = B::NPL, PPR = B::PANEL / 256;
     int pp[NPL], rmax[TW];
 #pragma unroll
     for (int i = 0; i < NPL; ++i) pp[i] = min(lane + 64 * i, B::PIECES - 1);
 #pragma unroll
-    for (int t = 0; t < TW; ++t) rmax[t] = a.N - 1 - min(lo + 16 * t, a.N - 1);
+    for (int t = 0; t < TW; ++t) rmax[t] = rt.rows - 1 - tile_lo(t);
 
     f32x4 acc[TW];
 #pragma unroll
@@ -594,24 +607,33 @@ __global__ __launch_bounds__(WG) void mmqs_kernel(MmqArgs a, int rows_per_wg, in
         if (m >= a.M || row >= hi) continue;
         float v = part[0][t][rr][m];
         for (int w = 1; w < W; ++w) v += part[w][t][rr][m];
-        if constexpr (BIAS) {
+        if constexpr (PAIR) {
+            float u = part[0][HT + t][rr][m];
+            for (int w = 1; w < W; ++w) u += part[w][HT + t][rr][m];
+            v = silu_mul(v, u);
+        }
+        if constexpr (MODE == 1) {
             if (!split) {
                 if (a.bias_mode == 2) v += a.bias[(size_t)m * a.N + row];
                 else v += row < a.bias_len ? a.bias[row] : 0.0f;
             }
         }
-        out[(size_t)m * a.N + row] = v;
+        out[(size_t)m * a.N + rt.col + row] = v;
     }
 }
 
 template <int F, int TW, int WG>
-const void* sfn(bool bias) {
-    return bias ? reinterpret_cast<const void*>(&mmqs_kernel<F, TW, WG, true>)
-                : reinterpret_cast<const void*>(&mmqs_kernel<F, TW, WG, false>);
+const void* sfn(int mode) {
+    if constexpr (TW % 2 == 0 && WG == 512) {
+        if (mode == 2) return reinterpret_cast<const void*>(&mmqs_kernel<F, TW, WG, 2>);
+    }
+    if (mode == 2) return nullptr;
+    return mode == 1 ? reinterpret_cast<const void*>(&mmqs_kernel<F, TW, WG, 1>)
+                     : reinterpret_cast<const void*>(&mmqs_kernel<F, TW, WG, 0>);
 }
 
 template <int F, int WG>
-const void* sfn_tw(int tw, bool bias) {
+const void* sfn_tw(int tw, int bias) {
     switch (tw) {
         case 1: return sfn<F, 1, WG>(bias);
         case 2: return sfn<F, 2, WG>(bias);
@@ -645,37 +667,40 @@ int mmqs_max_tiles(int dtype) { return dtype == Q8_0 ? 3 : dtype == Q6_K || dtyp
 
 hipError_t launch_mmqs(int dtype, const MmqArgs& a, int rows_per_wg, int wg, int splits,
                        hipStream_t st) {
-    const int tw = (rows_per_wg + 15) / 16;
+    const bool pair = a.mm == MM_PAIR;
+    const int tw = (rows_per_wg + 15) / 16 * (pair ? 2 : 1);
+    const int mode = pair ? 2 : a.bias_mode != 0;
+    if ((pair || a.mm == MM_CAT) && (splits != 1 || a.bias_mode != 0)) return hipErrorInvalidValue;
     const void* fn = nullptr;
     if (dtype == Q4_K) {
-        fn = wg == 256   ? sfn_tw<Q4_K, 256>(tw, a.bias_mode != 0)
-             : wg == 1024 ? sfn_tw<Q4_K, 1024>(tw, a.bias_mode != 0)
-                          : sfn_tw<Q4_K, 512>(tw, a.bias_mode != 0);
+        fn = wg == 256   ? sfn_tw<Q4_K, 256>(tw, mode)
+             : wg == 1024 ? sfn_tw<Q4_K, 1024>(tw, mode)
+                          : sfn_tw<Q4_K, 512>(tw, mode);
     } else if (dtype == Q4_0 || dtype == Q4_1 || dtype == Q8_0 || dtype == Q5_K ||
                dtype == Q5_0 || dtype == Q5_1 || dtype == IQ4_NL) {
         // rows must start 16-byte aligned (the panel loads are 16 bytes)
         if (a.K % 256 != 0 || a.row_bytes % 16 != 0 ||
             (reinterpret_cast<uintptr_t>(a.w) & 15) != 0 || wg != 512)
             return hipErrorInvalidValue;
-        fn = dtype == Q4_0   ? sfn_tw<Q4_0, 512>(tw, a.bias_mode != 0)
-             : dtype == Q4_1 ? sfn_tw<Q4_1, 512>(tw, a.bias_mode != 0)
-             : dtype == Q5_K ? sfn_tw<Q5_K, 512>(tw, a.bias_mode != 0)
-             : dtype == Q5_0 ? sfn_tw<Q5_0, 512>(tw, a.bias_mode != 0)
-             : dtype == Q5_1 ? sfn_tw<Q5_1, 512>(tw, a.bias_mode != 0)
-             : dtype == IQ4_NL ? sfn_tw<IQ4_NL, 512>(tw, a.bias_mode != 0)
-                             : sfn_tw<Q8_0, 512>(tw, a.bias_mode != 0);
+        fn = dtype == Q4_0   ? sfn_tw<Q4_0, 512>(tw, mode)
+             : dtype == Q4_1 ? sfn_tw<Q4_1, 512>(tw, mode)
+             : dtype == Q5_K ? sfn_tw<Q5_K, 512>(tw, mode)
+             : dtype == Q5_0 ? sfn_tw<Q5_0, 512>(tw, mode)
+             : dtype == Q5_1 ? sfn_tw<Q5_1, 512>(tw, mode)
+             : dtype == IQ4_NL ? sfn_tw<IQ4_NL, 512>(tw, mode)
+                             : sfn_tw<Q8_0, 512>(tw, mode);
     } else if (dtype == Q6_K || dtype == Q3_K) {  // rows at even addresses (shifts <= 14)
         if (a.K % 256 != 0 || (reinterpret_cast<uintptr_t>(a.w) & 1) != 0 || wg != 512)
             return hipErrorInvalidValue;
-        fn = dtype == Q6_K ? sfn_tw<Q6_K, 512>(tw, a.bias_mode != 0)
-                           : sfn_tw<Q3_K, 512>(tw, a.bias_mode != 0);
+        fn = dtype == Q6_K ? sfn_tw<Q6_K, 512>(tw, mode)
+                           : sfn_tw<Q3_K, 512>(tw, mode);
     }
     if (!fn) return hipErrorInvalidValue;
     const int nsb = a.K / 256;
     if (splits < 1 || splits > nsb || (splits > 1 && !a.part)) return hipErrorInvalidValue;
     int sps = (nsb + splits - 1) / splits;
     splits = (nsb + sps - 1) / sps;  // no empty split
-    const int grid = (a.N + rows_per_wg - 1) / rows_per_wg;
+    const int grid = row_tiles(a, pair ? 2 * rows_per_wg : rows_per_wg);
     MmqArgs args = a;
     int rpw = rows_per_wg;
     void* params[] = {&args, &rpw, &sps};
