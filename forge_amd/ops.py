@@ -44,8 +44,23 @@ class QWeight:
         return cls(t, int(dtype), int(N), int(K))
 
 
+# The current stream's handle by device index, without building a
+# torch.cuda.Stream object around it (2.0 -> 0.15 us of every call here, whose
+# kernels run 4 to 7 us at small-model sizes).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_ptr(t: torch.Tensor):
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def _f32_on(v: torch.Tensor, like: torch.Tensor) -> torch.Tensor:
+    """v as contiguous fp32 on like's device (like: fp32), itself if it is that already."""
+    if v.dtype != torch.float32 or v.device != like.device:
+        v = v.to(device=like.device, dtype=torch.float32)
+    return v.contiguous()
 
 
 def matmul_transB(a: torch.Tensor, b: QWeight, bias: torch.Tensor | None = None) -> torch.Tensor:
@@ -58,10 +73,10 @@ def matmul_transB(a: torch.Tensor, b: QWeight, bias: torch.Tensor | None = None)
                            f"b_shape=[{b.N},{b.K}]")
     if a.dtype != torch.float32 or not a.is_cuda or not a.is_contiguous():
         raise RuntimeError("matmul_transB: input must be a contiguous fp32 device tensor")
-    out = torch.empty((M, b.N), dtype=torch.float32, device=a.device)
+    out = a.new_empty((M, b.N))
     bias_ptr, bias_ndim, bias_len = None, 0, 0
     if bias is not None:
-        bias = bias.to(device=a.device, dtype=torch.float32).contiguous()
+        bias = _f32_on(bias, a)
         bias_ptr, bias_ndim, bias_len = bias.data_ptr(), bias.dim(), bias.numel()
     st = _lib.lib().fq_matmul_transB(b.dtype, a.data_ptr(), b.data.data_ptr(), bias_ptr,
                                      bias_ndim, bias_len, out.data_ptr(), M, K, b.N,
@@ -75,7 +90,7 @@ def matmul_transB(a: torch.Tensor, b: QWeight, bias: torch.Tensor | None = None)
 def gemv(x: torch.Tensor, b: QWeight) -> torch.Tensor:
     """Batch-1 GEMV through fq_gemv (x: [K] or [1, K])."""
     xv = x.reshape(-1)
-    y = torch.empty((b.N,), dtype=torch.float32, device=x.device)
+    y = x.new_empty((b.N,), dtype=torch.float32)
     _lib.check(_lib.lib().fq_gemv(b.dtype, xv.data_ptr(), b.data.data_ptr(), y.data_ptr(),
                                   b.K, b.N, _stream_ptr(x)), "fq_gemv")
     return y
@@ -83,7 +98,7 @@ def gemv(x: torch.Tensor, b: QWeight) -> torch.Tensor:
 
 def gemv_batch(x: torch.Tensor, b: QWeight) -> torch.Tensor:
     M = x.shape[0]
-    y = torch.empty((M, b.N), dtype=torch.float32, device=x.device)
+    y = x.new_empty((M, b.N), dtype=torch.float32)
     _lib.check(_lib.lib().fq_gemv_batch(b.dtype, x.data_ptr(), b.data.data_ptr(), y.data_ptr(),
                                         M, b.K, b.N, _stream_ptr(x)), "fq_gemv_batch")
     return y
@@ -91,7 +106,7 @@ def gemv_batch(x: torch.Tensor, b: QWeight) -> torch.Tensor:
 
 def matmul_prefill(x: torch.Tensor, b: QWeight) -> torch.Tensor:
     M = x.shape[0]
-    y = torch.empty((M, b.N), dtype=torch.float32, device=x.device)
+    y = x.new_empty((M, b.N), dtype=torch.float32)
     _lib.check(_lib.lib().fq_matmul_prefill(b.dtype, x.data_ptr(), b.data.data_ptr(),
                                             y.data_ptr(), M, b.K, b.N, _stream_ptr(x)),
                "fq_matmul_prefill")
@@ -150,10 +165,10 @@ def gemv_packed(x: torch.Tensor, p: PackedWeight, bias: torch.Tensor | None = No
     xv = x.reshape(-1)
     if xv.numel() != p.K:
         raise RuntimeError(f"gemv_packed dimension mismatch: K={xv.numel()} K2={p.K}")
-    y = torch.empty((p.N,), dtype=torch.float32, device=x.device)
+    y = x.new_empty((p.N,), dtype=torch.float32)
     bptr, blen = None, 0
     if bias is not None:
-        bias = bias.to(device=x.device, dtype=torch.float32).contiguous()
+        bias = _f32_on(bias, x)
         bptr, blen = bias.data_ptr(), bias.numel()
     _lib.check(_lib.lib().fq_gemv_packed(p.dtype, xv.data_ptr(), p.data.data_ptr(), bptr, blen,
                                          y.data_ptr(), p.K, p.N, _stream_ptr(x)), "fq_gemv_packed")
@@ -171,7 +186,7 @@ def ffn_up_fused(x: torch.Tensor, w_gate: QWeight, w_up: QWeight) -> torch.Tenso
     if K != w_gate.K:
         raise RuntimeError(f"ffn_up_fused dimension mismatch: K={K} K2={w_gate.K}")
     x = x.contiguous()
-    y = torch.empty((M, w_gate.N), dtype=torch.float32, device=x.device)
+    y = x.new_empty((M, w_gate.N), dtype=torch.float32)
     _lib.check(_lib.lib().fq_ffn_up_fused(w_gate.dtype, x.data_ptr(), w_gate.data.data_ptr(),
                                           w_up.data.data_ptr(), y.data_ptr(), M, K, w_gate.N,
                                           _stream_ptr(x)), "fq_ffn_up_fused")
@@ -185,7 +200,7 @@ def ffn_up_fused_packed(x: torch.Tensor, w_gate: PackedWeight, w_up: PackedWeigh
         raise RuntimeError("ffn_up_fused: gate and up weights differ in dtype or shape")
     if xv.numel() != w_gate.K:
         raise RuntimeError(f"ffn_up_fused dimension mismatch: K={xv.numel()} K2={w_gate.K}")
-    y = torch.empty((w_gate.N,), dtype=torch.float32, device=x.device)
+    y = x.new_empty((w_gate.N,), dtype=torch.float32)
     _lib.check(_lib.lib().fq_ffn_up_fused_packed(w_gate.dtype, xv.data_ptr(),
                                                  w_gate.data.data_ptr(), w_up.data.data_ptr(),
                                                  y.data_ptr(), w_gate.K, w_gate.N,
@@ -209,7 +224,7 @@ def fused_qkv(x: torch.Tensor, wq: QWeight, wk: QWeight, wv: QWeight) -> torch.T
     M, K = x.shape
     _same_k("fused_qkv", K, wq, wk, wv)
     x = x.contiguous()
-    y = torch.empty((M, wq.N + wk.N + wv.N), dtype=torch.float32, device=x.device)
+    y = x.new_empty((M, wq.N + wk.N + wv.N), dtype=torch.float32)
     _lib.check(_lib.lib().fq_fused_qkv(wq.dtype, x.data_ptr(), wq.data.data_ptr(),
                                        wk.data.data_ptr(), wv.data.data_ptr(), y.data_ptr(), M, K,
                                        wq.N, wk.N, wv.N, _stream_ptr(x)), "fq_fused_qkv")
@@ -221,7 +236,7 @@ def fused_qkv_packed(x: torch.Tensor, wq: PackedWeight, wk: PackedWeight,
     """Batch-1 fused QKV over packed weights (x: [K] or [1, K]); returns [Nq + Nk + Nv]."""
     xv = x.reshape(-1)
     _same_k("fused_qkv", xv.numel(), wq, wk, wv)
-    y = torch.empty((wq.N + wk.N + wv.N,), dtype=torch.float32, device=x.device)
+    y = x.new_empty((wq.N + wk.N + wv.N,), dtype=torch.float32)
     _lib.check(_lib.lib().fq_fused_qkv_packed(wq.dtype, xv.data_ptr(), wq.data.data_ptr(),
                                               wk.data.data_ptr(), wv.data.data_ptr(),
                                               y.data_ptr(), wq.K, wq.N, wk.N, wv.N,
@@ -239,8 +254,8 @@ def ffn_down_residual(x: torch.Tensor, w: QWeight, residual: torch.Tensor) -> to
     if tuple(residual.shape) != (M, w.N):
         raise RuntimeError("ffn_down_residual: residual shape mismatch")
     x = x.contiguous()
-    r = residual.to(device=x.device, dtype=torch.float32).contiguous()
-    y = torch.empty((M, w.N), dtype=torch.float32, device=x.device)
+    r = _f32_on(residual, x)
+    y = x.new_empty((M, w.N), dtype=torch.float32)
     _lib.check(_lib.lib().fq_ffn_down_residual(w.dtype, x.data_ptr(), w.data.data_ptr(),
                                                r.data_ptr(), y.data_ptr(), M, K, w.N,
                                                _stream_ptr(x)), "fq_ffn_down_residual")
@@ -252,10 +267,10 @@ def ffn_down_residual_packed(x: torch.Tensor, w: PackedWeight,
     """Batch-1 x W^T + residual over packed weights; returns [N]."""
     xv = x.reshape(-1)
     _same_k("ffn_down_residual", xv.numel(), w)
-    r = residual.reshape(-1).to(device=x.device, dtype=torch.float32).contiguous()
+    r = _f32_on(residual.reshape(-1), x)
     if r.numel() != w.N:
         raise RuntimeError("ffn_down_residual: residual shape mismatch")
-    y = torch.empty((w.N,), dtype=torch.float32, device=x.device)
+    y = x.new_empty((w.N,), dtype=torch.float32)
     _lib.check(_lib.lib().fq_ffn_down_residual_packed(w.dtype, xv.data_ptr(), w.data.data_ptr(),
                                                       r.data_ptr(), y.data_ptr(), w.K, w.N,
                                                       _stream_ptr(x)),
