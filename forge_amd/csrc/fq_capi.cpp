@@ -7,8 +7,8 @@
 // of fq_gemv1.hip under about 4 MB of weights); M = 2..4
 // the same batch-1 kernels with each weight unit dotted with every token;
 // M = 2..16 (by format and shape) the band kernel of fq_mmqs.hip
-// (Q6_K M = 4 on wide matrices: three tokens, then the fourth); M = 4..16 of
-// Q4_K, Q5_K and Q6_K on 24 MB and more and M = 17..32 the kernel of
+// (Q6_K M = 4 on wide matrices: three tokens, then the fourth); M = 4..16 on
+// matrices of 24 to 48 MB and more and M = 17..32 the kernel of
 // fq_mmqt.hip; M > 32 the prefill kernels
 // of fq_mmqk.hip and fq_mmqp.hip (rows in 16-byte chunks, K a multiple of 256); the rest --
 // the reference's batched GEMV (1 < M <= 32) and dequant + GEMM prefill
@@ -401,42 +401,43 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
     return e == hipSuccess ? FQ_OK : hip_fail(e);
 }
 
-// Small batches of Q4_K, Q5_K and Q6_K with the token operands shared by the
-// rows of a work-group (fq_mmqt.hip).
+// Small batches with the token operands shared by the rows of a work-group
+// (fq_mmqt.hip: every format but Q3_K).
 struct MmqtPlan {
     int rows, splits;
     size_t xop_b, sum_b, part_b, total;
 };
 
 // Rows per work-group and K-splits of the smallest estimated time: rounds of
-// work-groups x (iterations of one or two super-blocks + 1.5 us to fill the
-// pipeline), and for a split the slab sum (3.5 us and each slab written and
-// read at 4 TB/s).  us per iteration measured at 14336 x 4096 on 224
-// work-groups.
+// work-groups x (iterations of one super-block per wave group + 1.5 us to fill
+// the pipeline), and for a split the slab sum (3.5 us and each slab written
+// and read at 4 TB/s).  An iteration's time is what 14336 x 4096 measured on
+// 224 work-groups, or its weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x
+// 3584 at M = 16: 134 us on 128 rows, 156 on 64).
 MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
-    struct Shape {
-        int rows, kg;
-        double t;
-    };
     const bool q6 = dtype == FQ_DTYPE_Q6_K, wide = a.M > 16;
-    const Shape shapes[3] = {{256, 1, q6 ? 2.7 : wide ? 2.6 : 2.0},
-                             {128, q6 || wide ? 1 : 2, q6 ? (wide ? 2.2 : 1.7) : wide ? 1.6 : 1.7},
-                             {64, 2, q6 ? 1.8 : 1.3}};
     MmqtPlan p{};
     const int nsb = a.K / 256;
+    const double sb_bytes = (double)a.row_bytes / nsb;
     double best = 0.0;
-    for (const Shape& s : shapes) {
-        if (!fq::mmqt_has_rows((int)dtype, a.M, s.rows)) continue;
-        const long tiles = fq::mmqt_row_tiles(a, s.rows);
+    for (int rows : {256, 128, 64}) {
+        const int kg = fq::mmqt_groups((int)dtype, a.M, rows);
+        if (kg == 0) continue;
+        const double it = rows == 256   ? (q6 ? 2.7 : wide ? 2.6 : 2.0)
+                          : rows == 128 ? (q6 ? (wide ? 2.2 : 1.7) : wide ? 1.6 : 1.7)
+                                        : (q6 ? 1.8 : 1.3);
+        const long tiles = fq::mmqt_row_tiles(a, rows);
         for (int sp = 1; sp <= std::min(16, nsb); ++sp) {
             const int sps = (nsb + sp - 1) / sp;
             if (sps * (sp - 1) >= nsb) continue;  // an empty split
+            const double busy = (double)std::min<long>(tiles * sp, cus);
+            const double step = std::max(it, busy * kg * rows * sb_bytes / 5e6);
             const double t = (double)((tiles * sp + cus - 1) / cus) *
-                                 (1.5 + s.t * ((sps + s.kg - 1) / s.kg)) +
+                                 (1.5 + step * ((sps + kg - 1) / kg)) +
                              (sp > 1 ? 3.5 + (sp + 1.0) * a.M * fq::mm_cols(a) * 4.0 / 4e6 : 0.0);
             if (p.rows == 0 || t < best) {
                 best = t;
-                p.rows = s.rows;
+                p.rows = rows;
                 p.splits = sp;
             }
         }
@@ -450,17 +451,34 @@ MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
     return p;
 }
 
-// Whether 2..32 tokens on one matrix of this size (or on a gate/up pair of two)
-// go there.  17..32 tokens always (the fp16 MFMA path: Q4_K 4096 x 4096 at M =
-// 32 20.8 -> 14.7 us, 14336 x 4096 40.2 -> 23.2, Q6_K 4096 x 14336 56.4 ->
-// 29.0).  Up to 16 from 24 MB (Q6_K: 32 MB) of weights: below, the band
-// kernel's bands fill the chip without a K split and its slab sum (Q4_K 8192 x
-// 4096, 19 MB, M = 8: 12.6 us there, 13.5 here; 14336 x 4096, 33 MB: 18.7 and
-// 16.3; Q6_K 8192 x 4096, 28 MB: 16.5 and 16.8; 14336 x 4096: 27.6 and 20.9;
-// 152064 x 3584 at M = 16 216 and 139).
+// Whether 4..32 tokens on one matrix of this size go there.  17..32 tokens
+// always (the fp16 MFMA path: Q4_K 4096 x 4096 at M = 32 20.8 -> 14.7 us, 14336 x
+// 4096 40.2 -> 23.2, Q8_0 40.5 -> 25.2, Q6_K 4096 x 14336 56.4 -> 29.0).  Up to
+// 16 from 24 MiB of Q4_K and Q5_K, 48 of Q8_0, 32 of the others: below, the band
+// kernel's bands fill the chip without a K split and its slab sum (M = 8: Q4_K
+// 8192 x 4096, 19 MB, 12.6 us there, 13.5 here, 14336 x 4096, 33 MB, 18.7 and
+// 16.3; Q6_K 28 MB 16.5 and 16.8, 48 MB 27.6 and 20.9; Q8_0 36 MB 14.1 and
+// 15.3, 62 MB 23.5 and 19.2; Q4_0 33 MB 17.8 and 17.3, 38 MB 24.0 and 20.0;
+// 152064 x 3584: Q4_0 132 and 100, Q8_0 171 and 133, Q6_K 211 and 131).
 bool thin_takes(uint32_t dtype, int M, int64_t bytes) {
-    if (!fq::mmqt_supported((int)dtype) || M < 2 || M > 32) return false;
-    return M > 16 || bytes >= (dtype == FQ_DTYPE_Q6_K ? 32LL << 20 : 24LL << 20);
+    if (!fq::mmqt_supported((int)dtype) || M < 4 || M > 32) return false;
+    const int64_t mib = dtype == FQ_DTYPE_Q4_K || dtype == FQ_DTYPE_Q5_K ? 24
+                        : dtype == FQ_DTYPE_Q8_0                        ? 48
+                                                                        : 32;
+    return M > 16 || bytes >= mib << 20;
+}
+
+// Whether a gate/up pair of such matrices goes there: as one matrix, or two to
+// four tokens, which otherwise take two launches and a SiLU pass (M = 4: Q4_0
+// 5632 x 2048 18.4 -> 11.6 us, 18944 x 3584 52.4 -> 36; M = 2: 13.9 -> 11.6), but
+// not two on large matrices of the formats whose batch-1 kernel then reads at
+// nearly the rate of one token (M = 2: Q4_0 18944 x 3584 30.2 against 35.8, Q6_K
+// 37.6 against 44.3, Q8_0 14336 x 4096 33.8 against 34.5).
+bool thin_takes_pair(uint32_t dtype, int M, int64_t bytes) {
+    if (!fq::mmqt_supported((int)dtype) || M < 2) return false;
+    if (M == 2 && (dtype == FQ_DTYPE_Q4_0 || dtype == FQ_DTYPE_Q6_K || dtype == FQ_DTYPE_Q8_0))
+        return bytes < 24 << 20;
+    return M <= 4 || thin_takes(dtype, M, bytes);
 }
 
 // kNotTaken: another kernel runs the call (also where the workspace cannot
@@ -468,7 +486,7 @@ bool thin_takes(uint32_t dtype, int M, int64_t bytes) {
 int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, const float* bias,
              int bias_mode, int64_t bias_len, float* y, int M, int K, int N, int dev,
              const DevInfo& di, hipStream_t st, uint8_t* fixed, size_t fixed_cap) {
-    if (K <= 0 || K % 256 != 0) return kNotTaken;
+    if (!fq::mmqt_supported((int)dtype) || M < 2 || M > 32 || K <= 0 || K % 256 != 0) return kNotTaken;
     const bool q6k = dtype == FQ_DTYPE_Q6_K;
     const int64_t rb = (int64_t)(K / g.be) * g.bb;
     for (int i = 0; i < 3; ++i) {
@@ -782,7 +800,7 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
         return FQ_OK;
     }
 
-    if (M >= 4 && thin_takes(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {
+    if (thin_takes(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {
         const int rc = run_thin(dtype, g, x, Mats{fq::MM_ONE, {w}, {N}}, bias, bias_mode, bias_len, y, M,
                                 K, N, dev, di, st, fixed, fixed_cap);
         if (rc != kNotTaken) return rc;
@@ -1483,22 +1501,24 @@ int fq_ffn_up_fused(uint32_t dtype, const float* x, const void* w_gate, const vo
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e);
     const DevInfo di = device_info(dev);
-    if (thin_takes(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {  // gate and up rows in one launch
-        const int rc = run_thin(dtype, g, x, Mats{fq::MM_PAIR, {w_gate, w_up}, {N}}, nullptr, 0, 0, y, M,
-                                K, N, dev, di, st, nullptr, 0);
-        if (rc != kNotTaken) return rc;
-    }
     if (M > 32) {  // one prefill launch, gate and up rows in each tile
         const int rc = run_prefill(dtype, g, x, Mats{fq::MM_PAIR, {w_gate, w_up}, {N}}, nullptr, 0, 0,
                                    y, M, K, N, dev, di, st, nullptr, 0);
         if (rc != kNotTaken) return rc;
     }
-    if (M >= 5 && M <= 16 && K < 32 * 256 &&
-        band_rule(dtype, g, M, K, N, w_gate, di.cus).takes &&
-        band_rule(dtype, g, M, K, N, w_up, di.cus).takes) {  // one band launch, K unsplit
-        const int rc = run_band(dtype, g, x, Mats{fq::MM_PAIR, {w_gate, w_up}, {N}}, nullptr, 0, 0, y,
-                                M, K, N, dev, di, st, nullptr, 0, false);
-        if (rc != FQ_ERR_WORKSPACE) return rc;
+    if (M > 1 && M <= 32) {  // gate and up rows in one launch
+        const Mats ms{fq::MM_PAIR, {w_gate, w_up}, {N}};
+        int rc = kNotTaken;
+        if (!thin_takes_pair(dtype, M, (int64_t)N * (K / g.be) * g.bb) && M >= 5 && K < 32 * 256 &&
+            band_rule(dtype, g, M, K, N, w_gate, di.cus).takes &&
+            band_rule(dtype, g, M, K, N, w_up, di.cus).takes) {  // K unsplit
+            rc = run_band(dtype, g, x, ms, nullptr, 0, 0, y, M, K, N, dev, di, st, nullptr, 0, false);
+            if (rc == FQ_ERR_WORKSPACE) rc = kNotTaken;
+        } else if (M >= 5 || thin_takes_pair(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {
+            // (5..16 tokens that the band kernel does not take: here too)
+            rc = run_thin(dtype, g, x, ms, nullptr, 0, 0, y, M, K, N, dev, di, st, nullptr, 0);
+        }
+        if (rc != kNotTaken) return rc;
     }
     uint8_t* buf = nullptr;
     StreamScratch::Lease lease(stream_scratch(dev, st, 1));
@@ -1546,9 +1566,13 @@ int fq_reserve_workspace(int M_max, int K_max, int N_max, void* stream) {
                 t.M = m;
                 t.K = Kp;
                 t.N = t.n1 = n;
-                for (uint32_t dt : {FQ_DTYPE_Q4_K, FQ_DTYPE_Q6_K})
+                for (uint32_t dt : {FQ_DTYPE_Q4_0, FQ_DTYPE_Q4_1, FQ_DTYPE_Q8_0, FQ_DTYPE_Q5_0,
+                                    FQ_DTYPE_Q5_1, FQ_DTYPE_Q4_K, FQ_DTYPE_Q5_K, FQ_DTYPE_Q6_K})
                     for (int mm : {fq::MM_ONE, fq::MM_PAIR}) {
+                        Geometry g{};
+                        geometry(dt, g);
                         t.mm = mm;
+                        t.row_bytes = (int)std::min<int64_t>((int64_t)(Kp / g.be) * g.bb, INT32_MAX);
                         need0 = std::max(need0, plan_mmqt(t, dt, di.cus).total);
                     }
             }

@@ -152,11 +152,11 @@ int64_t mmqp_q6c_bytes(int N, int K);
 hipError_t launch_q6c(const uint8_t* w, int N, int K, int64_t row_bytes, uint8_t* out,
                       hipStream_t st);
 hipError_t launch_mmqp(int dtype, const MmqArgs& a, int splits, hipStream_t st);
-// 2..32 tokens of Q4_K, Q5_K and Q6_K (fq_mmqt.hip): operands of launch_xprept
+// 2..32 tokens of every format but Q3_K (fq_mmqt.hip): operands of launch_xprept
 // (a.xop, a.xsum), work-groups of 64, 128 or 256 rows, K split into slabs of ceil(K/256 / splits) super-blocks (none empty;
 // then reduce with launch_reduce)
 bool mmqt_supported(int dtype);
-bool mmqt_has_rows(int dtype, int M, int rows);  // work-groups of so many rows exist
+int mmqt_groups(int dtype, int M, int rows);  // wave groups of such work-groups (0: none)
 int mmqt_row_tiles(const MmqArgs& a, int rows);
 size_t mmqt_xop_bytes(int M, int K);
 size_t mmqt_sum_bytes(int M, int K);

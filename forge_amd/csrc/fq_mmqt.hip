@@ -1,12 +1,13 @@
-// fq_mmqt.hip -- small batches (M <= 32 tokens) of Q4_K, Q5_K and Q6_K on the
-// fp16 matrix cores, the token operands shared by 128 or 256 rows.
+// fq_mmqt.hip -- small batches (M <= 32 tokens) of every format but Q3_K on the
+// fp16 matrix cores, the token operands shared by the rows of a work-group.
 //
 // A work-group owns a tile of 64, 128 or 256 rows and a range of super-blocks
 // (256 elements of K).  Per super-block it copies into LDS, two or three
 // buffers deep and with no registers in between,
 //
-//   the rows' super-blocks as they lie in memory (16-byte pieces along each
-//   row: contiguous runs of 144 / 176 / 210 bytes), each wave its own 16 rows,
+//   the rows' super-blocks (or eight 32-element blocks) as they lie in memory
+//   (16-byte pieces along each row: contiguous runs of 144 to 272 bytes), each
+//   wave its own 16 rows,
 //   the tokens' operands (16 KiB per 16 tokens), an equal share per wave,
 //   the tokens' sub-block sums and scales,
 //
@@ -34,7 +35,9 @@
 //   rounding and W_lo the exact rest; x W = x_hi W_hi + x_lo W_hi + x_hi W_lo
 //   (the dropped x_lo W_lo is 2^-23 of the product).
 //
-// One MFMA chain per super-block, then acc += 2^e (d D - dmin Dm), e the
+//   the 32-element blocks: the integer code, d on the results (TQB below).
+//
+// Short MFMA chains, added up per super-block, then acc += 2^e (d D - dmin Dm), e the
 // token's exponent for this super-block (x 2^-e below 2^15, split into fp16
 // hi + lo: 22 significant bits).
 #include <hip/hip_runtime.h>
@@ -62,11 +65,11 @@ constexpr int SG = 144, SSB = 8 * SG;
 // ------------------------------------------------------------- token prep
 // One work-group per super-block and 16-token tile; thread 16 c + p holds
 // elements 16 p .. 16 p + 15 of token c.  Eight elements 8 e8 .. + 7 are slots
-// (slot_elem order) of lane group q in MFMA ks: Q4_K / Q5_K q = e8 / 8, ks =
-// e8 % 8; Q6_K (U6) element 128 n + 32 u + 16 h + 8 i: q = 2 n + h, ks = 2 u +
-// i.  The sums operand of lane (c, q) holds token c's sums (times 2^-5) over
+// (slot_elem order) of lane group q in MFMA ks: Q4_K / Q5_K (MAP 0) q = e8 /
+// 8, ks = e8 % 8; Q6_K (MAP 1) element 128 n + 32 u + 16 h + 8 i: q = 2 n + h,
+// ks = 2 u + i; 32-element blocks (MAP 2) ks the block, q = e8 % 4.  The sums operand of lane (c, q) holds token c's sums (times 2^-5) over
 // sub-blocks 2 q, 2 q + 1 in three fp16 parts: hi, hi, mid, mid, lo, lo, 0, 0.
-template <bool U6>
+template <int MAP>
 __global__ __launch_bounds__(256) void xprept_kernel(const float* __restrict__ x, int M, int K,
                                                      uint8_t* __restrict__ xop,
                                                      uint8_t* __restrict__ xs) {
@@ -95,8 +98,8 @@ __global__ __launch_bounds__(256) void xprept_kernel(const float* __restrict__ x
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int e8 = 2 * p + i;
-        const int q = U6 ? 2 * (e8 >> 4) + ((e8 >> 1) & 1) : e8 >> 3;
-        const int ks = U6 ? 2 * ((e8 >> 2) & 3) + (e8 & 1) : e8 & 7;
+        const int q = MAP == 2 ? e8 & 3 : MAP == 1 ? 2 * (e8 >> 4) + ((e8 >> 1) & 1) : e8 >> 3;
+        const int ks = MAP == 2 ? e8 >> 2 : MAP == 1 ? 2 * ((e8 >> 2) & 3) + (e8 & 1) : e8 & 7;
         float w[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) w[j] = __builtin_amdgcn_ldexpf(v[8 * i + j], -e);
@@ -115,7 +118,7 @@ __global__ __launch_bounds__(256) void xprept_kernel(const float* __restrict__ x
     uint8_t* const sbk = xs + ((size_t)T * nsb + sb) * SSB;
     if (p == 0) *reinterpret_cast<float*>(sbk + (c >> 2) * SG + 128 + 4 * (c & 3)) =
         __builtin_amdgcn_ldexpf(1.0f, e);
-    if constexpr (!U6) {
+    if constexpr (MAP != 1) {
         sum += __shfl_xor(sum, 1, 64);
         if ((p & 1) == 0) {
             const int b = p >> 1, l = 16 * (b >> 1) + c;
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(256) void xprept_kernel(const float* __restrict__ x
 }
 
 // ------------------------------------------------------------- weights
-// PPR: 16-byte pieces of a row's super-block in LDS; SHIFT: rows start at even
+// BLOCKS: a scale per 32-element block, outside the operand (below).  PPR: 16-byte pieces of a row's super-block in LDS; SHIFT: rows start at even
 // addresses only, each super-block copied from its aligned-down start and read
 // at its shift (Q6_K: 14 pieces always hold some of its 210 bytes; a 15th,
 // a repeat, keeps 16 rows' 16-byte units on distinct banks).
@@ -152,7 +155,7 @@ __device__ __forceinline__ uint32_t lds4(const uint8_t* p) {
 template <int F>
 struct TQK {
     static constexpr int SBB = F == Q5_K ? 176 : 144, PPR = SBB / 16, LAST = PPR - 1;
-    static constexpr bool SHIFT = false, MIN = true, SPLITW = false;
+    static constexpr bool SHIFT = false, MIN = true, SPLITW = false, BLOCKS = false;
     static constexpr float UNIT = F == Q5_K ? 8.0f : 16.0f, MID = F == Q5_K ? 16.0f : 8.0f;
     uint32_t w[8], h[8];
     h2 s[2], off[2];
@@ -226,7 +229,7 @@ struct TQ<Q5_K> : TQK<Q5_K> {};
 template <>
 struct TQ<Q6_K> {
     static constexpr int SBB = 210, PPR = 15, LAST = 13;
-    static constexpr bool SHIFT = true, MIN = false, SPLITW = true;
+    static constexpr bool SHIFT = true, MIN = false, SPLITW = true, BLOCKS = false;
     uint32_t lo[4], hi[4], qh[4];
     h2 s[4];
     float d;
@@ -276,6 +279,96 @@ struct TQ<Q6_K> {
         wlo = h8{vl[0][0], vl[0][1], vl[1][0], vl[1][1], vl[2][0], vl[2][1], vl[3][0], vl[3][1]};
     }
 };
+
+// The 32-element block formats (eight blocks are 144 / 160 / 272 / 176 / 192 /
+// 144 bytes of a row: Q4_0, Q4_1, Q8_0, Q5_0, Q5_1, IQ4_NL).  MFMA ks is block
+// ks of the super-block, lane group q its elements 8 q .. 8 q + 7: q < 2 the low
+// nibbles of qs bytes 8 q .., else the high ones of 8 (q - 2) ..; bits 8 q .. of
+// qh.  The operand holds the integer code (IQ4_NL: the table value), the
+// block's scale d multiplies the MFMA pair's results (d codes have up to 19
+// bits).  Q4_1 and Q5_1, w = d q + m, enter as d (q - c) + (m + c d), c 8 or 16,
+// with m and d (fp16 both) on the sub-block sums.  Rows of 160 and 192
+// bytes take a repeated piece, so that 16 rows start on eight banks, not four
+// or two.
+template <int F>
+struct TQB {
+    static constexpr int BB = Fmt<F>::BB, SBB = 8 * BB;
+    static constexpr int LAST = SBB / 16 - 1, PPR = SBB / 16 + (F == Q4_1 || F == Q5_1 ? 1 : 0);
+    static constexpr bool SHIFT = false, MIN = F == Q4_1 || F == Q5_1, SPLITW = false, BLOCKS = true;
+    static constexpr int QS = F == Q4_0 || F == IQ4_NL || F == Q8_0 ? 2 : F == Q4_1 ? 4 : F == Q5_0 ? 6 : 8;
+    static constexpr int QH = F == Q5_0 ? 2 : 4;
+    static constexpr float MID = F == Q5_0 || F == Q5_1 ? 16.0f : 8.0f;  // subtracted from a code
+    uint32_t w[16], h[8];
+    float db[8];
+    h8 mb, cb;
+    int sh;
+    // the dword at p + o, o even and known at compile time
+    template <int O>
+    __device__ static uint32_t dw(const uint8_t* p) {
+        if constexpr (O % 4 == 0) return lds4(p + O);
+        else return __builtin_amdgcn_alignbyte(lds4(p + O + 2), lds4(p + O - 2), 2);
+    }
+    template <int B>
+    __device__ void block(const uint8_t* p, const uint8_t* pq, int q) {
+        constexpr int O = BB * B;
+        if constexpr ((O + QS) % 4 == 0) {
+            w[2 * B] = lds4(pq + O + QS);
+            w[2 * B + 1] = lds4(pq + O + QS + 4);
+        } else {
+            const uint32_t a = lds4(pq + O + QS - 2), b = lds4(pq + O + QS + 2), c = lds4(pq + O + QS + 6);
+            w[2 * B] = __builtin_amdgcn_alignbyte(b, a, 2);
+            w[2 * B + 1] = __builtin_amdgcn_alignbyte(c, b, 2);
+        }
+        if constexpr (F == Q5_0 || F == Q5_1) h[B] = dw<O + QH>(p) >> (8 * q);
+        db[B] = f16_hw(*reinterpret_cast<const uint16_t*>(p + O));
+    }
+    __device__ void load(const uint8_t* p, int, int q) {
+        const uint8_t* pq = p + (F == Q8_0 ? 8 * q : 8 * (q & 1));
+        sh = 4 * (q >> 1);
+        block<0>(p, pq, q);
+        block<1>(p, pq, q);
+        block<2>(p, pq, q);
+        block<3>(p, pq, q);
+        block<4>(p, pq, q);
+        block<5>(p, pq, q);
+        block<6>(p, pq, q);
+        block<7>(p, pq, q);
+        if constexpr (MIN) {  // m and d of this lane group's sub-blocks 2 q, 2 q + 1
+            const uint32_t d0 = lds4(p + 2 * BB * q), d1 = lds4(p + 2 * BB * q + BB);
+            const h2 u = __builtin_bit_cast(h2, d0), v = __builtin_bit_cast(h2, d1);
+            const _Float16 z = (_Float16)0.0f;
+            mb = h8{u[1], v[1], u[1], v[1], u[1], v[1], z, z};
+            cb = h8{u[0], v[0], u[0], v[0], u[0], v[0], z, z};
+        }
+    }
+    template <int KSI>
+    __device__ h8 op() const {
+        if constexpr (F == Q8_0) {
+            return byte8(w[2 * KSI] ^ 0x80808080u, w[2 * KSI + 1] ^ 0x80808080u, (_Float16)1152.0f);
+        } else {
+            uint32_t a = (w[2 * KSI] >> sh) & 0x0F0F0F0Fu, b = (w[2 * KSI + 1] >> sh) & 0x0F0F0F0Fu;
+            if constexpr (F == IQ4_NL)
+                return byte8(iq4_lookup(a) ^ 0x80808080u, iq4_lookup(b) ^ 0x80808080u, (_Float16)1152.0f);
+            if constexpr (F == Q5_0 || F == Q5_1) {
+                a = five_bit(a, h[KSI]);
+                b = five_bit(b, h[KSI] >> 4);
+            }
+            return byte8(a, b, (_Float16)(1024.0f + MID));
+        }
+    }
+};
+template <>
+struct TQ<Q4_0> : TQB<Q4_0> {};
+template <>
+struct TQ<Q4_1> : TQB<Q4_1> {};
+template <>
+struct TQ<Q8_0> : TQB<Q8_0> {};
+template <>
+struct TQ<Q5_0> : TQB<Q5_0> {};
+template <>
+struct TQ<Q5_1> : TQB<Q5_1> {};
+template <>
+struct TQ<IQ4_NL> : TQB<IQ4_NL> {};
 
 // TT 16-token tiles; RW waves along the rows, 16 each (PAIR: the first half
 // gate, the second half up rows), in KG groups: group k takes super-blocks
@@ -389,12 +482,22 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int sb_pe
         auto ks = [&](auto ki) {
             constexpr int KSI = decltype(ki)::value;
             h8 whi, wlo;
-            w.template ops<KSI>(whi, wlo);
+            if constexpr (Q::BLOCKS) whi = w.template op<KSI>();
+            else w.template ops<KSI>(whi, wlo);
 #pragma unroll
             for (int T = 0; T < TT; ++T) {
                 const uint8_t* xp = xs + T * XSB + KSI * 2048 + 16 * lane;
                 const h8 xh = *reinterpret_cast<const h8*>(xp);
                 const h8 xl = *reinterpret_cast<const h8*>(xp + 1024);
+                if constexpr (Q::BLOCKS) {  // Dl: the sum of d D over the blocks so far
+                    // (x_lo first: 1.8e-7 against 1.2e-7 at K = 18944)
+                    f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, whi, z, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, whi, d, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        Dl[T][i] = KSI ? __builtin_fmaf(w.db[KSI], d[i], Dl[T][i]) : w.db[0] * d[i];
+                    continue;
+                }
                 f32x4& d = D[KSI >> 1][T];
                 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, whi, KSI & 1 ? d : z, 0, 0, 0);
                 Dl[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, whi, KSI ? Dl[T] : z, 0, 0, 0);
@@ -423,9 +526,14 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int sb_pe
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float v = ((D[0][T][i] + D[1][T][i]) + (D[2][T][i] + D[3][T][i])) + Dl[T][i];
-                if constexpr (Q::MIN) v = w.d * (v + Dc[i]) + w.dn * Dm[i];
-                else v *= w.d;
+                float v = Dl[T][i];
+                if constexpr (Q::BLOCKS) {
+                    if constexpr (Q::MIN) v += 32.0f * __builtin_fmaf(Q::MID, Dc[i], Dm[i]);
+                } else {
+                    v += (D[0][T][i] + D[1][T][i]) + (D[2][T][i] + D[3][T][i]);
+                    if constexpr (Q::MIN) v = w.d * (v + Dc[i]) + w.dn * Dm[i];
+                    else v *= w.d;
+                }
                 acc[T][i] = __builtin_fmaf(v, fv[i], acc[T][i]);
             }
         }
@@ -492,26 +600,49 @@ hipError_t go(const MmqArgs& a, int splits, hipStream_t st) {
         hipLaunchKernelGGL((mmqt_kernel<F, false, TT, RW, KG>), grid, wg, 0, st, a, sps);
     return hipGetLastError();
 }
-// Work-groups of 256, 128 or 64 rows; what does not fit LDS: Q6_K at 17..32
-// tokens in 256 rows, two groups of Q6_K in 128, 64 rows at 17..32 tokens.
+// Work-groups of 256, 128 or 64 rows, each in wave groups of as many waves as
+// fit: has<F, TT>(rows) is the group count, 0 where two buffers do not fit LDS.
+template <int F, int TT, int RW, int KG>
+constexpr bool fits() {
+    return 2 * KG * (16 * RW * TQ<F>::PPR * 16 + TT * (XSB + SSB)) <= 160 * 1024;
+}
+template <int F, int TT>
+constexpr int groups(int rows) {
+    return rows == 256   ? (fits<F, TT, 16, 1>() ? 1 : 0)
+           : rows == 128 ? (fits<F, TT, 8, 2>() ? 2 : fits<F, TT, 8, 1>() ? 1 : 0)
+           : rows == 64  ? (fits<F, TT, 4, 2>() ? 2 : 0)
+                         : 0;
+}
 template <int F, int TT>
 hipError_t go_f(const MmqArgs& a, int rows, int splits, hipStream_t st) {
-    if constexpr (TT == 1 || F != Q6_K) {
+    if constexpr (groups<F, TT>(256) != 0) {
         if (rows == 256) return go<F, TT, 16, 1>(a, splits, st);
     }
-    if (rows == 128) return go<F, TT, 8, TT == 1 && F != Q6_K ? 2 : 1>(a, splits, st);
-    if constexpr (TT == 1) {
+    if constexpr (groups<F, TT>(128) != 0) {
+        if (rows == 128) return go<F, TT, 8, groups<F, TT>(128)>(a, splits, st);
+    }
+    if constexpr (groups<F, TT>(64) != 0) {
         if (rows == 64) return go<F, TT, 4, 2>(a, splits, st);
     }
     return hipErrorInvalidValue;
 }
+template <class R, class Fn>
+R with_thin(int dtype, R dflt, Fn&& fn) {
+    if (dtype == Q3_K) return dflt;
+    return with_format(dtype, dflt, [&](auto f) -> R {
+        if constexpr (decltype(f)::value == Q3_K) return dflt;
+        else return fn(f);
+    });
+}
 
 }  // namespace
 
-bool mmqt_supported(int dtype) { return dtype == Q4_K || dtype == Q5_K || dtype == Q6_K; }
-bool mmqt_has_rows(int dtype, int M, int rows) {
-    if (rows == 128) return true;
-    return M <= 16 ? rows == 256 || rows == 64 : rows == 256 && dtype != Q6_K;
+bool mmqt_supported(int dtype) { return with_thin(dtype, false, [](auto) { return true; }); }
+int mmqt_groups(int dtype, int M, int rows) {
+    return with_thin(dtype, 0, [&](auto f) {
+        constexpr int F = decltype(f)::value;
+        return M <= 16 ? groups<F, 1>(rows) : groups<F, 2>(rows);
+    });
 }
 int mmqt_row_tiles(const MmqArgs& a, int rows) { return row_tiles(a, rows); }
 size_t mmqt_xop_bytes(int M, int K) { return (size_t)((M + 15) / 16) * (K / 256) * XSB; }
@@ -520,23 +651,21 @@ size_t mmqt_sum_bytes(int M, int K) { return (size_t)((M + 15) / 16) * (K / 256)
 hipError_t launch_xprept(int dtype, const float* x, int M, int K, uint8_t* xop, uint8_t* xs,
                          hipStream_t st) {
     const dim3 grid(K / 256, (M + 15) / 16);
-    if (dtype == Q6_K) hipLaunchKernelGGL(xprept_kernel<true>, grid, dim3(256), 0, st, x, M, K, xop, xs);
-    else hipLaunchKernelGGL(xprept_kernel<false>, grid, dim3(256), 0, st, x, M, K, xop, xs);
+    if (dtype == Q6_K)
+        hipLaunchKernelGGL(xprept_kernel<1>, grid, dim3(256), 0, st, x, M, K, xop, xs);
+    else if (dtype == Q4_K || dtype == Q5_K)
+        hipLaunchKernelGGL(xprept_kernel<0>, grid, dim3(256), 0, st, x, M, K, xop, xs);
+    else
+        hipLaunchKernelGGL(xprept_kernel<2>, grid, dim3(256), 0, st, x, M, K, xop, xs);
     return hipGetLastError();
 }
 
 hipError_t launch_mmqt(int dtype, const MmqArgs& a, int rows, int splits, hipStream_t st) {
     if (a.M > 32 || a.K % 256 != 0 || splits < 1) return hipErrorInvalidValue;
-    auto tt = [&](auto f) {
+    return with_thin(dtype, hipErrorInvalidValue, [&](auto f) {
         constexpr int F = decltype(f)::value;
         return a.M <= 16 ? go_f<F, 1>(a, rows, splits, st) : go_f<F, 2>(a, rows, splits, st);
-    };
-    switch (dtype) {
-        case Q4_K: return tt(FmtTag<Q4_K>{});
-        case Q5_K: return tt(FmtTag<Q5_K>{});
-        case Q6_K: return tt(FmtTag<Q6_K>{});
-    }
-    return hipErrorInvalidValue;
+    });
 }
 
 }  // namespace fq

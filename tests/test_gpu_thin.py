@@ -1,5 +1,5 @@
-"""Small batches of Q4_K, Q5_K and Q6_K with the token operands shared by a
-work-group (24 MB and more, or 17..32 tokens): partial row tiles, one
+"""Small batches with the token operands shared by a work-group (24 to 48 MiB
+and more, or 17..32 tokens; gate/up pairs of 2..4 tokens): partial row tiles, one
 super-block, odd counts of them over two wave groups and K-splits, both token
 tiles partly filled, offset bases, gate/up pairs and concatenated results."""
 from __future__ import annotations
@@ -16,13 +16,14 @@ from test_gpu_parity import dev_weight
 
 pytestmark = pytest.mark.gpu
 KQ = [F.Q4_K, F.Q5_K, F.Q6_K]
+ALL = KQ + [F.Q4_0, F.Q4_1, F.Q8_0, F.Q5_0, F.Q5_1, F.IQ4_NL]
 
 
 def wmax(dtype, ws, K):
     return max(float(np.max(np.abs(oracle.dequant(dtype, w[:2048], min(len(w), 2048), K)))) for w in ws)
 
 
-@pytest.mark.parametrize("dtype", KQ)
+@pytest.mark.parametrize("dtype", ALL)
 @pytest.mark.parametrize("M,N,K", [(17, 1, 256), (32, 127, 512), (18, 300, 768), (31, 129, 2816),
                                    (24, 4100, 1024), (32, 33, 18944),
                                    (4, 24001, 2048), (5, 9000, 5888), (16, 3584, 18944),
@@ -50,9 +51,10 @@ def test_shapes(dtype, M, N, K):
         assert torch.equal(ops.matmul_transB(xd, dev_weight(dtype, w, N, K, 2)), y)
 
 
-@pytest.mark.parametrize("dtype", KQ)
+@pytest.mark.parametrize("dtype", ALL)
 @pytest.mark.parametrize("M,N,K", [(17, 1, 256), (32, 65, 768), (20, 300, 2048), (2, 11008, 4096),
-                                   (8, 14336, 4096), (16, 18945, 3584), (3, 4096, 14336)])
+                                   (8, 14336, 4096), (16, 18945, 3584), (3, 4096, 14336),
+                                   (4, 33, 512), (2, 500, 1024)])
 def test_gate_up_pair(dtype, M, N, K):
     wg, wu = (synth.make_weights(dtype, N, K, s) for s in (50, 51))
     x = synth.make_x(M, K, seed=M) * np.float32(1e-2)
@@ -62,7 +64,7 @@ def test_gate_up_pair(dtype, M, N, K):
     assert_close_silu_mul(y.cpu().numpy(), g, u, x, wmax(dtype, [wg, wu], K), f"{dtype} {M}x{N}x{K}")
 
 
-@pytest.mark.parametrize("dtype", KQ)
+@pytest.mark.parametrize("dtype", ALL)
 @pytest.mark.parametrize("M,K,ns", [(17, 256, (257, 64, 1)), (32, 2048, (1, 300, 255)),
                                     (20, 512, (0, 96, 33)), (25, 1280, (31, 0, 256))])
 def test_qkv(dtype, M, K, ns):
