@@ -163,7 +163,7 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
     }
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds);
-    auto issue = [&](int s, bool first) {  // first: s is its super-block's first step
+    auto issue = [&](int s, bool first) __attribute__((always_inline)) {  // first: s is its super-block's first step
         const int buf = s % NBUF, sb = s >> 2;
         const uint32_t xl = lds_base + buf * Q::XBUF + wave * 4096;
         const uint8_t* xg = xbase + (size_t)s * 4 * XT * 2;
@@ -202,10 +202,12 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
             r[2 * h + 1] = *reinterpret_cast<const h8*>(xp + 512);
         }
     };
-    // one step, sub-block pair U of its super-block
-    auto step = [&](auto u, const _Float16* xs, const uint8_t* qs, const uint8_t* hs,
+    // one step, sub-block pair U of its super-block; NI: the wave's token tiles
+    // that hold tokens
+    auto step = [&](auto u, auto ni, const _Float16* xs, const uint8_t* qs, const uint8_t* hs,
                     const uint8_t* ss) {
-        constexpr int U = decltype(u)::value;
+        constexpr int U = decltype(u)::value, NI = decltype(ni)::value;
+        if constexpr (NI == 0) return;
         h8 A[2][4];
         read_a(xs, 0, 0, A[0]);
         const int rl = PAIR ? 32 * wn + c : 64 * wn + c;
@@ -239,10 +241,10 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
                 B[j][1] = scaled8(w[2], w[3], sc, off);
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int st = 2 * b + i;
+            for (int i = 0; i < NI; ++i) {
+                const int st = NI * b + i;
                 h8(&cur)[4] = A[st & 1];
-                if (st < 3) read_a(xs, (st + 1) >> 1, (st + 1) & 1, A[(st + 1) & 1]);
+                if (st + 1 < 2 * NI) read_a(xs, (st + 1) / NI, (st + 1) % NI, A[(st + 1) & 1]);
                 const f32x16 z = {};
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
@@ -278,7 +280,7 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
                 dn[j] = -32.0f * f16_hw(hdr[j].x >> 16);
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < NI; ++i) {
                 const h8 S = *reinterpret_cast<const h8*>(ss + (2 * wm + i) * STILE + 16 * lane);
                 const f32x16 z = {};
                 f32x16 dm[2];
@@ -306,7 +308,7 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
         issue(s0, true);
         issue(s0 + 1, false);
     }
-    auto run = [&](auto u, int s) {
+    auto run = [&](auto u, auto ni, int s) __attribute__((always_inline)) {
         constexpr int U = decltype(u)::value;
         // this wave's copies of step s are complete; those of step s + 1 may
         // be in flight
@@ -315,15 +317,25 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
         __syncthreads();
         if (s + 2 < s1) issue(s + 2, U == 2);
         const int buf = s % NBUF, sb = (s >> 2) & 1;
-        step(u, reinterpret_cast<const _Float16*>(xs0 + buf * Q::XBUF), qs0 + buf * Q::QBUF,
+        step(u, ni, reinterpret_cast<const _Float16*>(xs0 + buf * Q::XBUF), qs0 + buf * Q::QBUF,
              hs0 + sb * Q::HBUF, ss0 + sb * Q::SBUF);
     };
-    for (int s = s0; s < s1; s += 4) {
-        run(std::integral_constant<int, 0>{}, s);
-        run(std::integral_constant<int, 1>{}, s + 1);
-        run(std::integral_constant<int, 2>{}, s + 2);
-        run(std::integral_constant<int, 3>{}, s + 3);
-    }
+    // Token tiles past M are copied and waited for, not computed: the matrix
+    // cores' pace is the kernel's, so a tile of zeros costs as much as any
+    // (Q4_K 4096 -> 14336 at M = 77, preparation included, 49 -> 43 us).  Deeper
+    // buffers in the LDS that fewer tiles would leave measured no faster.
+    auto loop = [&](auto ni) __attribute__((always_inline)) {
+        for (int s = s0; s < s1; s += 4) {
+            run(std::integral_constant<int, 0>{}, ni, s);
+            run(std::integral_constant<int, 1>{}, ni, s + 1);
+            run(std::integral_constant<int, 2>{}, ni, s + 2);
+            run(std::integral_constant<int, 3>{}, ni, s + 3);
+        }
+    };
+    const int live = Tn - (m0 / 32 + 2 * wm);  // wave-uniform
+    if (live >= 2) loop(std::integral_constant<int, 2>{});
+    else if (live == 1) loop(std::integral_constant<int, 1>{});
+    else loop(std::integral_constant<int, 0>{});
 #pragma unroll
     for (int i = 0; i < 2; ++i)
         store_tiles<PAIR>(a, rt, m0 + 64 * wm + 32 * i, rt.n0 + (PAIR ? 32 : 64) * wn + c, g, acc[i],

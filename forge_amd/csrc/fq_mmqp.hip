@@ -45,32 +45,36 @@ constexpr int NW = 8;                // waves per work-group
 // (SUB16: elements 16 kq + 8 g + slot_elem(j), so that each quarter is one
 // 16-element sub-block).
 //
-// One launch: work-group j owns tokens 4 j .. 4 j + 3 (all of K).  Piece p = ((2 kq + g) 4 + t): token t's eight elements of quarter kq,
-// lane group g -- four consecutive threads write one 64-byte run (hi, and
-// lo 1 KiB on).  Pass 1 finds each token's largest |x| (x read once from
-// HBM), pass 2 writes the operands from the values kept in registers (those
-// of K beyond 8192 are read again, from L2).  The work-groups cover every
-// token slot of the last tile (slots past M are zero).
-template <bool SUB16>
+// One launch: work-group j owns tokens TPW j .. TPW j + TPW - 1 (all of K).
+// Piece p = ((2 kq + g) TPW + t): token t's eight elements of quarter kq, lane
+// group g -- TPW consecutive threads write one run of 16 TPW bytes (hi, and lo
+// 1 KiB on).  Pass 1 finds each token's largest |x| (x read once from HBM),
+// pass 2 writes the operands from the values kept in registers (CP pieces per
+// thread; those beyond are read again).  The work-groups cover every token
+// slot of the last tile (slots past M are zero).
+//
+// Four tokens per work-group, 64-byte runs, unless that leaves most CUs idle:
+// up to 128 tokens one each (77 x 4096 and 14336, median of both: 16 -> 8 us; at 512 x 4096 one token
+// measured 9.2 us against 6.4).  Rows beyond 8192 elements keep ten pieces per
+// thread instead of four (1999 x 18944: 82 -> 61 us, the second reading of x
+// gone).
+template <bool SUB16, int TPW, int CP>
 __global__ __launch_bounds__(1024) void xprep4_kernel(const float* __restrict__ x, int M, int K,
                                                       int* __restrict__ ex,
                                                       _Float16* __restrict__ xop,
                                                       float* __restrict__ xsum,
                                                       _Float16* __restrict__ xsum2) {
-    __shared__ float wmax[16][4];
-    __shared__ int es[4];
-    const int tid = threadIdx.x, t = tid & 3;
-    const int m = 4 * blockIdx.x + t;
+    __shared__ float wmax[16][TPW];
+    __shared__ int es[TPW];
+    const int tid = threadIdx.x, t = tid % TPW;
+    const int m = TPW * blockIdx.x + t;
     const bool live = m < M;
     const float* xr = x + (size_t)min(m, M - 1) * K;
-    const int KQ = K / 16, P = 8 * KQ;  // pieces per work-group
+    const int KQ = K / 16, P = 2 * TPW * KQ;  // pieces per work-group
     auto src = [&](int p) {
-        const int gq = p >> 2, g = gq & 1, kq = gq >> 1;
+        const int gq = p / TPW, g = gq & 1, kq = gq >> 1;
         return SUB16 ? xr + 16 * kq + 8 * g : xr + 32 * (kq >> 1) + 16 * g + 8 * (kq & 1);
     };
-    // the first CP pieces of a thread stay in registers for the second pass
-    // (all of them up to K = 8192); the rest are read again, from L2
-    constexpr int CP = 4;
     float4 ca[CP], cb[CP];
     float mx = 0.0f;
     auto amax = [](float4 a, float4 b) {
@@ -94,21 +98,21 @@ __global__ __launch_bounds__(1024) void xprep4_kernel(const float* __restrict__ 
                             *reinterpret_cast<const float4*>(s + 4)));
     }
 #pragma unroll
-    for (int o = 4; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    if ((tid & 63) < 4) wmax[tid >> 6][t] = mx;
+    for (int o = TPW; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    if ((tid & 63) < TPW) wmax[tid >> 6][t] = mx;
     __syncthreads();
-    if (tid < 4) {
+    if (tid < TPW) {
         float v = 0.0f;
         for (int w = 0; w < 16; ++w) v = fmaxf(v, wmax[w][tid]);
         const int e = (v > 0.0f && v <= 3.0e38f) ? ilogbf(v) - 14 : 0;
         es[tid] = e;
-        if (4 * blockIdx.x + tid < M) ex[4 * blockIdx.x + tid] = e;
+        if (TPW * (int)blockIdx.x + tid < M) ex[TPW * blockIdx.x + tid] = e;
     }
     __syncthreads();
     const int e = es[t];
     const int T = m >> 5, lm = m & 31;
     auto piece = [&](int p, float4 a, float4 b) {
-        const int gq = p >> 2, g = gq & 1, kq = gq >> 1;
+        const int gq = p / TPW, g = gq & 1, kq = gq >> 1;
         h8 hi = {}, lo = {};
         float w[8] = {};
         if (live) {
@@ -127,26 +131,27 @@ __global__ __launch_bounds__(1024) void xprep4_kernel(const float* __restrict__ 
         *reinterpret_cast<h8*>(dst + 512) = lo;
         if (xsum || xsum2) {
             // the token's sum of x 2^-e over its 32-element sub-block kq / 2:
-            // pieces p, p ^ 4, p ^ 8, p ^ 12 of one wave, added in a fixed tree
+            // four pieces TPW apart of one wave, added in a fixed tree
             float t8 = ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
-            t8 += __shfl_xor(t8, 4, 64);
-            t8 += __shfl_xor(t8, 8, 64);
-            if ((p & 12) == 0) {
+            t8 += __shfl_xor(t8, TPW, 64);
+            t8 += __shfl_xor(t8, 2 * TPW, 64);
+            if ((gq & 3) == 0) {
                 const int b = kq >> 1;  // sub-block
                 if (xsum) xsum[((size_t)T * (K / 32) + b) * 32 + lm] = t8;
                 if (xsum2) {
                     // times 2^-5 (below 2^15) as fp16 hi + lo:
                     // [super-block][hi, lo][token][sub-block of the super-block]
                     const float v = t8 * 0x1p-5f;
-                    const _Float16 hi = (_Float16)v;
+                    const _Float16 vh = (_Float16)v;
                     _Float16* d = xsum2 + ((size_t)T * (K / 256) + (b >> 3)) * 512 + lm * 8 + (b & 7);
-                    d[0] = hi;
-                    d[256] = (_Float16)(v - (float)hi);
+                    d[0] = vh;
+                    d[256] = (_Float16)(v - (float)vh);
                 }
             }
         }
     };
-    // P is a multiple of 64: whole waves take part in each piece's shuffles
+    // P is a multiple of 4 TPW (K of 256: of 32 TPW), so the lanes of a shuffle
+    // take part in it together
 #pragma unroll
     for (int it = 0; it < CP; ++it) {
         const int p = tid + 1024 * it;
@@ -439,7 +444,7 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
     const uint32_t wend = (uint32_t)rt.rows * (uint32_t)a.row_bytes - 16;
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds);
-    auto issue = [&](int s) {
+    auto issue = [&](int s) __attribute__((always_inline)) {
         const int buf = s % NBUF;
         const uint32_t xl = lds_base + buf * TL::XBUF + wave * 4096;
         const uint8_t* xg = xbase + (size_t)s * 4 * XT * 2;
@@ -491,8 +496,10 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
     f32x16 dp[2];   // chain results of the previous stage (token tile 1 at a step's end)
     float dbp[2];
     bool pend = false;
-    auto step = [&](auto o4, const _Float16* xs, const uint8_t* ws) {
-        constexpr int O4 = decltype(o4)::value;
+    // NI: the wave's token tiles that hold tokens
+    auto step = [&](auto o4, auto ni, const _Float16* xs, const uint8_t* ws) __attribute__((always_inline)) {
+        constexpr int O4 = decltype(o4)::value, NI = decltype(ni)::value;
+        if constexpr (NI == 0) return;
         float mn[2][2];  // dmin m of row tile j, block b (0 without a min term)
         h8 A[2][4];
         read_a(xs, 0, 0, A[0]);
@@ -521,10 +528,11 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
                 }
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int st = 2 * b + i;  // stage within the step
+            for (int i = 0; i < NI; ++i) {
+                const int st = NI * b + i;  // stage within the step
+                const int ip = NI == 2 ? 1 - i : 0;  // the previous stage's token tile
                 h8(&cur)[4] = A[st & 1];
-                if (st < 3) read_a(xs, (st + 1) >> 1, (st + 1) & 1, A[(st + 1) & 1]);
+                if (st + 1 < 2 * NI) read_a(xs, (st + 1) / NI, (st + 1) % NI, A[(st + 1) & 1]);
                 if constexpr (F == Q6_K) {
                     // one chain over both 16-element sub-blocks: the first
                     // sub-block's partial sums are scaled by r = sc0 / sc1
@@ -546,7 +554,7 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
                         for (int j = 0; j < 2; ++j)
 #pragma unroll
                             for (int e = 0; e < 16; ++e)
-                                acc[1 - i][j][e] = __builtin_fmaf(dbp[j], dp[j][e], acc[1 - i][j][e]);
+                                acc[ip][j][e] = __builtin_fmaf(dbp[j], dp[j][e], acc[ip][j][e]);
                     }
 #pragma unroll
                     for (int j = 0; j < 2; ++j)
@@ -578,13 +586,13 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
 #pragma unroll
                     for (int j = 0; j < 2; ++j)
                         d[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur[3], B[j][1], d[j], 0, 0, 0);
-                    // fold the previous stage (token tile 1 - i)
+                    // fold the previous stage (token tile ip)
                     if (pend) {
 #pragma unroll
                         for (int j = 0; j < 2; ++j)
 #pragma unroll
                             for (int e = 0; e < 16; ++e)
-                                acc[1 - i][j][e] = __builtin_fmaf(dbp[j], dp[j][e], acc[1 - i][j][e]);
+                                acc[ip][j][e] = __builtin_fmaf(dbp[j], dp[j][e], acc[ip][j][e]);
                     }
                     dp[0] = d[0];
                     dp[1] = d[1];
@@ -602,7 +610,7 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
             const float* sv = reinterpret_cast<const float*>(
                 reinterpret_cast<const uint8_t*>(xs) + TL::XOPB);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < NI; ++i) {
                 const float sa = sv[((2 * wm + i) * 2 + g) * 32 + c];
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
@@ -616,28 +624,40 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
     // one step: this wave's copies of step s are done; the barrier makes
     // every wave's visible and ends every wave's reads of step s - 1, whose
     // buffers step s + 2 then refills
-    auto run = [&](auto o4, int s) {
+    auto run = [&](auto o4, auto ni, int s) __attribute__((always_inline)) {
         wait_step(s + 1 < s1);
         __syncthreads();
         if (s + 2 < s1) issue(s + 2);
         const int buf = s % NBUF;
-        step(o4, reinterpret_cast<const _Float16*>(xs0 + buf * TL::XBUF), ws0 + buf * TL::WBUF);
+        step(o4, ni, reinterpret_cast<const _Float16*>(xs0 + buf * TL::XBUF), ws0 + buf * TL::WBUF);
     };
     // a row's step s starts 4 (s mod 4) bytes into its LDS slot (68 and 36
     // are 4 mod 16; s0 is a multiple of 4), so four steps per iteration
     // give every read a constant offset
-    for (int s = s0; s < s1; s += 4) {
-        run(std::integral_constant<int, Chunks<F>::o4(0)>{}, s);
-        if (s + 1 < s1) run(std::integral_constant<int, Chunks<F>::o4(1)>{}, s + 1);
-        if (s + 2 < s1) run(std::integral_constant<int, Chunks<F>::o4(2)>{}, s + 2);
-        if (s + 3 < s1) run(std::integral_constant<int, Chunks<F>::o4(3)>{}, s + 3);
-    }
-    if (pend) {
+    auto loop = [&](auto ni) __attribute__((always_inline)) {
+        constexpr int NI = decltype(ni)::value;
+        for (int s = s0; s < s1; s += 4) {
+            run(std::integral_constant<int, Chunks<F>::o4(0)>{}, ni, s);
+            if (s + 1 < s1) run(std::integral_constant<int, Chunks<F>::o4(1)>{}, ni, s + 1);
+            if (s + 2 < s1) run(std::integral_constant<int, Chunks<F>::o4(2)>{}, ni, s + 2);
+            if (s + 3 < s1) run(std::integral_constant<int, Chunks<F>::o4(3)>{}, ni, s + 3);
+        }
+        if constexpr (NI > 0) {
+            if (pend) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[1][j][e] = __builtin_fmaf(dbp[j], dp[j][e], acc[1][j][e]);
-    }
+                    for (int e = 0; e < 16; ++e)
+                        acc[NI - 1][j][e] = __builtin_fmaf(dbp[j], dp[j][e], acc[NI - 1][j][e]);
+            }
+        }
+    };
+    // token tiles past M are copied and waited for, not computed (Q8_0 14336 ->
+    // 4096 at M = 77 53 -> 50 us)
+    const int live = __builtin_amdgcn_readfirstlane(Tn - (m0 / 32 + 2 * wm));
+    if (live >= 2) loop(std::integral_constant<int, 2>{});
+    else if (live == 1) loop(std::integral_constant<int, 1>{});
+    else loop(std::integral_constant<int, 0>{});
 #pragma unroll
     for (int i = 0; i < 2; ++i)
         store_tiles<PAIR>(a, rt, m0 + 64 * wm + 32 * i, rt.n0 + (PAIR ? 32 : 64) * wn + c, g, acc[i],
@@ -718,12 +738,19 @@ int mmqp_row_tiles(const MmqArgs& a) { return row_tiles(a, BNT); }
 hipError_t launch_xprep32(const float* x, int M, int K, _Float16* xop, int* ex, float* xsum,
                           _Float16* xsum2, bool sub16, hipStream_t st) {
     if (K % 256 != 0) return hipErrorInvalidValue;
-    if (sub16)
-        hipLaunchKernelGGL(xprep4_kernel<true>, dim3(8 * ((M + 31) / 32)), dim3(1024), 0, st, x, M,
-                           K, ex, xop, xsum, xsum2);
-    else
-        hipLaunchKernelGGL(xprep4_kernel<false>, dim3(8 * ((M + 31) / 32)), dim3(1024), 0, st, x,
-                           M, K, ex, xop, xsum, xsum2);
+    auto go = [&](auto sub, auto tpw, auto cp) {
+        hipLaunchKernelGGL((xprep4_kernel<decltype(sub)::value, decltype(tpw)::value, decltype(cp)::value>),
+                           dim3(32 / tpw * ((M + 31) / 32)), dim3(1024), 0, st, x, M, K, ex, xop, xsum,
+                           xsum2);
+    };
+    auto shape = [&](auto sub) {
+        using std::integral_constant;
+        if (M <= 128) go(sub, integral_constant<int, 1>{}, integral_constant<int, 4>{});
+        else if (K <= 8192) go(sub, integral_constant<int, 4>{}, integral_constant<int, 4>{});
+        else go(sub, integral_constant<int, 4>{}, integral_constant<int, 10>{});
+    };
+    if (sub16) shape(std::true_type{});
+    else shape(std::false_type{});
     return hipGetLastError();
 }
 
