@@ -404,21 +404,22 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
 // Small batches with the token operands shared by the rows of a work-group
 // (fq_mmqt.hip: every format but Q3_K).
 struct MmqtPlan {
-    int rows, splits;
+    int rows, per, parts;
     size_t xop_b, sum_b, part_b, total;
 };
 
-// Rows per work-group and K-splits of the smallest estimated time: rounds of
-// work-groups x (iterations of one super-block per wave group + 1.5 us to fill
-// the pipeline), and for a split the slab sum (3.5 us and each slab written
-// and read at 4 TB/s).  An iteration's time is what 14336 x 4096 measured on
-// 224 work-groups, or its weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x
+// Rows per tile and steps per work-group of the smallest estimated time:
+// whole tiles, or the steps of all tiles shared out over the CUs (or over
+// half, a quarter .. of them, with fewer parts of a tile), at most one
+// work-group per CU: 1.5 us to fill the pipeline, the steps, 1 us per tile
+// ended, and for tiles in parts their sum (3.5 us and each slab written and
+// read at 4 TB/s).  A step's time is what 14336 x 4096 measured on 224
+// work-groups, or its weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x
 // 3584 at M = 16: 134 us on 128 rows, 156 on 64).
 MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
     const bool q6 = dtype == FQ_DTYPE_Q6_K, wide = a.M > 16;
     MmqtPlan p{};
-    const int nsb = a.K / 256;
-    const double sb_bytes = (double)a.row_bytes / nsb;
+    const double sb_bytes = (double)a.row_bytes / (a.K / 256);
     double best = 0.0;
     for (int rows : {256, 128, 64}) {
         const int kg = fq::mmqt_groups((int)dtype, a.M, rows);
@@ -426,27 +427,33 @@ MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
         const double it = rows == 256   ? (q6 ? 2.7 : wide ? 2.6 : 2.0)
                           : rows == 128 ? (q6 ? (wide ? 2.2 : 1.7) : wide ? 1.6 : 1.7)
                                         : (q6 ? 1.8 : 1.3);
-        const long tiles = fq::mmqt_row_tiles(a, rows);
-        for (int sp = 1; sp <= std::min(16, nsb); ++sp) {
-            const int sps = (nsb + sp - 1) / sp;
-            if (sps * (sp - 1) >= nsb) continue;  // an empty split
-            const double busy = (double)std::min<long>(tiles * sp, cus);
-            const double step = std::max(it, busy * kg * rows * sb_bytes / 5e6);
-            const double t = (double)((tiles * sp + cus - 1) / cus) *
-                                 (1.5 + step * ((sps + kg - 1) / kg)) +
-                             (sp > 1 ? 3.5 + (sp + 1.0) * a.M * fq::mm_cols(a) * 4.0 / 4e6 : 0.0);
-            if (p.rows == 0 || t < best) {
-                best = t;
-                p.rows = rows;
-                p.splits = sp;
+        const int tiles = fq::mmqt_row_tiles(a, rows), nst = fq::mmqt_steps(a.K, kg);
+        const int whole = nst * ((tiles + cus - 1) / cus);
+        const int64_t total = (int64_t)tiles * nst;
+        if (total >= (int64_t)1 << 31) continue;
+        for (int per = (int)((total + cus - 1) / cus);; per *= 2) {
+            per = std::min(per, whole);
+            const int parts = fq::mmqt_parts(nst, per);
+            if (parts <= 16) {
+                const double busy = (double)((total + per - 1) / per);
+                const double step = std::max(it, busy * kg * rows * sb_bytes / 5e6);
+                const double t = 1.5 + step * per + (double)((per + nst - 1) / nst) +
+                                 (parts > 1 ? 3.5 + (parts + 1.0) * a.M * fq::mm_cols(a) * 4.0 / 4e6 : 0.0);
+                if (p.rows == 0 || t < best) {
+                    best = t;
+                    p.rows = rows;
+                    p.per = per;
+                    p.parts = parts;
+                }
             }
+            if (per == whole) break;
         }
     }
     if (p.rows == 0) return p;
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     p.xop_b = fq::mmqt_xop_bytes(a.M, a.K);
     p.sum_b = fq::mmqt_sum_bytes(a.M, a.K);
-    p.part_b = p.splits > 1 ? (size_t)p.splits * a.M * fq::mm_cols(a) * 4 : 0;
+    p.part_b = p.parts > 1 ? (size_t)p.parts * a.M * fq::mm_cols(a) * 4 : 0;
     p.total = 256 + al(p.xop_b) + al(p.sum_b) + al(p.part_b);
     return p;
 }
@@ -524,15 +531,14 @@ int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, 
     a.xop = buf;
     uint8_t* const sums = buf + al(pl.xop_b);
     a.xsum = reinterpret_cast<const float*>(sums);
-    a.part = pl.splits > 1 ? reinterpret_cast<float*>(sums + al(pl.sum_b)) : nullptr;
+    a.part = pl.parts > 1 ? reinterpret_cast<float*>(sums + al(pl.sum_b)) : nullptr;
     a.y = y;
     a.bias = bias;
     a.bias_len = bias_mode ? bias_len : 0;
     a.bias_mode = bias_mode;
     hipError_t e = fq::launch_xprept((int)dtype, x, M, K, buf, sums, st);
     if (e != hipSuccess) return hip_fail(e);
-    e = fq::launch_mmqt((int)dtype, a, pl.rows, pl.splits, st);
-    if (e == hipSuccess && pl.splits > 1) e = fq::launch_reduce(a, pl.splits, st);
+    e = fq::launch_mmqt((int)dtype, a, pl.rows, pl.per, st);
     return e == hipSuccess ? FQ_OK : hip_fail(e);
 }
 

@@ -153,8 +153,10 @@ hipError_t launch_q6c(const uint8_t* w, int N, int K, int64_t row_bytes, uint8_t
                       hipStream_t st);
 hipError_t launch_mmqp(int dtype, const MmqArgs& a, int splits, hipStream_t st);
 // 2..32 tokens of every format but Q3_K (fq_mmqt.hip): operands of launch_xprept
-// (a.xop, a.xsum), work-groups of 64, 128 or 256 rows, K split into slabs of ceil(K/256 / splits) super-blocks (none empty;
-// then reduce with launch_reduce)
+// (a.xop, a.xsum), row tiles of 64, 128 or 256 rows.  A tile is mmqt_steps
+// steps; each work-group takes per steps of all tiles' in a row.  parts: some
+// tile's steps lie in several work-groups, up to mmqt_parts(steps, per), each
+// with a slab of a.part.
 bool mmqt_supported(int dtype);
 int mmqt_groups(int dtype, int M, int rows);  // wave groups of such work-groups (0: none)
 int mmqt_row_tiles(const MmqArgs& a, int rows);
@@ -162,7 +164,9 @@ size_t mmqt_xop_bytes(int M, int K);
 size_t mmqt_sum_bytes(int M, int K);
 hipError_t launch_xprept(int dtype, const float* x, int M, int K, uint8_t* xop, uint8_t* xs,
                          hipStream_t st);
-hipError_t launch_mmqt(int dtype, const MmqArgs& a, int rows, int splits, hipStream_t st);
+inline int mmqt_steps(int K, int groups) { return (K / 256 + groups - 1) / groups; }
+inline int mmqt_parts(int steps, int per) { return per % steps == 0 ? 1 : (steps + per - 2) / per + 1; }
+hipError_t launch_mmqt(int dtype, const MmqArgs& a, int rows, int per, hipStream_t st);
 hipError_t launch_reduce(const MmqArgs& a, int splits, hipStream_t st);
 hipError_t launch_dequant(int dtype, const uint8_t* w, float* out, int N, int K, int row_bytes,
                           int cus, hipStream_t st);

@@ -1,8 +1,8 @@
 // fq_mmqt.hip -- small batches (M <= 32 tokens) of every format but Q3_K on the
 // fp16 matrix cores, the token operands shared by the rows of a work-group.
 //
-// A work-group owns a tile of 64, 128 or 256 rows and a range of super-blocks
-// (256 elements of K).  Per super-block it copies into LDS, two or three
+// A work-group owns a range of steps: super-blocks (256 elements of K) of tiles
+// of 64, 128 or 256 rows.  Per super-block it copies into LDS, two or three
 // buffers deep and with no registers in between,
 //
 //   the rows' super-blocks (or eight 32-element blocks) as they lie in memory
@@ -15,12 +15,12 @@
 // fq_mmqs.hip every wave reads the token operands of its own super-blocks from
 // L2, for 32 or 64 rows: 3.5 times the weight bytes for a Q6_K head at 16
 // tokens (1.1 GB).  Here the operands of a super-block serve all rows of the
-// work-group.  152064 x 3584 Q6_K, M = 16: 216 -> 139 us; Q4_K, M = 8 131 ->
+// work-group.  152064 x 3584 Q6_K, M = 16: 216 -> 129 us; Q4_K, M = 8 131 ->
 // 98; 14336 x 4096 Q4_K, M = 8 18.7 -> 16.3, M = 32 (fp16 MFMA kernel) 40.2 ->
 // 23.2, gate and up of that size in one launch 37.7 -> 22.0 and 82.5 -> 36.0.
 // What bounds it: vector and matrix issue with the LDS reads of the token
-// operands, about equal (without the copies the head's time is 117 us, without
-// the arithmetic 105), so the waves per SIMD count: 256 rows on eight waves of
+// operands, about equal (with a work-group per tile half, 139 us in all, the head
+// took 117 without the copies, 105 without the arithmetic), so the waves per SIMD count: 256 rows on eight waves of
 // two tiles each ran the head in 152 us, on sixteen waves 139.
 //
 // Tokens are the A operand of v_mfma_f32_16x16x32_f16 (lane 16 q + c: token c,
@@ -371,8 +371,8 @@ template <>
 struct TQ<IQ4_NL> : TQB<IQ4_NL> {};
 
 // TT 16-token tiles; RW waves along the rows, 16 each (PAIR: the first half
-// gate, the second half up rows), in KG groups: group k takes super-blocks
-// b0 + k, b0 + KG + k, ...
+// gate, the second half up rows), in KG groups: step j of a row tile is group
+// k's super-block KG j + k.
 template <int F, int TT, int RW, int KG>
 struct Thin {
     using Q = TQ<F>;
@@ -385,11 +385,37 @@ struct Thin {
     static constexpr int XC = 16 / RW;                    // 1 KiB token copies per wave and tile
     static constexpr int SW = RW < 8 ? RW : 8;            // waves that copy a tile's sums
     static_assert(LDS <= 160 * 1024, "LDS");
-    static_assert(NW * TT * 1024 <= LDS, "the sums exchanged at the end");
+    static_assert(NW * TT * 1024 <= BUF, "the sums exchanged at a tile's end");
 };
 
-template <int F, bool PAIR, int TT, int RW, int KG>
-__global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int sb_per_split) {
+__device__ __forceinline__ float biased(const MmqArgs& a, float v, int m, int n) {
+    if (a.bias_mode == 1) return v + (n < a.bias_len ? a.bias[n] : 0.0f);
+    return a.bias_mode == 2 ? v + a.bias[(size_t)m * a.N + n] : v;
+}
+
+// The parts of row tile t, of nst steps, when each work-group takes per steps of
+// all tiles' in a row: the work-groups first .. first + n - 1.
+struct Parts {
+    int first, n;
+};
+__device__ __forceinline__ Parts tile_parts(int t, int nst, int per) {
+    const int f = t * nst / per;
+    return Parts{f, (t * nst + nst - 1) / per - f + 1};
+}
+
+// Work-group j takes steps per j .. of the row tiles' steps laid end to end, and
+// its copies run ahead over the tiles' ends: one work-group fills a CU's LDS, so
+// that work-groups in turn each fill and drain the pipeline alone (a step and
+// 1.5 us more), and a last round of them leaves CUs idle.  A tile within one
+// work-group goes to y, the parts of one cut by a range's end to slabs that
+// reducet_kernel adds.  Against a work-group per tile or K-split of one: Q6_K
+// 152064 x 3584 M = 16 140 -> 129 us, Q4_K M = 24 138 -> 126, gate and up of
+// 18944 x 3584 Q4_0 at M = 4 34 -> 29.
+// ONE: per divides the steps of a tile, so that a work-group has one tile or a
+// part of it; the code for several cost such a call 3 to 5 % (14336 x 4096 Q4_K
+// M = 8 16.9 -> 17.7).
+template <int F, bool PAIR, int TT, int RW, int KG, bool ONE>
+__global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int per, int total) {
     using Q = TQ<F>;
     using TH = Thin<F, TT, RW, KG>;
     __shared__ __attribute__((aligned(16))) uint8_t lds[TH::LDS];
@@ -397,34 +423,39 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int sb_pe
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int rw = wave % RW, kg = wave / RW;
     const int c = lane & 15, q = lane >> 4;
-    const RowTile rt = row_tile<PAIR>(a, blockIdx.x, TH::BN);
-    const int nsb = a.K / 256;
-    const int b0 = blockIdx.z * sb_per_split, b1 = min(nsb, b0 + sb_per_split);
-    // this wave's 16 rows: tile_row .. of base
+    const int nsb = a.K / 256, nst = (nsb + KG - 1) / KG;  // mmqt_steps
+    const int s0 = blockIdx.x * per, s1 = min(total, s0 + per);
+    // this wave's 16 rows of a tile
     const bool up = PAIR && rw >= RW / 2;
-    const int tile_row = rt.n0 + 16 * (PAIR ? rw % (RW / 2) : rw);
-    const uint8_t* const base = up ? a.w2 : rt.w;
+    const int wrow = 16 * (PAIR ? rw % (RW / 2) : rw);
 
-    // copy sources.  SHIFT: offsets from the matrix's aligned-down base, not
-    // yet aligned themselves (the super-block's start is added first)
-    const uint32_t mis = Q::SHIFT ? (uint32_t)(reinterpret_cast<uintptr_t>(base) & 15) : 0u;
-    const uint8_t* const wb = base - mis;
+    // copy sources in tile it, step ij.  SHIFT: offsets from the matrix's
+    // aligned-down base, not yet aligned themselves (the super-block's start is
+    // added first)
+    int it = s0 / nst, ij = s0 - it * nst;
+    const uint8_t* wb;
     uint32_t woff[TH::PI], wp[TH::PI];
+    auto source = [&](int t) __attribute__((always_inline)) {
+        const RowTile rt = row_tile<PAIR>(a, t, TH::BN);
+        const uint8_t* const base = up ? a.w2 : rt.w;
+        const uint32_t mis = Q::SHIFT ? (uint32_t)(reinterpret_cast<uintptr_t>(base) & 15) : 0u;
+        wb = base - mis;
 #pragma unroll
-    for (int i = 0; i < TH::PI; ++i) {
-        const int L = min(64 * i + lane, 16 * Q::PPR - 1), r = L / Q::PPR;
-        wp[i] = 16u * (uint32_t)min(L - r * Q::PPR, Q::LAST);
-        woff[i] = (uint32_t)min(tile_row + r, rt.rows - 1) * (uint32_t)a.row_bytes + mis +
-                  (Q::SHIFT ? 0u : wp[i]);
-    }
+        for (int i = 0; i < TH::PI; ++i) {
+            const int L = min(64 * i + lane, 16 * Q::PPR - 1), r = L / Q::PPR;
+            wp[i] = 16u * (uint32_t)min(L - r * Q::PPR, Q::LAST);
+            woff[i] = (uint32_t)min(rt.n0 + wrow + r, rt.rows - 1) * (uint32_t)a.row_bytes + mis +
+                      (Q::SHIFT ? 0u : wp[i]);
+        }
+    };
+    source(it);
     constexpr int XB = XSB / RW, SB = SSB / TH::SW;  // this wave's share of a tile's operands
     const uint8_t* const xb = reinterpret_cast<const uint8_t*>(a.xop) + XB * rw;
     const uint8_t* const sbase = reinterpret_cast<const uint8_t*>(a.xsum) + SB * rw;
     const uint32_t l0 = __builtin_amdgcn_readfirstlane(lds_addr(lds)) + kg * TH::GBUF;
     const bool sums = rw < TH::SW;  // wave-uniform
-    // super-block sb, the it-th of this wave's group
-    auto issue = [&](int sb, int it) {
-        const uint32_t lb = l0 + (uint32_t)(it % TH::NB) * TH::BUF;
+    auto copy = [&](int sb, int n) __attribute__((always_inline)) {
+        const uint32_t lb = l0 + (uint32_t)(n % TH::NB) * TH::BUF;
         const uint32_t lp = lb + (uint32_t)(16 * rw) * (Q::PPR * 16), so = (uint32_t)sb * Q::SBB;
 #pragma unroll
         for (int i = 0; i < TH::PI; ++i) {
@@ -443,32 +474,42 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int sb_pe
                 dma16s(16 * lane, sbase + blk * SSB, lb + TH::PANEL + TT * XSB + T * SSB + SB * rw);
         }
     };
-    // wait until this wave's copies of all but its newest `later` super-blocks
-    // are complete
+    // the copies of this wave for the next step, the n-th of the work-group
+    auto issue = [&](int n) __attribute__((always_inline)) {
+        const int sb = KG * ij + kg;
+        if (KG == 1 || sb < nsb) copy(sb, n);
+        if (++ij == nst && !ONE) {
+            ij = 0;
+            if (s0 + n + 1 < s1) source(++it);
+        }
+    };
+    // wait until this wave's copies of a step are complete; later: those of the
+    // next are under way and nothing else is
     auto wait = [&](bool later) {
         constexpr int C = TH::PI + TH::XC * TT;
         if (TH::NB == 2 || !later) wait_vm<0>();
         else if (sums) wait_vm<C + TT>();
         else wait_vm<C>();
     };
+
+    // a tile's steps enter two sums in turn (Q6_K 152064 x 3584: error against 64
+    // bits 1.17e-7 with one, 1.11e-7 with two)
+    f32x4 acc[TT], acc2[TT];
+#pragma unroll
+    for (int T = 0; T < TT; ++T) acc[T] = acc2[T] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // the tile and step computed
+    int ct = it, cj = ij;
+    RowTile rt = row_tile<PAIR>(a, ct, TH::BN);
     // byte shift of lane row c's super-block in its pieces, before sb's
-    const uint32_t rsh = (uint32_t)(reinterpret_cast<uintptr_t>(base) & 15) +
-                         (uint32_t)min(tile_row + c, rt.rows - 1) * (uint32_t)a.row_bytes;
+    auto row_shift = [&]() __attribute__((always_inline)) {
+        return (uint32_t)(reinterpret_cast<uintptr_t>(up ? a.w2 : rt.w) & 15) +
+               (uint32_t)min(rt.n0 + wrow + c, rt.rows - 1) * (uint32_t)a.row_bytes;
+    };
+    uint32_t rsh = row_shift();
 
-    f32x4 acc[TT];
-#pragma unroll
-    for (int T = 0; T < TT; ++T) acc[T] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-#pragma unroll
-    for (int i = 0; i < TH::NB - 1; ++i)
-        if (b0 + KG * i + kg < b1) issue(b0 + KG * i + kg, i);
-    for (int it = 0; b0 + KG * it < b1; ++it) {
-        const int sb = b0 + KG * it + kg;  // (past b1: this group has none left)
-        wait(sb + KG < b1);
-        __syncthreads();
-        if (sb >= b1) continue;
-        if (sb + KG * (TH::NB - 1) < b1) issue(sb + KG * (TH::NB - 1), it + TH::NB - 1);
-        const uint8_t* buf = lds + kg * TH::GBUF + (it % TH::NB) * TH::BUF;
+    auto compute = [&](int sb, int n) __attribute__((always_inline)) {
+        const uint8_t* buf = lds + kg * TH::GBUF + (n % TH::NB) * TH::BUF;
         const uint8_t* xs = buf + TH::PANEL;
         const uint8_t* ss = xs + TT * XSB;
         Q w;
@@ -534,70 +575,160 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int sb_pe
                     if constexpr (Q::MIN) v = w.d * (v + Dc[i]) + w.dn * Dm[i];
                     else v *= w.d;
                 }
-                acc[T][i] = __builtin_fmaf(v, fv[i], acc[T][i]);
+                v = __builtin_fmaf(v, fv[i], acc[T][i]);
+                acc[T][i] = acc2[T][i];
+                acc2[T][i] = v;
             }
         }
-    }
-    f32x4* const gs = reinterpret_cast<f32x4*>(lds);
-    if constexpr (KG > 1) {  // the groups' sums, added in group order
-        __syncthreads();
+    };
+
+    // the sums of tile ct, step n of the work-group its last one here
+    auto flush = [&](int n) __attribute__((always_inline)) {
+        const Parts ps = ONE && per == nst ? Parts{0, 1} : tile_parts(ct, nst, per);
+        const bool split = ps.n > 1;
 #pragma unroll
-        for (int T = 0; T < TT; ++T)
-            if (kg > 0) gs[(wave * TT + T) * 64 + lane] = acc[T];
-        __syncthreads();
-        if (kg == 0) {
+        for (int T = 0; T < TT; ++T) acc[T] += acc2[T];
+        // exchanged in the buffer just read: the next copies into it come after
+        // the next step's barrier
+        f32x4* const gs = reinterpret_cast<f32x4*>(lds + (n % TH::NB) * TH::BUF);
+        if constexpr (KG > 1) {  // the groups' sums, added in group order
+            __syncthreads();
 #pragma unroll
-            for (int k = 1; k < KG; ++k)
+            for (int T = 0; T < TT; ++T)
+                if (kg > 0) gs[(wave * TT + T) * 64 + lane] = acc[T];
+            __syncthreads();
+            if (kg == 0) {
 #pragma unroll
-                for (int T = 0; T < TT; ++T) acc[T] += gs[((k * RW + rw) * TT + T) * 64 + lane];
-        }
-    }
-    const bool split = gridDim.z > 1;
-    if constexpr (PAIR) {  // the up waves hand their sums to the gate waves
-        __syncthreads();
+                for (int k = 1; k < KG; ++k)
 #pragma unroll
-        for (int T = 0; T < TT; ++T)
-            if (kg == 0 && up && !split) gs[(wave * TT + T) * 64 + lane] = acc[T];
-        __syncthreads();
-    }
-    if (kg > 0 || (PAIR && up && !split)) return;
-    // lane (c, q): row c of the wave's tile, tokens 16 T + 4 q + i
-    const int cols = PAIR ? 2 * a.N : a.N, n = tile_row + c;
-    if (n >= rt.rows) return;
-    float* const out = split ? a.part + (size_t)blockIdx.z * a.M * cols : a.y;
-#pragma unroll
-    for (int T = 0; T < TT; ++T) {
-        f32x4 u = acc[T];
-        if constexpr (PAIR) {
-            if (!split) u = gs[((rw + RW / 2) * TT + T) * 64 + lane];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int m = 16 * T + 4 * q + i;
-            if (m >= a.M) continue;
-            if (split) {
-                out[(size_t)m * cols + rt.col + (up ? a.N : 0) + n] = acc[T][i];
-            } else if constexpr (PAIR) {
-                out[(size_t)m * a.N + n] = silu_mul(acc[T][i], u[i]);
-            } else {
-                float v = acc[T][i];
-                if (a.bias_mode == 1) v += n < a.bias_len ? a.bias[n] : 0.0f;
-                else if (a.bias_mode == 2) v += a.bias[(size_t)m * a.N + n];
-                out[(size_t)m * cols + rt.col + n] = v;
+                    for (int T = 0; T < TT; ++T) acc[T] += gs[((k * RW + rw) * TT + T) * 64 + lane];
             }
         }
+        if constexpr (PAIR) {  // the up waves hand their sums to the gate waves
+            __syncthreads();
+#pragma unroll
+            for (int T = 0; T < TT; ++T)
+                if (kg == 0 && up && !split) gs[(wave * TT + T) * 64 + lane] = acc[T];
+            __syncthreads();
+        }
+        // lane (c, q): row c of the wave's tile, tokens 16 T + 4 q + i (m0, opaque: the
+        // compiler would keep every address in registers through the steps)
+        int m0 = 4 * q;
+        asm volatile("" : "+v"(m0));
+        const int cols = PAIR ? 2 * a.N : a.N, nr = rt.n0 + wrow + c;
+        if (kg > 0 || (PAIR && up && !split) || nr >= rt.rows) return;
+        if (split) {
+            float* const out = a.part + (size_t)(blockIdx.x - ps.first) * a.M * cols + rt.col + nr;
+#pragma unroll
+            for (int T = 0; T < TT; ++T)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int m = 16 * T + m0 + i;
+                    if (m < a.M) out[(size_t)m * cols + (up ? a.N : 0)] = acc[T][i];
+                }
+            return;
+        }
+#pragma unroll
+        for (int T = 0; T < TT; ++T) {
+            f32x4 v = acc[T];
+            if constexpr (PAIR) {
+                const f32x4 u = gs[((rw + RW / 2) * TT + T) * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = silu_mul(v[i], u[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = 16 * T + m0 + i;
+                if (m < a.M) a.y[(size_t)m * a.N + rt.col + nr] = PAIR ? v[i] : biased(a, v[i], m, nr);
+            }
+        }
+    };
+
+#pragma unroll
+    for (int i = 0; i < TH::NB - 1; ++i)
+        if (s0 + i < s1) issue(i);
+    bool stored = false;  // the step before ended a tile: its stores are under way too
+    for (int s = s0; s < s1; ++s) {
+        const int n = s - s0, nj = cj + 1 == nst ? 0 : cj + 1;
+        wait((ONE || !stored) && s + 1 < s1 && (KG == 1 || KG * nj + kg < nsb));
+        __syncthreads();
+        if (s + TH::NB - 1 < s1) issue(n + TH::NB - 1);
+        const int sb = KG * cj + kg;
+        if (KG == 1 || sb < nsb) compute(sb, n);
+        cj = nj;
+        if constexpr (ONE) continue;
+        stored = nj == 0;
+        if (!stored || s + 1 == s1) continue;
+        flush(n);
+        rt = row_tile<PAIR>(a, ++ct, TH::BN);
+        rsh = row_shift();
+#pragma unroll
+        for (int T = 0; T < TT; ++T) acc[T] = acc2[T] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
+    flush(s1 - 1 - s0);
+}
+
+// y of the tiles in parts, added in order: a work-group per tile and 256 R of
+// its results.  R = 4 where a tile has few parts (a head's thousands of
+// work-groups of one result per thread, most with nothing to add, took 10 us),
+// else 1: a thread's loads are a serial chain of few at a time.
+template <bool PAIR, int R>
+__global__ __launch_bounds__(256) void reducet_kernel(MmqArgs a, int bn, int nst, int per) {
+    const Parts ps = tile_parts(blockIdx.x, nst, per);
+    if (ps.n == 1) return;
+    const RowTile rt = row_tile<PAIR>(a, blockIdx.x, bn);
+    const int nc = PAIR ? bn / 2 : bn, cols = PAIR ? 2 * a.N : a.N;
+    const size_t slab = (size_t)a.M * cols;
+    const float* p[R];
+    float v[R], u[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {  // past the end: the last one's values, not stored
+        const int i = blockIdx.y * (256 * R) + 256 * k + threadIdx.x;
+        p[k] = a.part + (size_t)min(i / nc, a.M - 1) * cols + rt.col + min(rt.n0 + i % nc, rt.rows - 1);
+        v[k] = p[k][0];
+        u[k] = PAIR ? p[k][a.N] : 0.0f;
+    }
+#pragma unroll(R == 1 ? 8 : 1)
+    for (int z = 1; z < ps.n; ++z)
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            v[k] += p[k][z * slab];
+            if constexpr (PAIR) u[k] += p[k][z * slab + a.N];
+        }
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int i = blockIdx.y * (256 * R) + 256 * k + threadIdx.x, m = i / nc, n = rt.n0 + i % nc;
+        if (m >= a.M || n >= rt.rows) continue;
+        if constexpr (PAIR) a.y[(size_t)m * a.N + n] = silu_mul(v[k], u[k]);
+        else a.y[(size_t)m * cols + rt.col + n] = biased(a, v[k], m, n);
+    }
+}
+template <bool PAIR>
+void reducet(const MmqArgs& a, int bn, int nst, int per, hipStream_t st) {
+    const int tiles = row_tiles(a, bn), n = a.M * (PAIR ? bn / 2 : bn);
+    if (mmqt_parts(nst, per) <= 3)
+        hipLaunchKernelGGL((reducet_kernel<PAIR, 4>), dim3(tiles, (n + 1023) / 1024), dim3(256), 0, st, a,
+                           bn, nst, per);
+    else
+        hipLaunchKernelGGL((reducet_kernel<PAIR, 1>), dim3(tiles, (n + 255) / 256), dim3(256), 0, st, a,
+                           bn, nst, per);
 }
 
 template <int F, int TT, int RW, int KG>
-hipError_t go(const MmqArgs& a, int splits, hipStream_t st) {
-    const int nsb = a.K / 256, sps = (nsb + splits - 1) / splits;
-    if (sps * (splits - 1) >= nsb) return hipErrorInvalidValue;  // an empty split
-    const dim3 grid(row_tiles(a, 16 * RW), 1, splits), wg(64 * RW * KG);
-    if (a.mm == MM_PAIR)
-        hipLaunchKernelGGL((mmqt_kernel<F, true, TT, RW, KG>), grid, wg, 0, st, a, sps);
-    else
-        hipLaunchKernelGGL((mmqt_kernel<F, false, TT, RW, KG>), grid, wg, 0, st, a, sps);
+hipError_t go(const MmqArgs& a, int per, hipStream_t st) {
+    const int tiles = row_tiles(a, 16 * RW), nst = mmqt_steps(a.K, KG), total = tiles * nst;
+    const bool parts = mmqt_parts(nst, per) > 1;
+    const dim3 grid((total + per - 1) / per), wg(64 * RW * KG);
+    auto run = [&](auto pair) {
+        constexpr bool P = decltype(pair)::value;
+        if (nst % per == 0)
+            hipLaunchKernelGGL((mmqt_kernel<F, P, TT, RW, KG, true>), grid, wg, 0, st, a, per, total);
+        else
+            hipLaunchKernelGGL((mmqt_kernel<F, P, TT, RW, KG, false>), grid, wg, 0, st, a, per, total);
+        if (parts) reducet<P>(a, 16 * RW, nst, per, st);
+    };
+    if (a.mm == MM_PAIR) run(std::true_type{});
+    else run(std::false_type{});
     return hipGetLastError();
 }
 // Work-groups of 256, 128 or 64 rows, each in wave groups of as many waves as
@@ -614,15 +745,15 @@ constexpr int groups(int rows) {
                          : 0;
 }
 template <int F, int TT>
-hipError_t go_f(const MmqArgs& a, int rows, int splits, hipStream_t st) {
+hipError_t go_f(const MmqArgs& a, int rows, int per, hipStream_t st) {
     if constexpr (groups<F, TT>(256) != 0) {
-        if (rows == 256) return go<F, TT, 16, 1>(a, splits, st);
+        if (rows == 256) return go<F, TT, 16, 1>(a, per, st);
     }
     if constexpr (groups<F, TT>(128) != 0) {
-        if (rows == 128) return go<F, TT, 8, groups<F, TT>(128)>(a, splits, st);
+        if (rows == 128) return go<F, TT, 8, groups<F, TT>(128)>(a, per, st);
     }
     if constexpr (groups<F, TT>(64) != 0) {
-        if (rows == 64) return go<F, TT, 4, 2>(a, splits, st);
+        if (rows == 64) return go<F, TT, 4, 2>(a, per, st);
     }
     return hipErrorInvalidValue;
 }
@@ -660,11 +791,11 @@ hipError_t launch_xprept(int dtype, const float* x, int M, int K, uint8_t* xop, 
     return hipGetLastError();
 }
 
-hipError_t launch_mmqt(int dtype, const MmqArgs& a, int rows, int splits, hipStream_t st) {
-    if (a.M > 32 || a.K % 256 != 0 || splits < 1) return hipErrorInvalidValue;
+hipError_t launch_mmqt(int dtype, const MmqArgs& a, int rows, int per, hipStream_t st) {
+    if (a.M > 32 || a.K % 256 != 0 || per < 1) return hipErrorInvalidValue;
     return with_thin(dtype, hipErrorInvalidValue, [&](auto f) {
         constexpr int F = decltype(f)::value;
-        return a.M <= 16 ? go_f<F, 1>(a, rows, splits, st) : go_f<F, 2>(a, rows, splits, st);
+        return a.M <= 16 ? go_f<F, 1>(a, rows, per, st) : go_f<F, 2>(a, rows, per, st);
     });
 }
 

@@ -106,3 +106,29 @@ def test_extreme_codes_and_scales(dtype):
         d = w.reshape(N, -1, f.block_bytes)[:, :, 0:4].copy().view(np.float16).astype(np.float64)
         scale = 63 * (31 * np.abs(d[..., 0]) + np.abs(d[..., 1]))[:, cols // 256].T
         assert (np.abs(y - deq[:, cols].T) <= 2.0 ** -22 * scale).all()
+
+
+# More row tiles than CUs: a work-group's range of steps runs over the ends of
+# several tiles, whole ones and parts, odd step counts over two wave groups,
+# from one matrix into the next
+@pytest.mark.parametrize("dtype", [F.Q4_K, F.Q6_K, F.Q5_1, F.Q8_0])
+@pytest.mark.parametrize("M,K,ns", [(21, 256, (70001,)), (32, 768, (40000,)), (18, 1280, (33333,)),
+                                    (27, 768, (17001, 130, 16400))])
+def test_ranges_over_tiles(dtype, M, K, ns):
+    ws = [synth.make_weights(dtype, n, K, 70 + i) for i, n in enumerate(ns)]
+    x = synth.make_x(M, K, seed=M)
+    xd, Ws = torch.from_numpy(x).cuda(), [dev_weight(dtype, w, n, K) for w, n in zip(ws, ns)]
+    y = ops.matmul_transB(xd, Ws[0]) if len(ns) == 1 else ops.fused_qkv(xd, *Ws)
+    ref = np.concatenate([oracle.matmul_f64(dtype, x, w, len(w), K) for w in ws], axis=1)
+    assert_close(y.cpu().numpy(), ref, x, np.array([wmax(dtype, ws, K)]), f"{dtype} {M} {ns} {K}")
+
+
+@pytest.mark.parametrize("dtype", [F.Q4_K, F.Q6_K, F.Q5_1, F.Q8_0])
+@pytest.mark.parametrize("M,N,K", [(3, 20003, 1280), (4, 40000, 256), (30, 20100, 768)])
+def test_pair_ranges_over_tiles(dtype, M, N, K):
+    wg, wu = (synth.make_weights(dtype, N, K, s) for s in (52, 53))
+    x = synth.make_x(M, K, seed=M) * np.float32(1e-2)
+    y = ops.ffn_up_fused(torch.from_numpy(x).cuda(), dev_weight(dtype, wg, N, K),
+                         dev_weight(dtype, wu, N, K))
+    g, u = (oracle.matmul_f64(dtype, x, w, N, K) for w in (wg, wu))
+    assert_close_silu_mul(y.cpu().numpy(), g, u, x, wmax(dtype, [wg, wu], K), f"{dtype} {M}x{N}x{K}")
