@@ -466,7 +466,7 @@ MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
 // 8192 x 4096, 19 MB, 12.6 us there, 13.5 here, 14336 x 4096, 33 MB, 18.7 and
 // 16.3; Q6_K 28 MB 16.5 and 16.8, 48 MB 27.6 and 20.9; Q8_0 36 MB 14.1 and
 // 15.3, 62 MB 23.5 and 19.2; Q4_0 33 MB 17.8 and 17.3, 38 MB 24.0 and 20.0;
-// 152064 x 3584: Q4_0 132 and 100, Q8_0 171 and 133, Q6_K 211 and 131).
+// 152064 x 3584: Q4_0 132 and 100, Q8_0 171 and 132, Q6_K 211 and 124).
 bool thin_takes(uint32_t dtype, int M, int64_t bytes) {
     if (!fq::mmqt_supported((int)dtype) || M < 4 || M > 32) return false;
     const int64_t mib = dtype == FQ_DTYPE_Q4_K || dtype == FQ_DTYPE_Q5_K ? 24

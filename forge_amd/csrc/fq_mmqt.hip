@@ -18,8 +18,9 @@
 // work-group.  152064 x 3584 Q6_K, M = 16: 216 -> 129 us; Q4_K, M = 8 131 ->
 // 98; 14336 x 4096 Q4_K, M = 8 18.7 -> 16.3, M = 32 (fp16 MFMA kernel) 40.2 ->
 // 23.2, gate and up of that size in one launch 37.7 -> 22.0 and 82.5 -> 36.0.
-// What bounds it: vector and matrix issue with the LDS reads of the token
-// operands, about equal (with a work-group per tile half, 139 us in all, the head
+// What bounds it: vector and matrix issue, then the LDS reads of the token
+// operands (Q6_K head, M = 16: vector issue 68 % of the cycles, the matrix
+// cores 22 %, LDS 33 %; with a work-group per tile half, 139 us in all, the head
 // took 117 without the copies, 105 without the arithmetic), so the waves per SIMD count: 256 rows on eight waves of
 // two tiles each ran the head in 152 us, on sixteen waves 139.
 //

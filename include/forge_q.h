@@ -186,8 +186,9 @@ int fq_ffn_up_fused_packed(uint32_t dtype, const float* x, const void* w_gate_pa
 
 /* GGUF-layout weights, any M >= 1.  Replaces matmul_transB_fused_qkv_q4_0 /
  * _q4_k (matmul.cpp:1535-1600, 1639-1692) and the CUDA fused QKV launcher
- * (cuda_fused.cu:924-1024); at M > 1 the three results pass through a
- * library-owned per-stream buffer. */
+ * (cuda_fused.cu:924-1024); at M > 1 one launch where one kernel takes all
+ * three matrices, else the three results pass through a library-owned
+ * per-stream buffer. */
 int fq_fused_qkv(uint32_t dtype, const float* x, const void* wq, const void* wk, const void* wv,
                  float* y, int M, int K, int Nq, int Nk, int Nv, void* stream);
 
