@@ -21,8 +21,9 @@
 // What bounds it: vector and matrix issue, then the LDS reads of the token
 // operands (Q6_K head, M = 16: vector issue 68 % of the cycles, the matrix
 // cores 22 %, LDS 33 %; with a work-group per tile half, 139 us in all, the head
-// took 117 without the copies, 105 without the arithmetic), so the waves per SIMD count: 256 rows on eight waves of
-// two tiles each ran the head in 152 us, on sixteen waves 139.
+// took 117 without the copies, 105 without the arithmetic), so the waves per
+// SIMD count: 256 rows on eight waves of two tiles each ran the head in 152 us,
+// on sixteen waves 139.
 //
 // Tokens are the A operand of v_mfma_f32_16x16x32_f16 (lane 16 q + c: token c,
 // eight elements of k group q) and weights the B operand (lane 16 q + c: row
