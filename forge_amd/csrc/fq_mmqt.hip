@@ -34,8 +34,8 @@
 //
 //   Q4_K, Q5_K: sc (q - c) as in fq_mmqk.hip, exact in fp16 (at most 1008);
 //   Q6_K: sc (q - 32) has up to 13 bits: W = W_hi + W_lo, W_hi its fp16
-//   rounding and W_lo the exact rest; x W = x_hi W_hi + x_lo W_hi + x_hi W_lo
-//   (the dropped x_lo W_lo is 2^-23 of the product).
+//   rounding and W_lo the exact rest; all four products are formed (without
+//   x_lo W_lo, up to 2^-22 of a product, the codes would not be exact).
 //
 //   the 32-element blocks: the integer code, d on the results (TQB below).
 //
@@ -544,8 +544,10 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int per, 
                 f32x4& d = D[KSI >> 1][T];
                 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, whi, KSI & 1 ? d : z, 0, 0, 0);
                 Dl[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, whi, KSI ? Dl[T] : z, 0, 0, 0);
-                if constexpr (Q::SPLITW)
+                if constexpr (Q::SPLITW) {
+                    Dl[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, wlo, Dl[T], 0, 0, 0);
                     Dl[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, wlo, Dl[T], 0, 0, 0);
+                }
             }
         };
         ks(std::integral_constant<int, 0>{});
