@@ -39,9 +39,14 @@
 //
 //   the 32-element blocks: the integer code, d on the results (TQB below).
 //
-// Short MFMA chains, added up per super-block, then acc += 2^e (d D - dmin Dm), e the
-// token's exponent for this super-block (x 2^-e below 2^15, split into fp16
-// hi + lo: 22 significant bits).
+// Short MFMA chains, added up per super-block, then acc += 2^e (d D + Dm), e the
+// token's exponent (x 2^-e below 2^15, split into fp16 hi + lo: 22 significant
+// bits) and Dm the minimum and centring terms, an fp32 product of the token's
+// sub-block sums.  The 32-element blocks have an exponent per 64 elements.  The
+// K-quants have one per super-block, whose 64-element quarters one MFMA spans;
+// their x_lo is kept 2^12 larger, in a chain of its own, so that an element
+// keeps its bits down to 2^-29 of the super-block's largest (fp16's least
+// value alone: 2^-17) and is 2^-51 of that largest off at most.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -59,18 +64,18 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int XSB = 16384;  // operand bytes of a (16-token tile, super-block): [ks][hi, lo][lane][8]
-// sums and scales of a (tile, super-block): eight groups of 144 bytes, group
-// w: the sums operand of lanes 8 w .. 8 w + 7, then (w < 4) the floats 2^e of
-// tokens 4 w .. 4 w + 3
-constexpr int SG = 144, SSB = 8 * SG;
+// sums and scales of a (tile, super-block), floats: lane 16 q + c's sums of token
+// c's sub-blocks 2 q and 2 q + 1, then 2^e of tokens 0 .. 15, of each 64-element
+// group (K-quants: the first alone, of the super-block)
+constexpr int SEXP = 64 * 8, SSB = SEXP + 4 * 64;
+constexpr float LO = 0x1p12f;  // what the K-quants' x_lo is larger by
 
 // ------------------------------------------------------------- token prep
 // One work-group per super-block and 16-token tile; thread 16 c + p holds
 // elements 16 p .. 16 p + 15 of token c.  Eight elements 8 e8 .. + 7 are slots
 // (slot_elem order) of lane group q in MFMA ks: Q4_K / Q5_K (MAP 0) q = e8 /
 // 8, ks = e8 % 8; Q6_K (MAP 1) element 128 n + 32 u + 16 h + 8 i: q = 2 n + h,
-// ks = 2 u + i; 32-element blocks (MAP 2) ks the block, q = e8 % 4.  The sums operand of lane (c, q) holds token c's sums (times 2^-5) over
-// sub-blocks 2 q, 2 q + 1 in three fp16 parts: hi, hi, mid, mid, lo, lo, 0, 0.
+// ks = 2 u + i; 32-element blocks (MAP 2) ks the block, q = e8 % 4.
 template <int MAP>
 __global__ __launch_bounds__(256) void xprept_kernel(const float* __restrict__ x, int M, int K,
                                                      uint8_t* __restrict__ xop,
@@ -93,7 +98,7 @@ __global__ __launch_bounds__(256) void xprept_kernel(const float* __restrict__ x
 #pragma unroll
     for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(v[i]));
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    for (int o = 1; o < (MAP == 2 ? 4 : 16); o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     const int e = (mx > 0.0f && mx <= 3.0e38f) ? ilogbf(mx) - 14 : 0;
     float sum = 0.0f;
     uint8_t* const ob = xop + ((size_t)T * nsb + sb) * XSB;
@@ -110,30 +115,22 @@ __global__ __launch_bounds__(256) void xprept_kernel(const float* __restrict__ x
         for (int j = 0; j < 8; ++j) {
             const float u = w[slot_elem(j)];
             hi[j] = (_Float16)u;
-            lo[j] = (_Float16)(u - (float)hi[j]);
+            lo[j] = (_Float16)((u - (float)hi[j]) * (MAP == 2 ? 1.0f : LO));
         }
         h8* o = reinterpret_cast<h8*>(ob + ks * 2048 + (16 * q + c) * 16);
         o[0] = hi;
         o[64] = lo;
         sum += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
     }
-    uint8_t* const sbk = xs + ((size_t)T * nsb + sb) * SSB;
-    if (p == 0) *reinterpret_cast<float*>(sbk + (c >> 2) * SG + 128 + 4 * (c & 3)) =
-        __builtin_amdgcn_ldexpf(1.0f, e);
+    float* const sbk = reinterpret_cast<float*>(xs + ((size_t)T * nsb + sb) * SSB);
+    if (p % (MAP == 2 ? 4 : 16) == 0) sbk[SEXP / 4 + 4 * p + c] = __builtin_amdgcn_ldexpf(1.0f, e);
     if constexpr (MAP != 1) {
         sum += __shfl_xor(sum, 1, 64);
-        if ((p & 1) == 0) {
-            const int b = p >> 1, l = 16 * (b >> 1) + c;
-            const float s = sum * 0x1p-5f;
-            const _Float16 s0 = (_Float16)s;
-            const float r = s - (float)s0;
-            const _Float16 s1 = (_Float16)r;
-            _Float16* d = reinterpret_cast<_Float16*>(sbk + (l >> 3) * SG + (l & 7) * 16) + (b & 1);
-            d[0] = s0;
-            d[2] = s1;
-            d[4] = (_Float16)(r - (float)s1);
-            d[6] = (_Float16)0.0f;
-        }
+        const int b = p >> 1;
+        // (K-quants: times 2^-e; the others, of several e, as they are, times
+        // 2^-5: no larger than the largest x)
+        if ((p & 1) == 0)
+            sbk[2 * (16 * (b >> 1) + c) + (b & 1)] = MAP == 2 ? __builtin_amdgcn_ldexpf(sum, e - 5) : sum;
     }
 }
 
@@ -161,8 +158,7 @@ struct TQK {
     static constexpr float UNIT = F == Q5_K ? 8.0f : 16.0f, MID = F == Q5_K ? 16.0f : 8.0f;
     uint32_t w[8], h[8];
     h2 s[2], off[2];
-    h8 mb, cb;
-    float d, dn;
+    float d, wm[2];
     // row's super-block at p (LDS), lane group q
     __device__ void load(const uint8_t* p, int, int q) {
         const fq_u32x4 hd = lds16(p);
@@ -189,12 +185,10 @@ struct TQK {
         s[1] = h2{u1, u1};
         off[0] = s[0] * h2{(_Float16)-1152.0f, (_Float16)-1152.0f};
         off[1] = s[1] * h2{(_Float16)-1152.0f, (_Float16)-1152.0f};
-        const _Float16 m0 = (_Float16)(float)ma, m1 = (_Float16)(float)mi, z = (_Float16)0.0f;
-        mb = h8{m0, m1, m0, m1, m0, m1, z, z};
-        const _Float16 c0 = (_Float16)(f0 * (32.0f * MID)), c1 = (_Float16)(f1 * (32.0f * MID));
-        cb = h8{c0, c1, c0, c1, c0, c1, z, z};
         d = f16_hw(hd.x & 0xFFFFu);
-        dn = -32.0f * f16_hw(hd.x >> 16);
+        const float dm = f16_hw(hd.x >> 16);
+        wm[0] = __builtin_fmaf(d * MID, f0, -(dm * (float)ma));
+        wm[1] = __builtin_fmaf(d * MID, f1, -(dm * (float)mi));
     }
     template <int KSI>
     __device__ uint32_t code(int k) const {
@@ -289,7 +283,7 @@ struct TQ<Q6_K> {
 // qh.  The operand holds the integer code (IQ4_NL: the table value), the
 // block's scale d multiplies the MFMA pair's results (d codes have up to 19
 // bits).  Q4_1 and Q5_1, w = d q + m, enter as d (q - c) + (m + c d), c 8 or 16,
-// with m and d (fp16 both) on the sub-block sums.  Rows of 160 and 192
+// the second term on the sub-block sums.  Rows of 160 and 192
 // bytes take a repeated piece, so that 16 rows start on eight banks, not four
 // or two.
 template <int F>
@@ -301,8 +295,7 @@ struct TQB {
     static constexpr int QH = F == Q5_0 ? 2 : 4;
     static constexpr float MID = F == Q5_0 || F == Q5_1 ? 16.0f : 8.0f;  // subtracted from a code
     uint32_t w[16], h[8];
-    float db[8];
-    h8 mb, cb;
+    float db[8], wm[2];
     int sh;
     // the dword at p + o, o even and known at compile time
     template <int O>
@@ -335,12 +328,10 @@ struct TQB {
         block<5>(p, pq, q);
         block<6>(p, pq, q);
         block<7>(p, pq, q);
-        if constexpr (MIN) {  // m and d of this lane group's sub-blocks 2 q, 2 q + 1
+        if constexpr (MIN) {  // m + c d of this lane group's sub-blocks 2 q, 2 q + 1
             const uint32_t d0 = lds4(p + 2 * BB * q), d1 = lds4(p + 2 * BB * q + BB);
-            const h2 u = __builtin_bit_cast(h2, d0), v = __builtin_bit_cast(h2, d1);
-            const _Float16 z = (_Float16)0.0f;
-            mb = h8{u[1], v[1], u[1], v[1], u[1], v[1], z, z};
-            cb = h8{u[0], v[0], u[0], v[0], u[0], v[0], z, z};
+            wm[0] = __builtin_fmaf(MID, f16_hw(d0 & 0xFFFFu), f16_hw(d0 >> 16));
+            wm[1] = __builtin_fmaf(MID, f16_hw(d1 & 0xFFFFu), f16_hw(d1 >> 16));
         }
     }
     template <int KSI>
@@ -519,8 +510,20 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int per, 
                Q::SHIFT ? (int)((rsh + (uint32_t)sb * Q::SBB) & 15u) : 0, q);
         // The matrix cores' additions round toward zero, so a chain's error
         // grows with its length times its magnitude: four chains of two for
-        // the large products (x_hi W_hi), one for the small ones
-        f32x4 D[4][TT], Dl[TT];
+        // the large products (x_hi W_hi), one each for those of x_lo and W_lo.
+        // 32-element blocks: D[0] the sum of d D over a 64-element group, Dl those
+        // groups' sum (added to the tile's sums one by one: 1.10e-7 against
+        // 1.02e-7, Q4_0 at K = 3584)
+        f32x4 D[4][TT], Dl[TT], Dw[TT];
+        auto exps = [&](int T, int g) {
+            return *reinterpret_cast<const f32x4*>(ss + T * SSB + SEXP + 64 * g + 16 * q);
+        };
+        // a value joins a tile's sums, the two in turn
+        auto add = [&](int T, int i, float v, float f) {
+            v = __builtin_fmaf(v, f, acc[T][i]);
+            acc[T][i] = acc2[T][i];
+            acc2[T][i] = v;
+        };
         const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
         auto ks = [&](auto ki) {
             constexpr int KSI = decltype(ki)::value;
@@ -532,13 +535,20 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int per, 
                 const uint8_t* xp = xs + T * XSB + KSI * 2048 + 16 * lane;
                 const h8 xh = *reinterpret_cast<const h8*>(xp);
                 const h8 xl = *reinterpret_cast<const h8*>(xp + 1024);
-                if constexpr (Q::BLOCKS) {  // Dl: the sum of d D over the blocks so far
+                if constexpr (Q::BLOCKS) {
                     // (x_lo first: 1.8e-7 against 1.2e-7 at K = 18944)
                     f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, whi, z, 0, 0, 0);
                     d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, whi, d, 0, 0, 0);
+                    f32x4& dd = D[0][T];
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        Dl[T][i] = KSI ? __builtin_fmaf(w.db[KSI], d[i], Dl[T][i]) : w.db[0] * d[i];
+                        dd[i] = KSI & 1 ? __builtin_fmaf(w.db[KSI], d[i], dd[i]) : w.db[KSI] * d[i];
+                    if constexpr (KSI & 1) {
+                        const f32x4 f = exps(T, KSI >> 1);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            Dl[T][i] = KSI > 1 ? __builtin_fmaf(dd[i], f[i], Dl[T][i]) : dd[i] * f[i];
+                    }
                     continue;
                 }
                 f32x4& d = D[KSI >> 1][T];
@@ -546,7 +556,7 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int per, 
                 Dl[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, whi, KSI ? Dl[T] : z, 0, 0, 0);
                 if constexpr (Q::SPLITW) {
                     Dl[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, wlo, Dl[T], 0, 0, 0);
-                    Dl[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, wlo, Dl[T], 0, 0, 0);
+                    Dw[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, wlo, KSI ? Dw[T] : z, 0, 0, 0);
                 }
             }
         };
@@ -560,28 +570,25 @@ __global__ __launch_bounds__(64 * RW * KG) void mmqt_kernel(MmqArgs a, int per, 
         ks(std::integral_constant<int, 7>{});
 #pragma unroll
         for (int T = 0; T < TT; ++T) {
-            const uint8_t* st = ss + T * SSB;
-            const float4 f = *reinterpret_cast<const float4*>(st + q * SG + 128);
-            const float fv[4] = {f.x, f.y, f.z, f.w};
-            f32x4 Dc = z, Dm = z;
+            f32x4 Dm = z;
             if constexpr (Q::MIN) {
-                const h8 S = *reinterpret_cast<const h8*>(st + (lane >> 3) * SG + (lane & 7) * 16);
-                Dc = __builtin_amdgcn_mfma_f32_16x16x32_f16(S, w.cb, z, 0, 0, 0);
-                Dm = __builtin_amdgcn_mfma_f32_16x16x32_f16(S, w.mb, z, 0, 0, 0);
+                const float2 S = *reinterpret_cast<const float2*>(ss + T * SSB + 8 * lane);
+                Dm = __builtin_amdgcn_mfma_f32_16x16x4f32(S.x, w.wm[0], z, 0, 0, 0);
+                Dm = __builtin_amdgcn_mfma_f32_16x16x4f32(S.y, w.wm[1], Dm, 0, 0, 0);
             }
+            if constexpr (!Q::BLOCKS) {
+                const f32x4 f = exps(T, 0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float v = Dl[T][i];
-                if constexpr (Q::BLOCKS) {
-                    if constexpr (Q::MIN) v += 32.0f * __builtin_fmaf(Q::MID, Dc[i], Dm[i]);
-                } else {
-                    v += (D[0][T][i] + D[1][T][i]) + (D[2][T][i] + D[3][T][i]);
-                    if constexpr (Q::MIN) v = w.d * (v + Dc[i]) + w.dn * Dm[i];
-                    else v *= w.d;
+                for (int i = 0; i < 4; ++i) {
+                    float v = (D[0][T][i] + D[1][T][i]) + (D[2][T][i] + D[3][T][i]);
+                    if constexpr (Q::SPLITW) v += __builtin_fmaf(Dl[T][i], 1.0f / LO, Dw[T][i]);
+                    else v = __builtin_fmaf(Dl[T][i], 1.0f / LO, v);
+                    add(T, i, __builtin_fmaf(w.d, v, Dm[i]), f[i]);
                 }
-                v = __builtin_fmaf(v, fv[i], acc[T][i]);
-                acc[T][i] = acc2[T][i];
-                acc2[T][i] = v;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    add(T, i, Q::MIN ? __builtin_fmaf(Dm[i], 32.0f, Dl[T][i]) : Dl[T][i], 1.0f);
             }
         }
     };

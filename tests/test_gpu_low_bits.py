@@ -1,20 +1,43 @@
 """Low bits of activations and weights on the fp16 matrix-core kernels, whose
-operands are split into parts: the product of the two low parts."""
+operands are split into parts: the product of the two low parts, and elements
+far below others that share their exponent."""
 from __future__ import annotations
 
 import numpy as np
 import pytest
 import torch
 
+import oracle
 from forge_amd import formats as F
 from forge_amd import ops, synth
 from test_gpu_parity import dev_weight
 
 pytestmark = pytest.mark.gpu
+KQ = [F.Q4_K, F.Q5_K, F.Q6_K]
+ALL = KQ + [F.Q4_0, F.Q4_1, F.Q8_0, F.Q5_0, F.Q5_1, F.IQ4_NL]
 
 
 def run(dtype, w, x, N, K):
     return ops.matmul_transB(torch.from_numpy(x).cuda(), dev_weight(dtype, w, N, K)).cpu().numpy()
+
+
+def rel(dtype, w, x, N, K):
+    ref = oracle.matmul_f64(dtype, x, w, N, K)
+    return np.linalg.norm(run(dtype, w, x, N, K) - ref) / np.linalg.norm(ref)
+
+
+def zero_first_64(dtype, w, N):
+    """Weights that are zero in the first 64 elements of every 256."""
+    f = F.fmt(dtype)
+    b = w.reshape(N, -1, f.block_bytes).copy()
+    if dtype == F.Q6_K:
+        b[:, :, 192:196] = 0
+    elif dtype in (F.Q4_K, F.Q5_K):
+        b[:, :, [4, 5, 8, 9]] &= 0xC0
+    else:
+        for i in (0, 1):
+            b[:, i::8, 0:4 if dtype in (F.Q4_1, F.Q5_1) else 2] = 0
+    return b.reshape(N, -1)
 
 
 # Q6_K, 17..32 tokens: x = hi + lo and sc (q - 32) = 2057 = hi + lo in fp16, both
@@ -34,3 +57,14 @@ def test_product_of_the_low_parts():
     x[np.arange(M), np.arange(M) * 15 + 7] = v
     exact = float(v) * 2057 * 2.0 ** -12
     assert np.abs(run(F.Q6_K, w, x, N, K) - exact).max() <= 3 * 2.0 ** -24 * exact
+
+
+# an element of 2^27 times the others in every super-block, in the 64 elements
+# whose weights are zero: the others' bits are theirs
+@pytest.mark.parametrize("dtype", ALL)
+def test_small_elements_beside_large_ones(dtype):
+    N, K, M = 130, 1024, 20
+    w = zero_first_64(dtype, synth.make_weights(dtype, N, K, seed=3), N)
+    x = synth.make_x(M, K, seed=4)
+    x[:, 5::256] = np.float32(2.0 ** 27)
+    assert rel(dtype, w, x, N, K) <= 1e-6
