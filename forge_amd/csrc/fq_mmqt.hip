@@ -99,7 +99,9 @@ __global__ __launch_bounds__(256) void xprept_kernel(const float* __restrict__ x
     for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(v[i]));
 #pragma unroll
     for (int o = 1; o < (MAP == 2 ? 4 : 16); o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    const int e = (mx > 0.0f && mx <= 3.0e38f) ? ilogbf(mx) - 14 : 0;
+    // (2^e a normal number: -e up to 126 brings every x but the subnormal ones
+    // to 2^0 and more, and those into fp16 exactly)
+    const int e = (mx > 0.0f && mx <= 3.0e38f) ? max(ilogbf(mx) - 14, -126) : 0;
     float sum = 0.0f;
     uint8_t* const ob = xop + ((size_t)T * nsb + sb) * XSB;
 #pragma unroll

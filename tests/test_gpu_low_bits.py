@@ -1,6 +1,6 @@
 """Low bits of activations and weights on the fp16 matrix-core kernels, whose
-operands are split into parts: the product of the two low parts, and elements
-far below others that share their exponent."""
+operands are split into parts: the product of the two low parts, elements far
+below others that share their exponent, and subnormal tokens."""
 from __future__ import annotations
 
 import numpy as np
@@ -68,3 +68,15 @@ def test_small_elements_beside_large_ones(dtype):
     x = synth.make_x(M, K, seed=4)
     x[:, 5::256] = np.float32(2.0 ** 27)
     assert rel(dtype, w, x, N, K) <= 1e-6
+
+
+# tokens of subnormal numbers against weights large enough for normal results
+@pytest.mark.parametrize("dtype", KQ)
+def test_subnormal_tokens(dtype):
+    N, K, M = 70, 512, 20
+    f = F.fmt(dtype)
+    w = synth.make_weights(dtype, N, K, seed=5).reshape(N, -1, f.block_bytes)
+    at = 208 if dtype == F.Q6_K else 0
+    w[:, :, at:at + 2] = np.frombuffer(np.float16(30000.0).tobytes(), dtype=np.uint8)
+    x = (np.random.default_rng(6).integers(-300, 301, (M, K)) * 2.0 ** -149).astype(np.float32)
+    assert rel(dtype, w.reshape(N, -1), x, N, K) <= 1e-6
