@@ -221,7 +221,8 @@ struct MmqpPlan {
 // tiles_n: work-groups along the rows, cols: columns of a partial slab,
 // q6_rows: Q6_K rows to rewrite (0: another format); cap: bytes the plan has
 // to fit where a smaller split count can (0: no limit).
-MmqpPlan plan_mmqp(int M, int K, long tiles_n, int cols, int q6_rows, int cus, size_t cap = 0) {
+MmqpPlan plan_mmqp(uint32_t dtype, int M, int K, long tiles_n, int cols, int q6_rows, int cus,
+                   size_t cap = 0) {
     MmqpPlan p{};
     const int Tn = (M + 31) / 32, nsteps = K / 64;
     const int tm = fq::mmqp_tile_tokens();
@@ -230,7 +231,7 @@ MmqpPlan plan_mmqp(int M, int K, long tiles_n, int cols, int q6_rows, int cus, s
     p.xop_b = (size_t)Tn * K * 64 * 2;
     p.ex_b = (size_t)M * 4;
     // sub-block sums (formats with a min term): floats, or mmqk's hi + lo
-    p.sum_b = (size_t)Tn * std::max<size_t>((size_t)K * 4, fq::mmqk_sum_bytes(K));
+    p.sum_b = (size_t)Tn * (fq::mmqk_supported((int)dtype) ? fq::mmqk_sum_bytes((int)dtype, K) : (size_t)K * 4);
     p.q6c_b = (size_t)fq::mmqp_q6c_bytes(q6_rows, K);  // Q6_K rows as 36-byte blocks
     const size_t fixed_b = 256 + al(p.xop_b) + al(p.ex_b) + al(p.sum_b) + al(p.q6c_b);
     // The split count of the smallest estimated time: rounds of work-groups x
@@ -348,8 +349,8 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
     a.M = M;
     a.N = N;
     a.K = K;
-    const MmqpPlan pl = plan_mmqp(M, K, fq::mmqp_row_tiles(a), fq::mm_cols(a), q6k ? rows : 0, di.cus,
-                                  fixed_cap);
+    const MmqpPlan pl = plan_mmqp(dtype, M, K, fq::mmqp_row_tiles(a), fq::mm_cols(a), q6k ? rows : 0,
+                                  di.cus, fixed_cap);
     const int splits = pl.splits;
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const size_t xop_b = pl.xop_b, ex_b = pl.ex_b, sum_b = pl.sum_b, need = pl.total;
@@ -392,9 +393,12 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
     a.bias = bias;
     a.bias_len = bias_mode ? bias_len : 0;
     a.bias_mode = bias_mode;
-    e = fq::launch_xprep32(x, M, K, reinterpret_cast<_Float16*>(buf), const_cast<int*>(a.ex),
-                           mmqk ? nullptr : sums, mmqk ? reinterpret_cast<_Float16*>(sums) : nullptr,
-                           q6k, st);
+    if (fq::mmqk_fine((int)dtype))
+        e = fq::launch_xprepk(x, M, K, reinterpret_cast<_Float16*>(buf), reinterpret_cast<uint8_t*>(sums), st);
+    else
+        e = fq::launch_xprep32(x, M, K, reinterpret_cast<_Float16*>(buf), const_cast<int*>(a.ex),
+                               mmqk ? nullptr : sums,
+                               mmqk ? reinterpret_cast<_Float16*>(sums) : nullptr, q6k, st);
     if (e != hipSuccess) return hip_fail(e);
     e = mmqk ? fq::launch_mmqk((int)dtype, a, splits, st) : fq::launch_mmqp((int)dtype, a, splits, st);
     if (e == hipSuccess && splits > 1) e = fq::launch_reduce(a, splits, st);
@@ -1564,8 +1568,9 @@ int fq_reserve_workspace(int M_max, int K_max, int N_max, void* stream) {
                 for (int mt : {4, 3, 2}) need0 = std::max(need0, mmqs_need(m, Kp, n, di.cus, mt));
             if (m > 32 && Kp > 0) {  // one matrix, and a gate/up pair
                 const int tn = fq::mmqp_tile_rows();
-                need0 = std::max(need0, plan_mmqp(m, Kp, (n + tn - 1) / tn, n, n, di.cus).total);
-                need0 = std::max(need0, plan_mmqp(m, Kp, (2L * n + tn - 1) / tn, 2 * n, 2 * n, di.cus).total);
+                // (with the larger sums of Q5_K and the rewritten rows of Q6_K)
+                need0 = std::max(need0, plan_mmqp(FQ_DTYPE_Q5_K, m, Kp, (n + tn - 1) / tn, n, n, di.cus).total);
+                need0 = std::max(need0, plan_mmqp(FQ_DTYPE_Q5_K, m, Kp, (2L * n + tn - 1) / tn, 2 * n, 2 * n, di.cus).total);
             }
             if (m <= 32 && Kp > 0) {  // one matrix, and a gate/up pair
                 fq::MmqArgs t{};

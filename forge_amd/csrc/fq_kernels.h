@@ -142,9 +142,12 @@ int mmqp_row_tiles(const MmqArgs& a);  // work-groups along the rows of a's matr
 hipError_t launch_xprep32(const float* x, int M, int K, _Float16* xop, int* ex, float* xsum,
                           _Float16* xsum2, bool sub16, hipStream_t st);
 // the same for Q4_K and Q5_K with the sub-block scales in the weight operand
-// (fq_mmqk.hip): a.xsum holds the hi + lo sums (mmqk_sum_bytes per 32 tokens)
+// (fq_mmqk.hip): a.xsum holds the hi + lo sums (mmqk_sum_bytes per 32 tokens).
+// mmqk_fine (Q5_K): operands of launch_xprepk, a.xsum with exponents, a.ex unused
 bool mmqk_supported(int dtype);
-size_t mmqk_sum_bytes(int K);
+bool mmqk_fine(int dtype);
+size_t mmqk_sum_bytes(int dtype, int K);
+hipError_t launch_xprepk(const float* x, int M, int K, _Float16* xop, uint8_t* xs, hipStream_t st);
 hipError_t launch_mmqk(int dtype, const MmqArgs& a, int splits, hipStream_t st);
 // Q6_K: the kernel reads 36-byte blocks that launch_q6c writes from the GGUF
 // rows (mmqp_q6c_bytes(N, K) bytes, 16-byte aligned)

@@ -11,7 +11,15 @@
 //         MFMAs per 32 x 32 tile) + c sum over its sub-blocks of S sc, S the
 //         token's sub-block sums as fp16 hi + lo (one MFMA: 16 slots)
 //   Dm  = sum over its sub-blocks of S m                       (one MFMA)
-//   acc += d D - dmin Dm                             (two FMAs per output)
+//   acc += 2^e (d D - dmin Dm)                       (three per output)
+//
+// with x 2^-e as x_hi + x_lo, e the token's exponent.  S's low part is kept 2^12
+// larger and meets weights 2^12 smaller, exact in fp16: it keeps its bits down to
+// 2^-29 of the token's largest, where fp16's least value alone ends at 2^-17.
+// Q5_K (FINE), whose tokens had an exponent per 64 elements in the fp16 MFMA
+// kernel, has one per super-block, and x_lo kept in the same way (xprepk_kernel;
+// its fold, acc += 2^e (..), costs 2 to 3 %: Q4_K 3584 -> 18944 pair, M = 1999,
+// 1125 -> 1157 us).
 //
 // (codes about zero keep the chain's partial sums small: with q as it stands
 // the result's error against 64 bits was 40 % larger, 3.2e-7 at K = 4096)
@@ -52,7 +60,72 @@ constexpr int KS = 64;               // K elements per step: one sub-block pair
 constexpr int XT = 1024;             // halves per (32-token tile, 16-k quarter): hi then lo
 constexpr int NBUF = 3;              // buffers of a step's operands: steps s, s + 1, s + 2
 constexpr int NW = 8;                // waves per work-group
-constexpr int STILE = 1024;          // bytes of a tile's sub-block sums: [hi, lo][token][sub-block]
+constexpr int SEXP = 1024;           // bytes of a tile's sub-block sums: [hi, lo][token][sub-block]
+constexpr int STILE_FINE = SEXP + 128;  // and 2^e of its tokens
+constexpr float LO = 0x1p12f;        // what the kept low parts are larger by
+
+// ------------------------------------------------------------- token prep
+// FINE: the A operand as xprep4_kernel lays it out, an exponent per token and
+// super-block.  A work-group is a tile and super-block, a wave four of
+// its tokens: lane t + 4 j has pieces (2 kq + g = j and j + 16) of token t, so that
+// four lanes write one 64-byte run and the exponent and the sums need no barrier.
+__global__ __launch_bounds__(512) void xprepk_kernel(const float* __restrict__ x, int M, int K,
+                                                     _Float16* __restrict__ xop,
+                                                     uint8_t* __restrict__ xs) {
+    const int lane = threadIdx.x & 63, t = lane & 3, j = lane >> 2;
+    const int sb = blockIdx.x, T = blockIdx.y, lm = 4 * (threadIdx.x >> 6) + t, m = 32 * T + lm;
+    float v[2][8] = {};
+    float mx = 0.0f;
+    if (m < M) {
+        const float* const xr = x + (size_t)m * K + 256 * sb;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int gq = j + 16 * i;
+            const float* s = xr + 32 * (gq >> 2) + 16 * (gq & 1) + 8 * ((gq >> 1) & 1);
+            const float4 a = *reinterpret_cast<const float4*>(s), b = *reinterpret_cast<const float4*>(s + 4);
+            const float u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                v[i][k] = u[k];
+                mx = fmaxf(mx, fabsf(u[k]));
+            }
+        }
+    }
+#pragma unroll
+    for (int o = 4; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    // (2^e a normal number)
+    const int e = (mx > 0.0f && mx <= 3.0e38f) ? max(ilogbf(mx) - 14, -126) : 0;
+    uint8_t* const sbk = xs + ((size_t)T * (K / 256) + sb) * STILE_FINE;
+    if (j == 0) *reinterpret_cast<float*>(sbk + SEXP + 4 * lm) = __builtin_amdgcn_ldexpf(1.0f, e);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int gq = j + 16 * i;
+        float w[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) w[k] = __builtin_amdgcn_ldexpf(v[i][k], -e);
+        h8 hi, lo;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float u = w[slot_elem(k)];
+            hi[k] = (_Float16)u;
+            lo[k] = (_Float16)((u - (float)hi[k]) * LO);
+        }
+        _Float16* const dst = xop + ((size_t)T * (K / 16) + 16 * sb + (gq >> 1)) * XT + (lm + 32 * (gq & 1)) * 8;
+        *reinterpret_cast<h8*>(dst) = hi;
+        *reinterpret_cast<h8*>(dst + 512) = lo;
+        // the sum over sub-block gq / 4: four pieces, times 2^-5 (below 2^15)
+        float s = ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+        s += __shfl_xor(s, 4, 64);
+        s += __shfl_xor(s, 8, 64);
+        if ((gq & 3) == 0) {
+            s *= 0x1p-5f;
+            const _Float16 h = (_Float16)s;
+            _Float16* const d = reinterpret_cast<_Float16*>(sbk) + lm * 8 + (gq >> 2);
+            d[0] = h;
+            d[256] = (_Float16)((s - (float)h) * LO);
+        }
+    }
+}
 
 // Super-block layout: header (d dmin scales[12]) @0, Q5_K: qh[32] @16, then
 // qs[128].  The header and qh are copied once per super-block as HP planes of
@@ -64,6 +137,8 @@ struct KQ {
     static constexpr int QOFF = 16 * HP;
     static constexpr float UNIT = F == Q5_K ? 8.0f : 16.0f;  // value of a code step in the half
     static constexpr float MID = F == Q5_K ? 16.0f : 8.0f;   // c
+    static constexpr bool FINE = F == Q5_K;
+    static constexpr int STILE = FINE ? STILE_FINE : SEXP;
     // LDS: token operands, code planes (NBUF each), super-block planes, sums (2 each)
     static constexpr int XBUF = 16 * XT * 2;
     static constexpr int QBUF = 2 * BNT * 16;
@@ -110,7 +185,7 @@ __device__ __forceinline__ fq_u32x4 lds16(const uint8_t* p) {
 // A work-group owns 128 tokens x 256 rows and a K range of whole super-blocks
 // (split-K when that shortens the busiest CU's work).  Eight waves, each 64
 // tokens x 64 rows (2 x 2 tiles of 32 x 32), tokens as the A operand
-// (xprep4_kernel: x 2^-e(token) as fp16 hi + lo), weights as B, so that a
+// (xprep4_kernel, xprepk_kernel), weights as B, so that a
 // lane's 16 results of a tile belong to one row and d, dmin are one value per
 // lane.  All operands reach LDS by direct copies, three buffers deep for a
 // step's, two for a super-block's; one barrier per step publishes step s and
@@ -118,6 +193,7 @@ __device__ __forceinline__ fq_u32x4 lds16(const uint8_t* p) {
 template <int F, bool PAIR>
 __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_split) {
     using Q = KQ<F>;
+    constexpr int STILE = Q::STILE;
     constexpr int RJ = PAIR ? BNT / 2 : 32;  // tile rows between a wave's two row tiles
     __shared__ __attribute__((aligned(16))) uint8_t lds[Q::LDS];
     uint8_t* const xs0 = lds;
@@ -220,7 +296,7 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
         }
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            h8 B[2][2];
+            h8 B[2][2], Bl[2][2];  // Bl: for x_lo
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const float sf = (float)sub_scale(hdr[j], 2 * U + b);
@@ -239,6 +315,8 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
                 }
                 B[j][0] = scaled8(w[0], w[1], sc, off);
                 B[j][1] = scaled8(w[2], w[3], sc, off);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) Bl[j][h] = Q::FINE ? B[j][h] * (_Float16)(1.0f / LO) : B[j][h];
             }
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
@@ -252,18 +330,20 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
                         cur[0], B[j][0], U == 0 && b == 0 ? z : D[i][j], 0, 0, 0);
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur[1], B[j][0], D[i][j], 0, 0, 0);
+                    D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur[1], Bl[j][0], D[i][j], 0, 0, 0);
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
                     D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur[2], B[j][1], D[i][j], 0, 0, 0);
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur[3], B[j][1], D[i][j], 0, 0, 0);
+                    D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur[3], Bl[j][1], D[i][j], 0, 0, 0);
             }
         }
         if constexpr (U == 3) {
-            // the super-block's fold: acc += d D - dmin Dm.  Sums operand:
-            // lane (c, g) the hi (g = 0) or lo parts of token c, times 2^-5
+            // the super-block's fold: acc += d D - dmin Dm (FINE: times 2^e).
+            // Sums operand: lane (c, g) the hi (g = 0) or lo parts of token c,
+            // times 2^-5 (lo: times LO)
+            const float gs = g ? 1.0f / LO : 1.0f;
             h8 Mb[2], Sb[2];
             float d[2], dn[2];
 #pragma unroll
@@ -271,8 +351,8 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
                 h8 m, sc;
 #pragma unroll
                 for (int b = 0; b < 8; ++b) {
-                    m[b] = (_Float16)(float)sub_min(hdr[j], b);
-                    sc[b] = (_Float16)((float)sub_scale(hdr[j], b) * (32.0f * Q::MID));
+                    m[b] = (_Float16)((float)sub_min(hdr[j], b) * gs);
+                    sc[b] = (_Float16)((float)sub_scale(hdr[j], b) * (gs * 32.0f * Q::MID));
                 }
                 Mb[j] = m;
                 Sb[j] = sc;
@@ -291,15 +371,25 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
                 for (int j = 0; j < 2; ++j)
                     dm[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(S, Mb[j], z, 0, 0, 0);
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int e4 = 0; e4 < 4; ++e4) {  // the lane's tokens 8 e4 + 4 g ..
+                    float4 f4 = {};
+                    if constexpr (Q::FINE)
+                        f4 = *reinterpret_cast<const float4*>(ss + (2 * wm + i) * STILE + SEXP + 32 * e4 + 16 * g);
+                    const float f[4] = {f4.x, f4.y, f4.z, f4.w};
 #pragma unroll
-                    for (int e = 0; e < 16; ++e)
-                        acc[i][j][e] = __builtin_fmaf(d[j], D[i][j][e], acc[i][j][e]);
+                    for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e)
-                        acc[i][j][e] = __builtin_fmaf(dn[j], dm[j][e], acc[i][j][e]);
+                        for (int k = 0; k < 4; ++k) {
+                            const int e = 4 * e4 + k;
+                            if constexpr (Q::FINE) {
+                                const float v = __builtin_fmaf(d[j], D[i][j][e], dn[j] * dm[j][e]);
+                                acc[i][j][e] = __builtin_fmaf(v, f[k], acc[i][j][e]);
+                            } else {
+                                acc[i][j][e] = __builtin_fmaf(d[j], D[i][j][e], acc[i][j][e]);
+                                acc[i][j][e] = __builtin_fmaf(dn[j], dm[j][e], acc[i][j][e]);
+                            }
+                        }
+                }
             }
         }
     };
@@ -338,7 +428,7 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
     else loop(std::integral_constant<int, 0>{});
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-        store_tiles<PAIR>(a, rt, m0 + 64 * wm + 32 * i, rt.n0 + (PAIR ? 32 : 64) * wn + c, g, acc[i],
+        store_tiles<PAIR, !Q::FINE>(a, rt, m0 + 64 * wm + 32 * i, rt.n0 + (PAIR ? 32 : 64) * wn + c, g, acc[i],
                           gridDim.z > 1, blockIdx.z);
 }
 
@@ -346,8 +436,18 @@ __global__ __launch_bounds__(512) void mmqk_kernel(MmqArgs a, int steps_per_spli
 
 bool mmqk_supported(int dtype) { return dtype == Q4_K || dtype == Q5_K; }
 
+bool mmqk_fine(int dtype) { return dtype == Q5_K; }
+
 // Bytes of the sub-block sums of one 32-token tile
-size_t mmqk_sum_bytes(int K) { return (size_t)(K / 256) * STILE; }
+size_t mmqk_sum_bytes(int dtype, int K) {
+    return (size_t)(K / 256) * (mmqk_fine(dtype) ? KQ<Q5_K>::STILE : KQ<Q4_K>::STILE);
+}
+
+hipError_t launch_xprepk(const float* x, int M, int K, _Float16* xop, uint8_t* xs, hipStream_t st) {
+    if (K % 256 != 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(xprepk_kernel, dim3(K / 256, (M + 31) / 32), dim3(512), 0, st, x, M, K, xop, xs);
+    return hipGetLastError();
+}
 
 hipError_t launch_mmqk(int dtype, const MmqArgs& a, int splits, hipStream_t st) {
     const int nsteps = a.K / KS;

@@ -139,13 +139,13 @@ __global__ __launch_bounds__(1024) void xprep4_kernel(const float* __restrict__ 
                 const int b = kq >> 1;  // sub-block
                 if (xsum) xsum[((size_t)T * (K / 32) + b) * 32 + lm] = t8;
                 if (xsum2) {
-                    // times 2^-5 (below 2^15) as fp16 hi + lo:
+                    // times 2^-5 (below 2^15) as fp16 hi + lo, lo 2^12 larger:
                     // [super-block][hi, lo][token][sub-block of the super-block]
                     const float v = t8 * 0x1p-5f;
                     const _Float16 vh = (_Float16)v;
                     _Float16* d = xsum2 + ((size_t)T * (K / 256) + (b >> 3)) * 512 + lm * 8 + (b & 7);
                     d[0] = vh;
-                    d[256] = (_Float16)(v - (float)vh);
+                    d[256] = (_Float16)((v - (float)vh) * 0x1p12f);
                 }
             }
         }
@@ -660,7 +660,7 @@ __global__ __launch_bounds__(512) void mmqp_kernel(MmqArgs a, int steps_per_spli
     else loop(std::integral_constant<int, 0>{});
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-        store_tiles<PAIR>(a, rt, m0 + 64 * wm + 32 * i, rt.n0 + (PAIR ? 32 : 64) * wn + c, g, acc[i],
+        store_tiles<PAIR, true>(a, rt, m0 + 64 * wm + 32 * i, rt.n0 + (PAIR ? 32 : 64) * wn + c, g, acc[i],
                           gridDim.z > 1, blockIdx.z);
 }
 

@@ -46,15 +46,15 @@ __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f +
 // The results of a wave's two row tiles (acc[.][0], acc[.][1]) of 32 x 32
 // tokens x rows: lane (c, g) holds column c of each, tokens 8 (e / 4) + 4 g +
 // e % 4.  n: the lane's row of tile j = 0 within its matrix (PAIR: of both);
-// split: the partial slab of split z.
-template <bool PAIR, class V>
+// split: the partial slab of split z.  EX: times 2^a.ex[token].
+template <bool PAIR, bool EX, class V>
 __device__ __forceinline__ void store_tiles(const MmqArgs& a, const RowTile& rt, int m, int n, int g,
                                             const V (&acc)[2], bool split, int z) {
     const int cols = PAIR ? 2 * a.N : a.N;
     float* const slab = split ? a.part + (size_t)z * a.M * cols : a.y;
     int ei[16];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) ei[e] = a.ex[min(m + 8 * (e >> 2) + 4 * g + (e & 3), a.M - 1)];
+    for (int e = 0; e < 16; ++e) ei[e] = !EX ? 0 : a.ex[min(m + 8 * (e >> 2) + 4 * g + (e & 3), a.M - 1)];
     if constexpr (PAIR) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {

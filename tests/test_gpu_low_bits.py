@@ -61,19 +61,35 @@ def test_product_of_the_low_parts():
 
 # an element of 2^27 times the others in every super-block, in the 64 elements
 # whose weights are zero: the others' bits are theirs
-@pytest.mark.parametrize("dtype", ALL)
-def test_small_elements_beside_large_ones(dtype):
-    N, K, M = 130, 1024, 20
+@pytest.mark.parametrize("dtype,M", [(d, 20) for d in ALL] + [(F.Q5_K, 40)])
+def test_small_elements_beside_large_ones(dtype, M):
+    N, K = 130, 1024
     w = zero_first_64(dtype, synth.make_weights(dtype, N, K, seed=3), N)
     x = synth.make_x(M, K, seed=4)
     x[:, 5::256] = np.float32(2.0 ** 27)
     assert rel(dtype, w, x, N, K) <= 1e-6
 
 
+# such an element in a super-block of zero weights, minima of zero: the sums that
+# centre the codes keep the bits of the other super-blocks.  Q4_K prefill has one
+# exponent per token: its elements keep 2^-39 of the largest, 2^-39 2^19 of the
+# others, 1e-6 of the result at most; sums in fp16 hi + lo kept 2^-34
+@pytest.mark.parametrize("dtype,log2", [(F.Q4_K, 19), (F.Q5_K, 20), (F.Q5_K, 60)])
+def test_small_super_blocks_beside_large_ones(dtype, log2):
+    N, K, M = 130, 1024, 40
+    w = synth.make_weights(dtype, N, K, seed=7).reshape(N, -1, F.fmt(dtype).block_bytes)
+    w[:, 1, 0:2] = 0  # d
+    w[:, :, 2:4] = 0  # dmin
+    x = synth.make_x(M, K, seed=8)
+    x[:, 256 + 77] = np.float32(2.0 ** log2)
+    assert rel(dtype, w.reshape(N, -1), x, N, K) <= 1e-6
+
+
 # tokens of subnormal numbers against weights large enough for normal results
+@pytest.mark.parametrize("M", [20, 40])
 @pytest.mark.parametrize("dtype", KQ)
-def test_subnormal_tokens(dtype):
-    N, K, M = 70, 512, 20
+def test_subnormal_tokens(dtype, M):
+    N, K = 70, 512
     f = F.fmt(dtype)
     w = synth.make_weights(dtype, N, K, seed=5).reshape(N, -1, f.block_bytes)
     at = 208 if dtype == F.Q6_K else 0
