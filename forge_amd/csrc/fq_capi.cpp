@@ -210,6 +210,9 @@ size_t mmqs_need(int M, int K, int N, int cus, int mt) {
     return 256 + al(pl.xop_b) + al(pl.xsum_b) + al(pl.ex_b) + al(part_b);
 }
 
+// Bytes of the fixed workspace of fq_matmul_transB_noalloc.
+constexpr size_t kNoAllocBytes = (size_t)64 << 20;
+
 // Workspace bytes and K-splits of the prefill kernels (M > 32, K a multiple
 // of 256): one work-group per CU and tile, each split a multiple of four
 // 64-element steps.
@@ -218,22 +221,39 @@ struct MmqpPlan {
     size_t xop_b, ex_b, sum_b, part_b, q6c_b, total;
 };
 
-// tiles_n: work-groups along the rows, cols: columns of a partial slab,
-// q6_rows: Q6_K rows to rewrite (0: another format); cap: bytes the plan has
-// to fit where a smaller split count can (0: no limit).
-MmqpPlan plan_mmqp(uint32_t dtype, int M, int K, long tiles_n, int cols, int q6_rows, int cus,
-                   size_t cap = 0) {
+// Of `splits` slabs; cols: columns of a partial slab, q6_rows: Q6_K rows to
+// rewrite (0: another format).
+MmqpPlan mmqp_sizes(uint32_t dtype, int M, int K, int cols, int q6_rows, int splits) {
     MmqpPlan p{};
-    const int Tn = (M + 31) / 32, nsteps = K / 64;
-    const int tm = fq::mmqp_tile_tokens();
-    const long tiles = tiles_n * ((M + tm - 1) / tm);
+    const int Tn = (M + 31) / 32;
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    p.splits = splits;
     p.xop_b = (size_t)Tn * K * 64 * 2;
     p.ex_b = (size_t)M * 4;
     // sub-block sums (formats with a min term): floats, or mmqk's hi + lo
     p.sum_b = (size_t)Tn * (fq::mmqk_supported((int)dtype) ? fq::mmqk_sum_bytes((int)dtype, K) : (size_t)K * 4);
     p.q6c_b = (size_t)fq::mmqp_q6c_bytes(q6_rows, K);  // Q6_K rows as 36-byte blocks
-    const size_t fixed_b = 256 + al(p.xop_b) + al(p.ex_b) + al(p.sum_b) + al(p.q6c_b);
+    p.part_b = splits > 1 ? (size_t)splits * M * cols * 4 : 0;
+    p.total = 256 + al(p.xop_b) + al(p.ex_b) + al(p.sum_b) + al(p.q6c_b) + al(p.part_b);
+    return p;
+}
+
+// The fewest tokens the prefill kernels can run at a time with the bits of the
+// whole call: with a minimum per block (fq_mmqp.hip), a token's additions come in
+// an order that depends on which 32 of a wave's 64 tokens it is in, and whether
+// both hold tokens.
+int prefill_granule(uint32_t dtype) { return dtype == FQ_DTYPE_Q4_1 || dtype == FQ_DTYPE_Q5_1 ? 64 : 1; }
+
+// tiles_n: work-groups along the rows.  one: a single matrix, whose plan
+// fq_matmul_transB_noalloc runs in a fixed array, fewer tokens at a time if
+// need be (run_prefill): so the slabs of the fewest have to fit there where the
+// operands of all do.
+MmqpPlan plan_mmqp(uint32_t dtype, int M, int K, long tiles_n, int cols, int q6_rows, bool one, int cus) {
+    const int nsteps = K / 64;
+    const int tm = fq::mmqp_tile_tokens();
+    const long tiles = tiles_n * ((M + tm - 1) / tm);
+    MmqpPlan p = mmqp_sizes(dtype, M, K, cols, q6_rows, 1);
+    const bool fits = p.total <= kNoAllocBytes || dtype == FQ_DTYPE_Q5_K;
     // The split count of the smallest estimated time: rounds of work-groups x
     // (steps per split at 2.1 us, 3 us to fill the pipeline and store), and
     // for a split the slab sum, a launch of 4 us and each slab written and
@@ -241,23 +261,21 @@ MmqpPlan plan_mmqp(uint32_t dtype, int M, int K, long tiles_n, int cols, int q6_
     // gate/up pair at K = 4096, M = 77: 117 + 23 us against 80 + 7 with 2, and
     // 8 for a 6144-row QKV at M = 512: 82 + 19 us against 72 + 8.)
     double best = 0.0;
-    p.splits = 1;
     for (int sp = 1; sp <= std::max(1, std::min(16, nsteps / 4)); ++sp) {
         const int sps = ((nsteps + sp - 1) / sp + 3) & ~3;
         const int eff = (nsteps + sps - 1) / sps;  // non-empty splits
         if (eff != sp) continue;
-        const size_t part_b = sp > 1 ? (size_t)sp * M * cols * 4 : 0;
-        if (sp > 1 && cap && fixed_b + al(part_b) > cap) continue;
+        if (sp > 1 && one && fits &&
+            mmqp_sizes(dtype, std::min(M, prefill_granule(dtype)), K, cols, q6_rows, sp).total > kNoAllocBytes)
+            continue;
         const double t = (double)((tiles * sp + cus - 1) / cus) * (2.1 * sps + 3.0) +
                          (sp > 1 ? 4.0 + ((double)sp + 1.0) * M * cols * 4.0 / 4e6 : 0.0);
         if (sp == 1 || t < best) {
             best = t;
             p.splits = sp;
-            p.part_b = part_b;
         }
     }
-    p.total = fixed_b + al(p.part_b);
-    return p;
+    return mmqp_sizes(dtype, M, K, cols, q6_rows, p.splits);
 }
 
 // M > 1 on the matrix cores: token operand preparation, then one tile per
@@ -346,30 +364,39 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
     a.n2 = ms.n[1];
     a.n3 = ms.n[2];
     a.row_bytes = (K / g.be) * g.bb;
-    a.M = M;
     a.N = N;
     a.K = K;
-    const MmqpPlan pl = plan_mmqp(dtype, M, K, fq::mmqp_row_tiles(a), fq::mm_cols(a), q6k ? rows : 0,
-                                  di.cus, fixed_cap);
+    const int cols = fq::mm_cols(a), q6_rows = q6k ? rows : 0;
+    MmqpPlan pl = plan_mmqp(dtype, M, K, fq::mmqp_row_tiles(a), cols, q6_rows, ms.mm == fq::MM_ONE, di.cus);
     const int splits = pl.splits;
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    const size_t xop_b = pl.xop_b, ex_b = pl.ex_b, sum_b = pl.sum_b, need = pl.total;
     std::unique_ptr<StreamScratch::Lease> lease;
     uint8_t* buf = fixed;
+    int mc = M;  // tokens at a time
     if (fixed) {
-        // (Q5_K in a fixed workspace that its K-splits here do not fit, 2040 x
-        // 256 x 4096 for instance, runs on the fp16 MFMA kernel, whose plan
-        // may)
-        if (need > fixed_cap) return dtype == FQ_DTYPE_Q5_K ? kNotTaken : FQ_ERR_WORKSPACE;
+        // The operands of all tokens have to fit (Q5_K: those of the fp16 MFMA
+        // kernel may, which differ by a few per cent for rows of 46 thousand
+        // elements); where the slabs beside them do not, the same launches run
+        // for as many tokens as do: a token's sums do not depend on the others,
+        // so the bits are those of the call on a stream's workspace (642 x 18944
+        // x 14336: four splits, 194 MB of slabs).
+        if (mmqp_sizes(dtype, M, K, cols, q6_rows, 1).total > fixed_cap &&
+            !(dtype == FQ_DTYPE_Q5_K && plan_mmq(M, K, N, di.cus).total <= fixed_cap))
+            return FQ_ERR_WORKSPACE;
+        while (pl.total > fixed_cap && mc > prefill_granule(dtype)) {
+            mc = mc > 64 ? (mc - 1) / 64 * 64 : mc / 2;
+            pl = mmqp_sizes(dtype, mc, K, cols, q6_rows, splits);
+        }
+        if (pl.total > fixed_cap) return FQ_ERR_WORKSPACE;
     } else {
         lease.reset(new StreamScratch::Lease(stream_scratch(dev, st, 0)));
-        const int rc = lease->get(need, st, &buf);
+        const int rc = lease->get(pl.total, st, &buf);
         if (rc == FQ_ERR_WORKSPACE && ms.mm != fq::MM_ONE) return kNotTaken;
         if (rc != FQ_OK) return rc;
     }
     hipError_t e = hipSuccess;
     if (q6k) {
-        uint8_t* conv = buf + al(xop_b) + al(ex_b) + al(sum_b) + al(pl.part_b);
+        uint8_t* conv = buf + al(pl.xop_b) + al(pl.ex_b) + al(pl.sum_b) + al(pl.part_b);
         const uint8_t** w[3] = {&a.w, &a.w2, &a.w3};
         for (int i = 0; i < 3; ++i) {
             const int n = ms.mm == fq::MM_PAIR && i < 2 ? ms.n[0] : ms.n[i];
@@ -381,28 +408,34 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
         }
         a.row_bytes = (int)rb;
     }
+    _Float16* const xop = reinterpret_cast<_Float16*>(buf);
+    int* const ex = reinterpret_cast<int*>(buf + al(pl.xop_b));
+    uint8_t* const sums = mmqk || dtype == FQ_DTYPE_Q4_1 || dtype == FQ_DTYPE_Q5_1
+                              ? buf + al(pl.xop_b) + al(pl.ex_b)
+                              : nullptr;
     a.xop = buf;
-    a.ex = reinterpret_cast<const int*>(buf + al(xop_b));
-    float* const sums = mmqk || dtype == FQ_DTYPE_Q4_1 || dtype == FQ_DTYPE_Q5_1
-                            ? reinterpret_cast<float*>(buf + al(xop_b) + al(ex_b))
-                            : nullptr;
-    a.xsum = sums;
-    a.part = splits > 1 ? reinterpret_cast<float*>(buf + al(xop_b) + al(ex_b) + al(sum_b))
+    a.ex = ex;
+    a.xsum = reinterpret_cast<const float*>(sums);
+    a.part = splits > 1 ? reinterpret_cast<float*>(buf + al(pl.xop_b) + al(pl.ex_b) + al(pl.sum_b))
                         : nullptr;
-    a.y = y;
-    a.bias = bias;
     a.bias_len = bias_mode ? bias_len : 0;
     a.bias_mode = bias_mode;
-    if (fq::mmqk_fine((int)dtype))
-        e = fq::launch_xprepk(x, M, K, reinterpret_cast<_Float16*>(buf), reinterpret_cast<uint8_t*>(sums), st);
-    else
-        e = fq::launch_xprep32(x, M, K, reinterpret_cast<_Float16*>(buf), const_cast<int*>(a.ex),
-                               mmqk ? nullptr : sums,
-                               mmqk ? reinterpret_cast<_Float16*>(sums) : nullptr, q6k, st);
-    if (e != hipSuccess) return hip_fail(e);
-    e = mmqk ? fq::launch_mmqk((int)dtype, a, splits, st) : fq::launch_mmqp((int)dtype, a, splits, st);
-    if (e == hipSuccess && splits > 1) e = fq::launch_reduce(a, splits, st);
-    return e == hipSuccess ? FQ_OK : hip_fail(e);
+    for (int t0 = 0; t0 < M; t0 += mc) {
+        const float* const xt = x + (size_t)t0 * K;
+        a.M = std::min(mc, M - t0);
+        a.y = y + (size_t)t0 * N;
+        a.bias = bias_mode == 2 ? bias + (size_t)t0 * N : bias;
+        if (fq::mmqk_fine((int)dtype))
+            e = fq::launch_xprepk(xt, a.M, K, xop, sums, st);
+        else
+            e = fq::launch_xprep32(xt, a.M, K, xop, ex, mmqk ? nullptr : reinterpret_cast<float*>(sums),
+                                   mmqk ? reinterpret_cast<_Float16*>(sums) : nullptr, q6k, st);
+        if (e != hipSuccess) return hip_fail(e);
+        e = mmqk ? fq::launch_mmqk((int)dtype, a, splits, st) : fq::launch_mmqp((int)dtype, a, splits, st);
+        if (e == hipSuccess && splits > 1) e = fq::launch_reduce(a, splits, st);
+        if (e != hipSuccess) return hip_fail(e);
+    }
+    return FQ_OK;
 }
 
 // Small batches with the token operands shared by the rows of a work-group
@@ -420,9 +453,16 @@ struct MmqtPlan {
 // read at 4 TB/s).  A step's time is what 14336 x 4096 measured on 224
 // work-groups, or its weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x
 // 3584 at M = 16: 134 us on 128 rows, 156 on 64).
+//
+// No plan takes more than the fixed array of fq_matmul_transB_noalloc, so that
+// the plan is the same there.
 MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
     const bool q6 = dtype == FQ_DTYPE_Q6_K, wide = a.M > 16;
     MmqtPlan p{};
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    p.xop_b = fq::mmqt_xop_bytes(a.M, a.K);
+    p.sum_b = fq::mmqt_sum_bytes(a.M, a.K);
+    const size_t ops_b = 256 + al(p.xop_b) + al(p.sum_b);
     const double sb_bytes = (double)a.row_bytes / (a.K / 256);
     double best = 0.0;
     for (int rows : {256, 128, 64}) {
@@ -438,7 +478,8 @@ MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
         for (int per = (int)((total + cus - 1) / cus);; per *= 2) {
             per = std::min(per, whole);
             const int parts = fq::mmqt_parts(nst, per);
-            if (parts <= 16) {
+            const size_t part_b = parts > 1 ? (size_t)parts * a.M * fq::mm_cols(a) * 4 : 0;
+            if (parts <= 16 && ops_b + al(part_b) <= kNoAllocBytes) {
                 const double busy = (double)((total + per - 1) / per);
                 const double step = std::max(it, busy * kg * rows * sb_bytes / 5e6);
                 const double t = 1.5 + step * per + (double)((per + nst - 1) / nst) +
@@ -448,17 +489,13 @@ MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
                     p.rows = rows;
                     p.per = per;
                     p.parts = parts;
+                    p.part_b = part_b;
                 }
             }
             if (per == whole) break;
         }
     }
-    if (p.rows == 0) return p;
-    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    p.xop_b = fq::mmqt_xop_bytes(a.M, a.K);
-    p.sum_b = fq::mmqt_sum_bytes(a.M, a.K);
-    p.part_b = p.parts > 1 ? (size_t)p.parts * a.M * fq::mm_cols(a) * 4 : 0;
-    p.total = 256 + al(p.xop_b) + al(p.sum_b) + al(p.part_b);
+    p.total = ops_b + al(p.part_b);
     return p;
 }
 
@@ -492,8 +529,8 @@ bool thin_takes_pair(uint32_t dtype, int M, int64_t bytes) {
     return M <= 4 || thin_takes(dtype, M, bytes);
 }
 
-// kNotTaken: another kernel runs the call (also where the workspace cannot
-// hold this one's operands: capture, the fixed array).
+// kNotTaken: another kernel runs the call (also where the workspace cannot grow
+// to this one's operands under capture).
 int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, const float* bias,
              int bias_mode, int64_t bias_len, float* y, int M, int K, int N, int dev,
              const DevInfo& di, hipStream_t st, uint8_t* fixed, size_t fixed_cap) {
@@ -525,7 +562,7 @@ int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, 
     std::unique_ptr<StreamScratch::Lease> lease;
     uint8_t* buf = fixed;
     if (fixed) {
-        if (pl.total > fixed_cap) return kNotTaken;
+        if (pl.total > fixed_cap) return FQ_ERR_WORKSPACE;
     } else {
         lease.reset(new StreamScratch::Lease(stream_scratch(dev, st, 0)));
         const int rc = lease->get(pl.total, st, &buf);
@@ -727,7 +764,6 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
 // shared by every call of that entry point on the device: calls that overlap
 // on one GPU race on it.  Nothing in it has to start at zero (the token
 // preparation writes every operand, each K-split writes its whole slab).
-constexpr size_t kNoAllocBytes = (size_t)64 << 20;
 __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
 
 // The device address of `scratch` on the current device, looked up once per
@@ -1569,8 +1605,8 @@ int fq_reserve_workspace(int M_max, int K_max, int N_max, void* stream) {
             if (m > 32 && Kp > 0) {  // one matrix, and a gate/up pair
                 const int tn = fq::mmqp_tile_rows();
                 // (with the larger sums of Q5_K and the rewritten rows of Q6_K)
-                need0 = std::max(need0, plan_mmqp(FQ_DTYPE_Q5_K, m, Kp, (n + tn - 1) / tn, n, n, di.cus).total);
-                need0 = std::max(need0, plan_mmqp(FQ_DTYPE_Q5_K, m, Kp, (2L * n + tn - 1) / tn, 2 * n, 2 * n, di.cus).total);
+                need0 = std::max(need0, plan_mmqp(FQ_DTYPE_Q5_K, m, Kp, (n + tn - 1) / tn, n, n, true, di.cus).total);
+                need0 = std::max(need0, plan_mmqp(FQ_DTYPE_Q5_K, m, Kp, (2L * n + tn - 1) / tn, 2 * n, 2 * n, false, di.cus).total);
             }
             if (m <= 32 && Kp > 0) {  // one matrix, and a gate/up pair
                 fq::MmqArgs t{};

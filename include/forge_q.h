@@ -220,7 +220,9 @@ int fq_ffn_down_residual_packed(uint32_t dtype, const float* x, const void* w_pa
  * capture, serving loops and harnesses that forbid hipMalloc).  Returns
  * FQ_ERR_WORKSPACE when a call needs more than 64 MiB (for example M = 512 at
  * K = N = 4096 needs 40-42 MiB with 4 K-splits, 58 MiB for Q6_K, whose
- * rewritten rows take N * K * 9 / 8 bytes more).  All calls on one GPU
+ * rewritten rows take N * K * 9 / 8 bytes more).  A prefill call whose K-splits'
+ * slabs alone go beyond it runs fewer tokens at a time, with the same splits and
+ * so the same bits.  All calls on one GPU
  * share the array: calls that overlap on one GPU (several streams or host
  * threads) race on it and must be serialised by the caller. */
 int fq_matmul_transB_noalloc(uint32_t dtype, const float* x, const void* w, const float* bias,

@@ -67,3 +67,13 @@ def test_noalloc_prefill_and_limit():
     x = torch.zeros(M, K, device="cuda")
     y = torch.zeros(M, N, device="cuda")
     assert _call(L.fq_matmul_transB_noalloc, F.Q8_0, x, w, y, M, K, N) == _lib.FQ_ERR_WORKSPACE
+
+
+# plans that need more than the array (K-splits of the prefill kernels, whose
+# slabs are then those of fewer tokens at a time, with a bias per element and
+# with a ragged last pass; tiles in parts of the small-batch kernel)
+@pytest.mark.parametrize("dtype,M,K,N", [(F.Q5_K, 2040, 4096, 256), (F.Q4_K, 512, 18944, 1024),
+                                         (F.Q8_0, 1024, 14336, 1024), (F.Q6_K, 391, 18944, 1000),
+                                         (F.Q4_1, 650, 14336, 2600), (F.Q4_0, 32, 3584, 262145)])
+def test_noalloc_plans_beyond_the_array(dtype, M, K, N):
+    _pair(dtype, M, K, N, 100, bias=M in (391, 650))
