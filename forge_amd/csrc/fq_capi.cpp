@@ -244,6 +244,27 @@ MmqpPlan mmqp_sizes(uint32_t dtype, int M, int K, int cols, int q6_rows, int spl
 // both hold tokens.
 int prefill_granule(uint32_t dtype) { return dtype == FQ_DTYPE_Q4_1 || dtype == FQ_DTYPE_Q5_1 ? 64 : 1; }
 
+// Slabs of one prefill call at most (they only even out the rounds of
+// work-groups: of 2 million sizes up to 4096 x 160000 x 20480 under 1 % would
+// take more, 9 % faster at best by the estimate below), and rewritten Q6_K rows
+// of several matrices in one launch (gate and up of 18944 x 3584: 146 MiB): what
+// fq_reserve_workspace has to set aside.
+constexpr size_t kMaxSlabs = (size_t)256 << 20, kMaxRewrite = (size_t)160 << 20;
+
+// Estimated time of a prefill launch over K in sp splits (0: some would be
+// empty): rounds of work-groups x (steps per split at 2.1 us, 3 us to fill the
+// pipeline and store), and for a split the launch of the slab sum.  Beside it each
+// slab element is written and read once at 4 TB/s, kSlabUs per element and slab.
+// (Counting steps alone took 16 splits for a 14336-row gate/up pair at K = 4096,
+// M = 77: 117 + 23 us against 80 + 7 with 2, and 8 for a 6144-row QKV at M = 512:
+// 82 + 19 us against 72 + 8.)
+constexpr double kSlabUs = 4.0 / 4e6;
+double mmqp_us(long tiles, int nsteps, int sp, int cus) {
+    const int sps = ((nsteps + sp - 1) / sp + 3) & ~3;
+    if ((nsteps + sps - 1) / sps != sp) return 0.0;
+    return (double)((tiles * sp + cus - 1) / cus) * (2.1 * sps + 3.0) + (sp > 1 ? 4.0 : 0.0);
+}
+
 // tiles_n: work-groups along the rows.  one: a single matrix, whose plan
 // fq_matmul_transB_noalloc runs in a fixed array, fewer tokens at a time if
 // need be (run_prefill): so the slabs of the fewest have to fit there where the
@@ -254,28 +275,49 @@ MmqpPlan plan_mmqp(uint32_t dtype, int M, int K, long tiles_n, int cols, int q6_
     const long tiles = tiles_n * ((M + tm - 1) / tm);
     MmqpPlan p = mmqp_sizes(dtype, M, K, cols, q6_rows, 1);
     const bool fits = p.total <= kNoAllocBytes || dtype == FQ_DTYPE_Q5_K;
-    // The split count of the smallest estimated time: rounds of work-groups x
-    // (steps per split at 2.1 us, 3 us to fill the pipeline and store), and
-    // for a split the slab sum, a launch of 4 us and each slab written and
-    // read at 4 TB/s.  (Counting steps alone took 16 splits for a 14336-row
-    // gate/up pair at K = 4096, M = 77: 117 + 23 us against 80 + 7 with 2, and
-    // 8 for a 6144-row QKV at M = 512: 82 + 19 us against 72 + 8.)
-    double best = 0.0;
+    double best = 0.0;  // the split count of the smallest estimated time
     for (int sp = 1; sp <= std::max(1, std::min(16, nsteps / 4)); ++sp) {
-        const int sps = ((nsteps + sp - 1) / sp + 3) & ~3;
-        const int eff = (nsteps + sps - 1) / sps;  // non-empty splits
-        if (eff != sp) continue;
-        if (sp > 1 && one && fits &&
-            mmqp_sizes(dtype, std::min(M, prefill_granule(dtype)), K, cols, q6_rows, sp).total > kNoAllocBytes)
-            continue;
-        const double t = (double)((tiles * sp + cus - 1) / cus) * (2.1 * sps + 3.0) +
-                         (sp > 1 ? 4.0 + ((double)sp + 1.0) * M * cols * 4.0 / 4e6 : 0.0);
+        double t = mmqp_us(tiles, nsteps, sp, cus);
+        if (t == 0.0) continue;
+        if (sp > 1) {
+            if ((size_t)sp * M * cols * 4 > kMaxSlabs) break;
+            if (one && fits &&
+                mmqp_sizes(dtype, std::min(M, prefill_granule(dtype)), K, cols, q6_rows, sp).total > kNoAllocBytes)
+                break;
+            t += (sp + 1.0) * M * cols * kSlabUs;
+        }
         if (sp == 1 || t < best) {
             best = t;
             p.splits = sp;
         }
     }
     return mmqp_sizes(dtype, M, K, cols, q6_rows, p.splits);
+}
+
+// No plan_mmqp of up to M tokens, K elements (whole super-blocks) and cols
+// columns has more bytes of slabs: for every K and tile count, a split count is
+// the best only while there are few enough elements that its slabs cost less than
+// the time they save over each smaller count.
+size_t mmqp_max_slabs(int M, int K, int64_t cols, int cus) {
+    const int tm = fq::mmqp_tile_tokens(), tn = fq::mmqp_tile_rows();
+    const long tiles_max = (long)((M + tm - 1) / tm) * (long)((cols + tn - 1) / tn + 2);
+    double most = 0.0;
+    for (int nsteps = K / 64; nsteps >= 8; nsteps -= 4)
+        for (long tiles = 1; tiles <= tiles_max; ++tiles) {
+            const double n = std::min((double)M * (double)cols, (double)tiles * tm * tn);
+            double us[17];
+            for (int sp = 1; sp <= std::min(16, nsteps / 4); ++sp) {
+                us[sp] = mmqp_us(tiles, nsteps, sp, cus);
+                if (us[sp] == 0.0 || sp * n <= most) continue;
+                double ns = n;
+                for (int q = 1; q < sp; ++q)
+                    if (us[q] != 0.0)
+                        ns = std::min(ns, (us[q] - us[sp]) / ((q == 1 ? sp + 1 : sp - q) * kSlabUs) + 1.0);
+                if (sp > 1) most = std::max(most, sp * ns);
+            }
+            if (most * 4.0 >= (double)kMaxSlabs) return kMaxSlabs;
+        }
+    return (size_t)(most * 4.0) + 64;
 }
 
 // M > 1 on the matrix cores: token operand preparation, then one tile per
@@ -355,6 +397,7 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
             return kNotTaken;
         rows += n;
     }
+    if (q6k && ms.mm != fq::MM_ONE && (size_t)fq::mmqp_q6c_bytes(rows, K) > kMaxRewrite) return kNotTaken;
     fq::MmqArgs a{};
     a.mm = ms.mm;
     a.w = static_cast<const uint8_t*>(ms.w[0]);
@@ -1591,41 +1634,38 @@ int fq_reserve_workspace(int M_max, int K_max, int N_max, void* stream) {
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e);
     const DevInfo di = device_info(dev);
-    // slot 0: the largest MFMA-path plan for up to M_max tokens (the split-K
-    // slabs grow with splits x N, and fewer rows can mean more splits: every
-    // row count that changes the tile count is tried, with K_max and, for the
-    // prefill and band kernels, the largest multiple of 256 up to K_max)
+    // slot 0: the largest plan of up to M_max tokens, K_max columns and N_max rows
+    // per matrix, up to three of them in one launch
     size_t need0 = 0;
     const int Kp = K_max - K_max % 256;
-    for (int n = N_max; n > 0; n = n > 128 ? ((n - 1) / 128) * 128 : 0) {
+    const int64_t cols = 3 * (int64_t)N_max;
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    // the fp16 MFMA kernel (the split-K slabs grow with splits x N, and fewer rows
+    // can mean more splits: every row count that changes the tile count is
+    // tried), and the batch-1 kernel's K-split slabs for 2..4 tokens (at most 8)
+    for (int n = N_max; n > 0; n = n > 128 ? ((n - 1) / 128) * 128 : 0)
         for (int m = 2; m <= M_max; ++m) {
             need0 = std::max(need0, plan_mmq(m, K_max, n, di.cus).total);
-            if (m <= 16 && Kp > 0)  // band kernel (from M = 2), four- and two-tile bands
-                for (int mt : {4, 3, 2}) need0 = std::max(need0, mmqs_need(m, Kp, n, di.cus, mt));
-            if (m > 32 && Kp > 0) {  // one matrix, and a gate/up pair
-                const int tn = fq::mmqp_tile_rows();
-                // (with the larger sums of Q5_K and the rewritten rows of Q6_K)
-                need0 = std::max(need0, plan_mmqp(FQ_DTYPE_Q5_K, m, Kp, (n + tn - 1) / tn, n, n, true, di.cus).total);
-                need0 = std::max(need0, plan_mmqp(FQ_DTYPE_Q5_K, m, Kp, (2L * n + tn - 1) / tn, 2 * n, 2 * n, false, di.cus).total);
-            }
-            if (m <= 32 && Kp > 0) {  // one matrix, and a gate/up pair
-                fq::MmqArgs t{};
-                t.M = m;
-                t.K = Kp;
-                t.N = t.n1 = n;
-                for (uint32_t dt : {FQ_DTYPE_Q4_0, FQ_DTYPE_Q4_1, FQ_DTYPE_Q8_0, FQ_DTYPE_Q5_0,
-                                    FQ_DTYPE_Q5_1, FQ_DTYPE_Q4_K, FQ_DTYPE_Q5_K, FQ_DTYPE_Q6_K})
-                    for (int mm : {fq::MM_ONE, fq::MM_PAIR}) {
-                        Geometry g{};
-                        geometry(dt, g);
-                        t.mm = mm;
-                        t.row_bytes = (int)std::min<int64_t>((int64_t)(Kp / g.be) * g.bb, INT32_MAX);
-                        need0 = std::max(need0, plan_mmqt(t, dt, di.cus).total);
-                    }
-            }
-            // the batch-1 kernel's K-split slabs for 2..4 tokens (at most 8)
             if (m <= 4) need0 = std::max(need0, (size_t)8 * m * n * sizeof(float));
         }
+    if (M_max >= 2 && N_max > 0 && Kp > 0) {  // the band kernel (at most nsb / 8 splits of cus bands)
+        const int m = std::min(M_max, 16);
+        const MmqPlan pl = plan_mmq(m, Kp, N_max, di.cus);
+        const int64_t slabs = std::min<int64_t>(64LL * di.cus, (int64_t)(Kp / 2048) * N_max);
+        need0 = std::max(need0, 256 + al(pl.xop_b) + al(pl.xsum_b) + al(pl.ex_b) + al((size_t)slabs * m * 4));
+        // the shared-operand kernel: parts - 2 of a tile's columns are at most a
+        // step of every CU, so (parts - 2) cols <= 256 cus; 64 MiB in all
+        const int mt = std::min(M_max, 32);
+        const size_t ops = 256 + al(fq::mmqt_xop_bytes(mt, Kp)) + al(fq::mmqt_sum_bytes(mt, Kp));
+        const int64_t parts = std::min<int64_t>(16 * cols, 2 * cols + 256LL * di.cus);
+        need0 = std::max(need0, std::min(kNoAllocBytes, ops + al((size_t)parts * mt * 4)));
+    }
+    if (M_max > 32 && N_max > 0 && Kp > 0) {  // the prefill kernels
+        // (the larger sums of Q5_K, the rewritten rows of Q6_K)
+        const MmqpPlan pl = mmqp_sizes(FQ_DTYPE_Q5_K, M_max, Kp, 0, 0, 1);
+        const size_t row_b = (size_t)fq::mmqp_q6c_bytes(1, Kp);
+        const size_t q6c_b = std::max(row_b * N_max, std::min(row_b * (size_t)cols, kMaxRewrite));
+        need0 = std::max(need0, pl.total + al(q6c_b) + al(mmqp_max_slabs(M_max, Kp, cols, di.cus)));
     }
     const size_t need1 = 2 * (size_t)M_max * N_max * sizeof(float);
     uint8_t* p = nullptr;

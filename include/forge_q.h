@@ -31,8 +31,9 @@
  *    and the GGUF fused ops use a
  *    library-owned per-device, per-stream workspace (token operands, split-K
  *    partial slabs, intermediate rows; for Q6_K prefill, M > 32, the rows
- *    rewritten into 36-byte blocks of int8 codes: N * K * 9 / 8 bytes).  It grows on demand inside a call
- *    (hipMalloc, no host synchronisation; a superseded buffer is kept until
+ *    rewritten into 36-byte blocks of int8 codes: N * K * 9 / 8 bytes, those of
+ *    the two or three matrices of a fused op together while they take at most
+ *    160 MiB).  It grows on demand inside a call (hipMalloc, no host synchronisation; a superseded buffer is kept until
  *    fq_release_workspace) and lives until the process ends.  Under HIP-graph
  *    capture a call that would have to grow it returns FQ_ERR_WORKSPACE:
  *    size it first with fq_reserve_workspace.  The matmul.cpp:31-54
@@ -230,9 +231,11 @@ int fq_matmul_transB_noalloc(uint32_t dtype, const float* x, const void* w, cons
                              void* stream);
 
 /* Sizes the calling stream's workspace (current device) for every call with
- * at most M_max tokens, K_max columns and N_max rows, so that later calls
- * allocate nothing and can be captured into a HIP graph.  The size covers
- * every format, Q6_K prefill's rewritten rows included.  Replaces the
+ * at most M_max tokens, K_max columns and N_max rows (of each matrix of a
+ * fused op), so that later calls allocate nothing and can be captured into a
+ * HIP graph, where they run what they run outside of one.  The size covers
+ * every format, Q6_K prefill's rewritten rows included, and up to 256 MiB of
+ * the prefill kernels' K-split slabs.  Replaces the
  * reference's grow-on-first-use scratch (src/operators/cpu/matmul.cpp:31-54,
  * the thread-local buffer behind the CUDA Q8_0 M > 32 path), which has no
  * reserve call of its own. */

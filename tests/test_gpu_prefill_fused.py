@@ -105,3 +105,12 @@ def test_capture_with_a_workspace_for_single_matrices():
         torch.cuda.synchronize()
     del g
     assert L.fq_release_workspace(side.cuda_stream) == 0
+
+
+def test_q6k_pair_beyond_the_rewrite_limit():
+    # 167 MiB of rewritten rows: one call per matrix
+    dtype, M, N, K = F.Q6_K, 33, 19000, 4096
+    G, U = (dev_weight(dtype, synth.make_weights(dtype, N, K, s), N, K) for s in (80, 81))
+    x = torch.from_numpy(synth.make_x(M, K, seed=82) * np.float32(1e-2)).cuda()
+    ref = torch.nn.functional.silu(ops.matmul_transB(x, G)) * ops.matmul_transB(x, U)
+    torch.testing.assert_close(ops.ffn_up_fused(x, G, U), ref, rtol=2e-6, atol=1e-9)

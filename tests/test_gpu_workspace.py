@@ -145,3 +145,67 @@ def test_fused_qkv_small_batch_graph_replays():
         torch.cuda.synchronize()
     del g
     assert L.fq_release_workspace(side.cuda_stream) == 0
+
+
+def _fused(op, dtype, K, ns):
+    """x -> a fused call over matrices of ns rows."""
+    from forge_amd import ops
+    Ws = [ops.QWeight.from_numpy(synth.make_weights(dtype, n, K, 110 + i), dtype, n, K, device="cuda")
+          for i, n in enumerate(ns)]
+    fn = ops.fused_qkv if op == "qkv" else ops.ffn_up_fused
+    return lambda x: fn(x, *Ws)
+
+
+# Fused launches after a reserve for larger sizes: smaller K and N can take more
+# K-splits, three matrices more rows than any one.  The reserve covers them, so
+# the captured call is the eager one and neither allocates: the shared-operand
+# kernel (2..32 tokens) and the prefill kernels.
+@pytest.mark.parametrize("op,dtype,M,K,ns,reserve", [
+    ("pair", F.Q6_K, 307, 3584, (738, 738), (307, 4864, 739)),
+    ("pair", F.Q6_K, 408, 4096, (365, 365), (408, 5632, 365)),
+    ("qkv", F.Q8_0, 161, 4096, (470, 470, 470), (161, 4096, 470)),
+    ("pair", F.Q6_K, 15, 11520, (764, 764), (15, 12288, 764)),
+    ("pair", F.Q4_0, 3, 4096, (5632, 5632), (4, 4096, 5632)),
+    ("qkv", F.Q5_1, 27, 2048, (2048, 256, 256), (32, 5632, 2048)),
+    ("pair", F.Q5_K, 77, 4096, (14336, 14336), (77, 14336, 14336))])
+def test_reserve_covers_fused_launches(op, dtype, M, K, ns, reserve):
+    L = _lib.lib()
+    run = _fused(op, dtype, K, ns)
+    x = torch.from_numpy(synth.make_x(M, K, 121) * np.float32(1e-2)).cuda()
+    ref = run(x)  # on a workspace of its own that grows as it likes
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    assert L.fq_reserve_workspace(*reserve, side.cuda_stream) == 0
+    with torch.cuda.stream(side):
+        torch.empty_like(ref)  # the result's memory, before free memory is read
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        y = run(x)
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref)
+        with torch.cuda.stream(side):
+            assert torch.equal(run(x), ref)
+            run(x * 2)
+        torch.cuda.synchronize()
+    grown = free - torch.cuda.mem_get_info()[0]
+    assert grown < 32 << 20, f"{grown} bytes allocated after the reserve"  # torch's own blocks
+    del g
+    assert L.fq_release_workspace(side.cuda_stream) == 0
+
+
+def test_reserve_is_no_larger_than_its_calls_need():
+    # 512 tokens at 14336: the operands (33 MB), the rewritten rows of one Q6_K
+    # matrix (231 MB), at most 256 MiB of slabs, the rows of a fused op (59 MB)
+    L = _lib.lib()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    assert L.fq_reserve_workspace(512, 14336, 14336, side.cuda_stream) == 0
+    assert free - torch.cuda.mem_get_info()[0] <= 600 << 20
+    assert L.fq_release_workspace(side.cuda_stream) == 0
