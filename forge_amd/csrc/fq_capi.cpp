@@ -61,6 +61,9 @@ bool geometry(uint32_t dtype, Geometry& g) {
     }
 }
 
+// Whether a row's bytes fit the kernels' int.
+bool row_fits(const Geometry& g, int K) { return (int64_t)(K / g.be) * g.bb <= INT32_MAX; }
+
 // Formats with the aligned packed layout (fq_pack.h).
 bool packable(uint32_t dtype) { return fq::packed_row_bytes((int)dtype, 256) > 0; }
 
@@ -844,7 +847,7 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
     if (!x || !w || !y) return FQ_ERR_NULL;
     if (bias_mode != 0 && !bias) return FQ_ERR_NULL;
     if (bias_mode == 2 && bias_len < (int64_t)M * N) return FQ_ERR_SHAPE;
-    if ((int64_t)(K / g.be) * g.bb > INT32_MAX) return FQ_ERR_SHAPE;
+    if (!row_fits(g, K)) return FQ_ERR_SHAPE;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e);
@@ -1462,6 +1465,7 @@ int fq_fused_qkv(uint32_t dtype, const float* x, const void* wq, const void* wk,
     const int Nt = Nq + Nk + Nv;
     if (M == 0 || Nt == 0) return FQ_OK;
     if (!x || !y || (Nq && !wq) || (Nk && !wk) || (Nv && !wv)) return FQ_ERR_NULL;
+    if (!row_fits(g, K)) return FQ_ERR_SHAPE;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const void* ws[3] = {wq, wk, wv};
     const int ns[3] = {Nq, Nk, Nv};
@@ -1577,6 +1581,7 @@ int fq_ffn_up_fused(uint32_t dtype, const float* x, const void* w_gate, const vo
     if (M < 0 || N < 0 || K < 0 || K % g.be != 0) return FQ_ERR_SHAPE;
     if (M == 0 || N == 0) return FQ_OK;
     if (!x || !w_gate || !w_up || !y) return FQ_ERR_NULL;
+    if (!row_fits(g, K)) return FQ_ERR_SHAPE;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (M == 1 && packable(dtype)) {
         // one launch at every size: gate and up rows interleaved,

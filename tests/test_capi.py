@@ -79,6 +79,16 @@ def test_matmul_transB_bias_validation():
     assert L.fq_dequant_rows(F.Q4_0, None, one, 1, 32, None) == _lib.FQ_ERR_NULL
 
 
+@pytest.mark.parametrize("M", [1, 2, 8, 40])
+def test_rows_beyond_the_kernels_int_are_refused(M):
+    # Q8_0 rows of 2^31 - 32 elements are 2.28e9 bytes
+    L = _lib.lib()
+    one, K = ctypes.c_void_p(16), 2 ** 31 - 32
+    assert L.fq_matmul_transB(F.Q8_0, one, one, None, 0, 0, one, M, K, 1, None) == _lib.FQ_ERR_SHAPE
+    assert L.fq_fused_qkv(F.Q8_0, one, one, one, one, one, M, K, 1, 1, 1, None) == _lib.FQ_ERR_SHAPE
+    assert L.fq_ffn_up_fused(F.Q8_0, one, one, one, one, M, K, 1, None) == _lib.FQ_ERR_SHAPE
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "nope.so"))
