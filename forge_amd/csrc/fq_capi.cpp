@@ -1388,12 +1388,13 @@ int fq_dequant_rows(uint32_t dtype, const void* w, float* out, int N, int K, voi
     if (N < 0 || K < 0) return FQ_ERR_SHAPE;
     if (N == 0 || K == 0) return FQ_OK;
     if (!w || !out) return FQ_ERR_NULL;
+    const int64_t row_b = ((int64_t)K / g.be + (K % g.be != 0)) * g.bb;
+    if (row_b > INT32_MAX) return FQ_ERR_SHAPE;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e);
     const DevInfo di = device_info(dev);
-    const int nblk = (K + g.be - 1) / g.be;
-    e = fq::launch_dequant((int)dtype, static_cast<const uint8_t*>(w), out, N, K, nblk * g.bb,
+    e = fq::launch_dequant((int)dtype, static_cast<const uint8_t*>(w), out, N, K, (int)row_b,
                            di.cus, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? FQ_OK : hip_fail(e);
 }

@@ -162,13 +162,15 @@ struct Quad<Q3_K> {
 // a row is cut (its codes lie inside the row's last whole block), and rows
 // that are not whole 16-byte pieces are stored value by value.
 constexpr int CH = 4;
+// chunks per row (K up to the largest int)
+__host__ __device__ inline int dequant_chunks(int K) { return K / 256 + (K % 256 != 0); }
 template <int F>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ w,
                                                       float* __restrict__ out, int N, int K,
                                                       int row_bytes, int vec) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int cpr = (K + 255) / 256;  // chunks per row
+    const int cpr = dequant_chunks(K);
     const int64_t total = (int64_t)N * cpr, stride = (int64_t)gridDim.x * 4 * CH;
     for (int64_t c0 = ((int64_t)blockIdx.x * 4 + wave) * CH; c0 < total; c0 += stride) {
         int64_t row = c0 / cpr;
@@ -257,7 +259,7 @@ hipError_t launch_dequant(int dtype, const uint8_t* w, float* out, int N, int K,
                           int cus, hipStream_t st) {
     // whole 16-byte pieces: every row then starts on one
     const int vec = K % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    const int64_t chunks = (int64_t)N * ((K + 255) / 256);
+    const int64_t chunks = (int64_t)N * dequant_chunks(K);
     const int grid = (int)std::min<int64_t>((chunks + 4 * CH - 1) / (4 * CH), (int64_t)cus * 32);
     return with_format(dtype, hipErrorInvalidValue, [&](auto f) {
         hipLaunchKernelGGL(dequant_kernel<decltype(f)::value>, dim3(grid), dim3(256), 0, st, w,

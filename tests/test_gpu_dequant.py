@@ -30,3 +30,20 @@ def test_dequant_ragged_rows_and_bases(dtype, N, K, shift):
     got = out.cpu().numpy()
     assert np.array_equal(got[shift:shift + N * K].view(np.uint32), ref.reshape(-1).view(np.uint32))
     assert np.isnan(got[:shift]).all() and np.isnan(got[shift + N * K:]).all()
+
+
+# the longest row: its last chunk ends 31 below the largest int
+def test_dequant_longest_row():
+    K = 2 ** 31 - 32
+    w = torch.randint(0, 256, (K // 32 * 18,), dtype=torch.uint8, device="cuda")
+    w[0::18] = 0  # scales of 2^-14 and below
+    w[1::18] &= 0x83
+    out = torch.full((K,), float("nan"), device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    assert _lib.lib().fq_dequant_rows(F.Q4_0, w.data_ptr(), out.data_ptr(), 1, K, st) == 0
+    assert not torch.isnan(out.sum())
+    n = 4096  # of either end
+    for s, o in ((w[:n // 32 * 18], out[:n]), (w[-n // 32 * 18:], out[-n:])):
+        ref = oracle.dequant(F.Q4_0, s.cpu().numpy().reshape(1, -1), 1, n).reshape(n)
+        assert np.array_equal(o.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+    assert _lib.lib().fq_dequant_rows(F.Q8_0, w.data_ptr(), out.data_ptr(), 1, K, st) == _lib.FQ_ERR_SHAPE
