@@ -7,8 +7,8 @@
 // of fq_gemv1.hip under about 4 MB of weights); M = 2..4
 // the same batch-1 kernels with each weight unit dotted with every token;
 // M = 2..16 (by format and shape) the band kernel of fq_mmqs.hip
-// (Q6_K M = 4 on wide matrices: three tokens, then the fourth); M = 4..16 on
-// matrices of 24 to 48 MB and more and M = 17..32 the kernel of
+// (Q6_K M = 4 on wide matrices of 24 to 32 MiB: three tokens, then the fourth);
+// M = 4..16 on matrices of 24 to 48 MiB and more and M = 17..32 the kernel of
 // fq_mmqt.hip; M > 32 the prefill kernels
 // of fq_mmqk.hip and fq_mmqp.hip (rows in 16-byte chunks, K a multiple of 256); the rest --
 // the reference's batched GEMV (1 < M <= 32) and dequant + GEMM prefill
@@ -873,14 +873,21 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
         if (rc != FQ_ERR_SHAPE) return rc;
     }
 
+    if (thin_takes(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {
+        const int rc = run_thin(dtype, g, x, Mats{fq::MM_ONE, {w}, {N}}, bias, bias_mode, bias_len, y, M,
+                                K, N, dev, di, st, fixed, fixed_cap);
+        if (rc != kNotTaken) return rc;
+    }
+
     if (dtype == FQ_DTYPE_Q6_K && M == 4 && K > 0 && N > 16384 &&
         (int64_t)N * (K / g.be) * g.bb >= (24 << 20)) {
-        // four Q6_K tokens on 24 MB and more of more than 16384 rows: three on
-        // the batch-1 kernel, then the fourth (its four-token form spills;
-        // 152064 x 3584 196-203 us against 209 on the band kernel, 18944 x
-        // 3584 34.7 against 37.3); fewer rows, and five tokens, take the band
-        // kernel below (3584 x 18944 35.0 against 45.9 this way, 14336 x 4096
-        // 27.8 against 30.8, lm_head at M = 5 about 211 against 222)
+        // four Q6_K tokens on 24 MB and more of more than 16384 rows that the
+        // shared-operand kernel above does not take (under 32 MiB; 152064 x 3584
+        // 126 us there, 203 this way, 18944 x 3584 26.2 and 36.2, 20000 x 2048,
+        // 32.0 MiB, 19.2 and 31.6): three on the batch-1 kernel, whose four-token
+        // form spills, then the fourth (18944 x 3584 34.7 against 37.3 on the
+        // band kernel); fewer rows take the band kernel below (14336 x 4096 27.8
+        // against 30.8)
         for (int t0 = 0; t0 < M; t0 += 3) {
             const int m = std::min(3, M - t0);
             const int rc = run_matmul(dtype, x + (size_t)t0 * K, w,
@@ -890,12 +897,6 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
             if (rc != FQ_OK) return rc;
         }
         return FQ_OK;
-    }
-
-    if (thin_takes(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {
-        const int rc = run_thin(dtype, g, x, Mats{fq::MM_ONE, {w}, {N}}, bias, bias_mode, bias_len, y, M,
-                                K, N, dev, di, st, fixed, fixed_cap);
-        if (rc != kNotTaken) return rc;
     }
 
     const BandRule rule = band_rule(dtype, g, M, K, N, w, di.cus);

@@ -132,3 +132,11 @@ def test_pair_ranges_over_tiles(dtype, M, N, K):
                          dev_weight(dtype, wu, N, K))
     g, u = (oracle.matmul_f64(dtype, x, w, N, K) for w in (wg, wu))
     assert_close_silu_mul(y.cpu().numpy(), g, u, x, wmax(dtype, [wg, wu], K), f"{dtype} {M}x{N}x{K}")
+
+
+def test_q6k_four_tokens_on_many_rows():
+    # as five tokens: the same kernel, a token's bits its own
+    N, K = 24001, 2048
+    W = dev_weight(F.Q6_K, synth.make_weights(F.Q6_K, N, K, 90), N, K)
+    x = torch.from_numpy(synth.make_x(5, K, seed=91)).cuda()
+    assert torch.equal(ops.matmul_transB(x[:4], W), ops.matmul_transB(x, W)[:4])
