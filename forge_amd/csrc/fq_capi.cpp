@@ -497,7 +497,7 @@ struct MmqtPlan {
 // work-group per CU: 1.5 us to fill the pipeline, the steps, 1 us per tile
 // ended, and for tiles in parts their sum (3.5 us and each slab written and
 // read at 4 TB/s).  A step's time is what 14336 x 4096 measured on 224
-// work-groups, or its weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x
+// work-groups (Q6_K without the product of its low parts, 4 % of it), or its weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x
 // 3584 at M = 16: 134 us on 128 rows, 156 on 64).
 //
 // No plan takes more than the fixed array of fq_matmul_transB_noalloc, so that
@@ -546,14 +546,14 @@ MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
 }
 
 // Whether 4..32 tokens on one matrix of this size go there.  17..32 tokens
-// always (the fp16 MFMA path: Q4_K 4096 x 4096 at M = 32 20.8 -> 14.7 us, 14336 x
-// 4096 40.2 -> 23.2, Q8_0 40.5 -> 25.2, Q6_K 4096 x 14336 56.4 -> 29.0).  Up to
+// always (the fp16 MFMA path: Q4_K 4096 x 4096 at M = 32 20.8 -> 14.1 us, 14336 x
+// 4096 40.2 -> 24.0, Q8_0 40.5 -> 28.6, Q6_K 4096 x 14336 56.4 -> 30.3).  Up to
 // 16 from 24 MiB of Q4_K and Q5_K, 48 of Q8_0, 32 of the others: below, the band
 // kernel's bands fill the chip without a K split and its slab sum (M = 8: Q4_K
 // 8192 x 4096, 19 MB, 12.6 us there, 13.5 here, 14336 x 4096, 33 MB, 18.7 and
-// 16.3; Q6_K 28 MB 16.5 and 16.8, 48 MB 27.6 and 20.9; Q8_0 36 MB 14.1 and
-// 15.3, 62 MB 23.5 and 19.2; Q4_0 33 MB 17.8 and 17.3, 38 MB 24.0 and 20.0;
-// 152064 x 3584: Q4_0 132 and 100, Q8_0 171 and 132, Q6_K 211 and 124).
+// 16.3; Q6_K 28 MB 16.5 and 16.8, 48 MB 27.6 and 21.7; Q8_0 36 MB 14.1 and
+// 15.3, 62 MB 23.5 and 20.0; Q4_0 33 MB 17.8 and 16.7, 38 MB 24.0 and 20.6;
+// 152064 x 3584: Q4_0 132 and 96, Q8_0 171 and 131, Q6_K 211 and 127).
 bool thin_takes(uint32_t dtype, int M, int64_t bytes) {
     if (!fq::mmqt_supported((int)dtype) || M < 4 || M > 32) return false;
     const int64_t mib = dtype == FQ_DTYPE_Q4_K || dtype == FQ_DTYPE_Q5_K ? 24
@@ -564,7 +564,7 @@ bool thin_takes(uint32_t dtype, int M, int64_t bytes) {
 
 // Whether a gate/up pair of such matrices goes there: as one matrix, or two to
 // four tokens, which otherwise take two launches and a SiLU pass (M = 4: Q4_0
-// 5632 x 2048 18.4 -> 11.6 us, 18944 x 3584 52.4 -> 36; M = 2: 13.9 -> 11.6), but
+// 5632 x 2048 18.4 -> 10.9 us, 18944 x 3584 52.4 -> 31.2; M = 2: 13.9 -> 10.8), but
 // not two on large matrices of the formats whose batch-1 kernel then reads at
 // nearly the rate of one token (M = 2: Q4_0 18944 x 3584 30.2 against 35.8, Q6_K
 // 37.6 against 44.3, Q8_0 14336 x 4096 33.8 against 34.5).

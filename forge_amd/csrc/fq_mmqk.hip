@@ -25,20 +25,22 @@
 // the result's error against 64 bits was 40 % larger, 3.2e-7 at K = 4096)
 //
 // against one FMA per output and 32-element block and an fp32 MFMA per 64
-// elements for the minimum: the chip's power limit sets the rate of these
-// kernels (a loop of nothing but v_mfma_f32_32x32x16_f16 on random operands
-// sustains 1.42 PFLOP/s, on zeros 2.47; 128 FMAs and 16 LDS reads beside each
-// 32 MFMAs cost a fifth of it), so every vector instruction taken out of a
-// step counts, also where it would have overlapped a matrix instruction.
+// elements for the minimum.  A loop of nothing but v_mfma_f32_32x32x16_f16 runs
+// at 2.49 PFLOP/s on zeros with one wave per SIMD, 1.64 on random operands, and
+// with two waves, as here, at 1.66 and 1.21: the rate falls with what the
+// operands and the waves cost in power, and 128 FMAs and 16 LDS reads beside each
+// 32 MFMAs took a fifth of it.  This kernel reaches 0.93 with its matrix cores
+// busy 55 % of the cycles, so every vector instruction taken out of a step
+// counts, also where it would have overlapped a matrix instruction.
 // The multiply by sc replaces the subtract that removes the 1024 of the
 // byte-to-half trick: with the code in the top bits of its byte the half reads
 // 1024 + 16 q (Q5_K 1024 + 8 q), and (1024 + 16 q) (sc / 16) - 72 sc =
 // sc (q - 8) is one packed FMA whose operands and result are exact (72 sc =
 // 9 * 63 * 8 at most: 10 bits).
 //
-// Measured (whole calls): Q4_K 3584 -> 18944, M = 1999 698 -> 615 us; 4096 ->
-// 14336, M = 512 170 -> 146; Q5_K, which had no such kernel, 4096 -> 14336 at
-// M = 77 101 -> 52, M = 512 148; Q4_K error against 64 bits 2.0e-7 (3.3e-7).
+// Measured (whole calls): Q4_K 3584 -> 18944, M = 1999 698 -> 595 us; 4096 ->
+// 14336, M = 512 170 -> 134; Q5_K, which had no such kernel, 4096 -> 14336 at
+// M = 77 101 -> 44, M = 512 149; Q4_K error against 64 bits 2.0e-7 (3.2e-7).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -15,15 +15,15 @@
 // fq_mmqs.hip every wave reads the token operands of its own super-blocks from
 // L2, for 32 or 64 rows: 3.5 times the weight bytes for a Q6_K head at 16
 // tokens (1.1 GB).  Here the operands of a super-block serve all rows of the
-// work-group.  152064 x 3584 Q6_K, M = 16: 216 -> 129 us; Q4_K, M = 8 131 ->
-// 98; 14336 x 4096 Q4_K, M = 8 18.7 -> 16.3, M = 32 (fp16 MFMA kernel) 40.2 ->
-// 23.2, gate and up of that size in one launch 37.7 -> 22.0 and 82.5 -> 36.0.
+// work-group.  152064 x 3584 Q6_K, M = 16: 216 -> 131 us; Q4_K, M = 8 131 ->
+// 94; 14336 x 4096 Q4_K, M = 8 18.7 -> 16.3, M = 32 (fp16 MFMA kernel) 40.2 ->
+// 24.0, gate and up of that size in one launch 37.7 -> 23.8 and 82.5 -> 35.8.
 // What bounds it: vector and matrix issue, then the LDS reads of the token
-// operands (Q6_K head, M = 16: vector issue 68 % of the cycles, the matrix
-// cores 22 %, LDS 33 %; with a work-group per tile half, 139 us in all, the head
-// took 117 without the copies, 105 without the arithmetic), so the waves per
-// SIMD count: 256 rows on eight waves of two tiles each ran the head in 152 us,
-// on sixteen waves 139.
+// operands (Q6_K head, M = 16: vector issue 69 % of the cycles, the matrix
+// cores 28 %, LDS 32 %; an earlier form with a work-group per tile half and
+// without the x_lo W_lo product, 139 us in all, took 117 without the copies, 105
+// without the arithmetic), so the waves per SIMD count: that form with 256 rows
+// on eight waves of two tiles each ran the head in 152 us, on sixteen waves 139.
 //
 // Tokens are the A operand of v_mfma_f32_16x16x32_f16 (lane 16 q + c: token c,
 // eight elements of k group q) and weights the B operand (lane 16 q + c: row
@@ -35,7 +35,8 @@
 //   Q4_K, Q5_K: sc (q - c) as in fq_mmqk.hip, exact in fp16 (at most 1008);
 //   Q6_K: sc (q - 32) has up to 13 bits: W = W_hi + W_lo, W_hi its fp16
 //   rounding and W_lo the exact rest; all four products are formed (without
-//   x_lo W_lo, up to 2^-22 of a product, the codes would not be exact).
+//   x_lo W_lo, up to 2^-22 of a product, the codes would not be exact; the
+//   head at M = 16 takes 131 us with it, 125 without).
 //
 //   the 32-element blocks: the integer code, d on the results (TQB below).
 //

@@ -164,8 +164,10 @@ int fq_gemv_packed(uint32_t dtype, const float* x, const void* w_packed, const f
  * silu(g) = g / (1 + exp(-g)); Wgate and Wup have the same dtype and shape.
  * ---------------------------------------------------------------------- */
 
-/* GGUF-layout weights, any M >= 1: two matmuls (as fq_matmul_transB) into a
- * library-owned per-stream buffer, then the SiLU-multiply.  Replaces the
+/* GGUF-layout weights, any M >= 1: one launch where one kernel takes both
+ * matrices (most calls), else two matmuls (as fq_matmul_transB) into a
+ * library-owned per-stream buffer, then the SiLU-multiply.  A token's result may
+ * differ in its last bits between values of M, whose kernels differ.  Replaces the
  * device branch of ops::ffn_up_fused (matmul.cpp:1472-1533): the launchers
  * cuda::launch_ffn_up_fused_q4_0 / _q4_k and their batch forms
  * (cuda_fused.cu:15-106, 622-748) and the matmul_transB + silu_multiply

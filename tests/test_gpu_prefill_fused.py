@@ -72,10 +72,11 @@ def test_one_matrix_at_an_offset_base(dtype):
 
 def test_capture_with_a_workspace_for_single_matrices():
     # the one-launch QKV wants a larger workspace than its matrices one by
-    # one; where that cannot grow (capture) the call still runs, as it does
-    # with the same reservation eagerly
+    # one (16 K-splits of 3072 columns, the rewritten rows of three matrices);
+    # where a reservation for smaller matrices cannot grow to it (capture) the
+    # call still runs, one matrix at a time
     L = _lib.lib()
-    dtype, M, K, ns = F.Q4_K, 64, 4096, (1024, 1024, 1024)
+    dtype, M, K, ns = F.Q6_K, 64, 4096, (1024, 1024, 1024)
     ws = [torch.from_numpy(synth.make_weights(dtype, n, K, 70 + i).reshape(-1)).cuda()
           for i, n in enumerate(ns)]
     x = torch.from_numpy(synth.make_x(M, K, 73)).cuda()
@@ -87,7 +88,7 @@ def test_capture_with_a_workspace_for_single_matrices():
                               *ns, side.cuda_stream)
 
     with torch.cuda.stream(side):
-        assert L.fq_reserve_workspace(M, K, 1024, side.cuda_stream) == 0
+        assert L.fq_reserve_workspace(M, K, 512, side.cuda_stream) == 0
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g, stream=side):
         st = call(y)
