@@ -129,6 +129,7 @@ struct StreamScratch {
             *out = s_.p;
             return FQ_OK;
         }
+        size_t held() const { return s_.n; }
 
       private:
         std::unique_lock<std::mutex> lk_;
@@ -414,7 +415,6 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
     a.K = K;
     const int cols = fq::mm_cols(a), q6_rows = q6k ? rows : 0;
     MmqpPlan pl = plan_mmqp(dtype, M, K, fq::mmqp_row_tiles(a), cols, q6_rows, ms.mm == fq::MM_ONE, di.cus);
-    const int splits = pl.splits;
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     std::unique_ptr<StreamScratch::Lease> lease;
     uint8_t* buf = fixed;
@@ -431,15 +431,22 @@ int run_prefill(uint32_t dtype, const Geometry& g, const float* x, const Mats& m
             return FQ_ERR_WORKSPACE;
         while (pl.total > fixed_cap && mc > prefill_granule(dtype)) {
             mc = mc > 64 ? (mc - 1) / 64 * 64 : mc / 2;
-            pl = mmqp_sizes(dtype, mc, K, cols, q6_rows, splits);
+            pl = mmqp_sizes(dtype, mc, K, cols, q6_rows, pl.splits);
         }
         if (pl.total > fixed_cap) return FQ_ERR_WORKSPACE;
     } else {
         lease.reset(new StreamScratch::Lease(stream_scratch(dev, st, 0)));
-        const int rc = lease->get(pl.total, st, &buf);
-        if (rc == FQ_ERR_WORKSPACE && ms.mm != fq::MM_ONE) return kNotTaken;
+        int rc = lease->get(pl.total, st, &buf);
+        if (rc == FQ_ERR_WORKSPACE) {
+            // capture on a workspace that another call sized: fewer tokens can
+            // take more splits, one split takes the operands alone
+            pl = mmqp_sizes(dtype, M, K, cols, q6_rows, 1);
+            if (pl.total > lease->held()) return ms.mm != fq::MM_ONE ? kNotTaken : rc;
+            rc = lease->get(pl.total, st, &buf);
+        }
         if (rc != FQ_OK) return rc;
     }
+    const int splits = pl.splits;
     hipError_t e = hipSuccess;
     if (q6k) {
         uint8_t* conv = buf + al(pl.xop_b) + al(pl.ex_b) + al(pl.sum_b) + al(pl.part_b);
@@ -497,12 +504,13 @@ struct MmqtPlan {
 // work-group per CU: 1.5 us to fill the pipeline, the steps, 1 us per tile
 // ended, and for tiles in parts their sum (3.5 us and each slab written and
 // read at 4 TB/s).  A step's time is what 14336 x 4096 measured on 224
-// work-groups (Q6_K without the product of its low parts, 4 % of it), or its weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x
-// 3584 at M = 16: 134 us on 128 rows, 156 on 64).
+// work-groups (Q6_K without the product of its low parts, 4 % of it), or its
+// weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x 3584 at M = 16: 134 us on
+// 128 rows, 156 on 64).
 //
 // No plan takes more than the fixed array of fq_matmul_transB_noalloc, so that
-// the plan is the same there.
-MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
+// the plan is the same there (cap: what a workspace under capture holds).
+MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus, size_t cap = kNoAllocBytes) {
     const bool q6 = dtype == FQ_DTYPE_Q6_K, wide = a.M > 16;
     MmqtPlan p{};
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
@@ -525,7 +533,7 @@ MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus) {
             per = std::min(per, whole);
             const int parts = fq::mmqt_parts(nst, per);
             const size_t part_b = parts > 1 ? (size_t)parts * a.M * fq::mm_cols(a) * 4 : 0;
-            if (parts <= 16 && ops_b + al(part_b) <= kNoAllocBytes) {
+            if (parts <= 16 && ops_b + al(part_b) <= cap) {
                 const double busy = (double)((total + per - 1) / per);
                 const double step = std::max(it, busy * kg * rows * sb_bytes / 5e6);
                 const double t = 1.5 + step * per + (double)((per + nst - 1) / nst) +
@@ -602,7 +610,7 @@ int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, 
     a.M = M;
     a.N = N;
     a.K = K;
-    const MmqtPlan pl = plan_mmqt(a, dtype, di.cus);
+    MmqtPlan pl = plan_mmqt(a, dtype, di.cus);
     if (pl.rows == 0) return kNotTaken;
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     std::unique_ptr<StreamScratch::Lease> lease;
@@ -611,8 +619,14 @@ int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, 
         if (pl.total > fixed_cap) return FQ_ERR_WORKSPACE;
     } else {
         lease.reset(new StreamScratch::Lease(stream_scratch(dev, st, 0)));
-        const int rc = lease->get(pl.total, st, &buf);
-        if (rc == FQ_ERR_WORKSPACE) return kNotTaken;
+        int rc = lease->get(pl.total, st, &buf);
+        if (rc == FQ_ERR_WORKSPACE) {
+            // capture on a workspace that another call sized: fewer tokens can
+            // take more parts (14336 x 4096 Q4_K pair, 17 tokens 8.3 MB, 32 0.5)
+            pl = plan_mmqt(a, dtype, di.cus, std::min(kNoAllocBytes, lease->held()));
+            if (pl.rows == 0) return kNotTaken;
+            rc = lease->get(pl.total, st, &buf);
+        }
         if (rc != FQ_OK) return rc;
     }
     a.xop = buf;

@@ -35,8 +35,9 @@
  *    the two or three matrices of a fused op together while they take at most
  *    160 MiB).  It grows on demand inside a call (hipMalloc, no host synchronisation; a superseded buffer is kept until
  *    fq_release_workspace) and lives until the process ends.  Under HIP-graph
- *    capture a call that would have to grow it returns FQ_ERR_WORKSPACE:
- *    size it first with fq_reserve_workspace.  The matmul.cpp:31-54
+ *    capture a call that would have to grow it takes fewer K-splits where that
+ *    fits (its last bits may differ), else returns FQ_ERR_WORKSPACE: size it
+ *    first with fq_reserve_workspace.  The matmul.cpp:31-54
  *    thread-local grow-only buffer of the reference plays the same role.
  */
 #ifndef FORGE_Q_H

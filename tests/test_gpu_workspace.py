@@ -209,3 +209,41 @@ def test_reserve_is_no_larger_than_its_calls_need():
     assert L.fq_reserve_workspace(512, 14336, 14336, side.cuda_stream) == 0
     assert free - torch.cuda.mem_get_info()[0] <= 600 << 20
     assert L.fq_release_workspace(side.cuda_stream) == 0
+
+
+# No reserve, the workspace sized by an eager call of more tokens: a plan for
+# fewer tokens can want more of it (parts of row tiles, K-splits), so under
+# capture it makes do with what is there
+@pytest.mark.parametrize("op,dtype,Mw,M,K,ns", [
+    ("one", F.Q4_K, 32, 17, 1024, (8192,)), ("one", F.Q4_K, 32, 19, 4096, (4096,)),
+    ("pair", F.Q4_K, 32, 17, 4096, (14336, 14336)), ("qkv", F.Q4_K, 32, 19, 4096, (2048, 512, 512)),
+    ("pair", F.Q8_0, 256, 130, 4096, (2048, 2048)), ("one", F.Q5_K, 512, 130, 4096, (4096,))])
+def test_capture_of_fewer_tokens_than_warmed_up(op, dtype, Mw, M, K, ns):
+    from forge_amd import ops
+    L = _lib.lib()
+    if op == "one":
+        W = ops.QWeight.from_numpy(synth.make_weights(dtype, ns[0], K, 130), dtype, ns[0], K, device="cuda")
+        run = lambda x: ops.matmul_transB(x, W)  # noqa: E731
+    else:
+        run = _fused(op, dtype, K, ns)
+    x = torch.from_numpy(synth.make_x(Mw, K, 131) * np.float32(1e-2)).cuda()
+    ref = run(x[:M])
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        run(x)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        y = run(x[:M])
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert float((y - ref).norm() / ref.norm()) < 1e-6
+        with torch.cuda.stream(side):
+            assert torch.equal(run(x[:M]), ref)  # outside of capture it grows
+        torch.cuda.synchronize()
+    del g
+    assert L.fq_release_workspace(side.cuda_stream) == 0
