@@ -506,12 +506,16 @@ struct MmqtPlan {
 // read at 4 TB/s).  A step's time is what 14336 x 4096 measured on 224
 // work-groups (Q6_K without the product of its low parts, 4 % of it), or its
 // weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x 3584 at M = 16: 134 us on
-// 128 rows, 156 on 64).
+// 128 rows, 156 on 64).  Of Q8_0's tiles 128 rows run in one wave group and 64 in two:
+// a step of either reads the same bytes, and where tiles outnumber the CUs 64 rows take
+// as long per step, up to 16 tokens (at 1.3 us a step a pair of 17408 x 8192 took 98 us on 64 rows at M =
+// 3, 72 on 128, 18944 x 4096 48.8 and 39.2; fewer tiles, parts to sum: 3072 x 2816 12.6
+// on 64, 15.5 on 128).
 //
 // No plan takes more than the fixed array of fq_matmul_transB_noalloc, so that
 // the plan is the same there (cap: what a workspace under capture holds).
 MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus, size_t cap = kNoAllocBytes) {
-    const bool q6 = dtype == FQ_DTYPE_Q6_K, wide = a.M > 16;
+    const bool q6 = dtype == FQ_DTYPE_Q6_K, q8 = dtype == FQ_DTYPE_Q8_0, wide = a.M > 16;
     MmqtPlan p{};
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     p.xop_b = fq::mmqt_xop_bytes(a.M, a.K);
@@ -522,10 +526,10 @@ MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus, size_t cap = k
     for (int rows : {256, 128, 64}) {
         const int kg = fq::mmqt_groups((int)dtype, a.M, rows);
         if (kg == 0) continue;
-        const double it = rows == 256   ? (q6 ? 2.7 : wide ? 2.6 : 2.0)
-                          : rows == 128 ? (q6 ? (wide ? 2.2 : 1.7) : wide ? 1.6 : 1.7)
-                                        : (q6 ? 1.8 : 1.3);
         const int tiles = fq::mmqt_row_tiles(a, rows), nst = fq::mmqt_steps(a.K, kg);
+        const double it = rows == 256 ? (q6 ? 2.7 : wide ? 2.6 : 2.0)
+                          : rows == 128 ? (q6 ? (wide ? 2.2 : 1.7) : wide ? 1.6 : 1.7)
+                                        : (q6 ? 1.8 : q8 && !wide && tiles > cus ? 1.8 : 1.3);
         const int whole = nst * ((tiles + cus - 1) / cus);
         const int64_t total = (int64_t)tiles * nst;
         if (total >= (int64_t)1 << 31) continue;
