@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdlib>
 #include <cstdio>
 #include <cstdint>
@@ -508,9 +509,9 @@ struct MmqtPlan {
 // weight bytes on all busy CUs at 5 TB/s (Q8_0 152064 x 3584 at M = 16: 134 us on
 // 128 rows, 156 on 64).  Of Q8_0's tiles 128 rows run in one wave group and 64 in two:
 // a step of either reads the same bytes, and where tiles outnumber the CUs 64 rows take
-// as long per step, up to 16 tokens (at 1.3 us a step a pair of 17408 x 8192 took 98 us on 64 rows at M =
-// 3, 72 on 128, 18944 x 4096 48.8 and 39.2; fewer tiles, parts to sum: 3072 x 2816 12.6
-// on 64, 15.5 on 128).
+// as long per step, up to 16 tokens (at 1.3 us a step a pair of 17408 x 8192 took 98
+// us on 64 rows at M = 3, 72 on 128, 18944 x 4096 48.8 and 39.2; fewer tiles, parts to
+// sum: 3072 x 2816 12.6 on 64, 15.5 on 128).
 //
 // No plan takes more than the fixed array of fq_matmul_transB_noalloc, so that
 // the plan is the same there (cap: what a workspace under capture holds).
@@ -557,7 +558,39 @@ MmqtPlan plan_mmqt(const fq::MmqArgs& a, uint32_t dtype, int cus, size_t cap = k
     return p;
 }
 
-// Whether 4..32 tokens on one matrix of this size go there.  17..32 tokens
+// Estimates of whole calls up to 16 tokens, us, for the choice between this kernel and
+// the band kernel, fitted to 5632 .. 18944 rows x 1024 .. 8192 (this kernel: 5750 calls,
+// 3.1 % rms, band: 840, 3.2 %).  thin: a super-block of 128 rows here (256 rows take
+// 1.7 times as long, 64 0.66 where 128 run in two wave groups, 0.61 in one); band: a
+// super-block of a 16-row tile there.
+struct SmallUs {
+    double thin, band;
+};
+SmallUs small_us(uint32_t dtype) {
+    switch (dtype) {
+        case FQ_DTYPE_Q4_0: return {1.00, 0.145};
+        case FQ_DTYPE_Q4_1: return {1.04, 0.169};
+        case FQ_DTYPE_Q8_0: return {1.30, 0.168};
+        case FQ_DTYPE_Q5_0: return {1.24, 0.185};
+        case FQ_DTYPE_Q5_1: return {1.41, 0.185};
+        case FQ_DTYPE_IQ4_NL: return {1.27, 0.199};
+        case FQ_DTYPE_Q4_K: return {0.91, 0.161};
+        case FQ_DTYPE_Q5_K: return {1.02, 0.173};
+        default: return {1.53, 0.246};  // Q6_K
+    }
+}
+double thin_us(const MmqtPlan& p, const fq::MmqArgs& a, uint32_t dtype) {
+    const double r = p.rows == 256                                ? 1.7
+                     : p.rows == 128                              ? 1.0
+                     : fq::mmqt_groups((int)dtype, a.M, 128) == 2 ? 0.66
+                                                                  : 0.61;
+    return 6.0 + r * small_us(dtype).thin * p.per * fq::mmqt_groups((int)dtype, a.M, p.rows) +
+           (p.parts > 1 ? 4.6 + 0.37e-6 * (double)p.part_b : 0.0) +
+           0.033e-6 * a.row_bytes * fq::mm_cols(a);
+}
+
+// Whether 4..32 tokens on one matrix of this size go there, up to 16 unless the
+// band kernel is estimated faster by 4 %.  17..32 tokens
 // always (the fp16 MFMA path: Q4_K 4096 x 4096 at M = 32 20.8 -> 14.1 us, 14336 x
 // 4096 40.2 -> 24.0, Q8_0 40.5 -> 28.6, Q6_K 4096 x 14336 56.4 -> 30.3).  Up to
 // 16 from 24 MiB of Q4_K and Q5_K, 48 of Q8_0, 32 of the others: below, the band
@@ -574,24 +607,27 @@ bool thin_takes(uint32_t dtype, int M, int64_t bytes) {
     return M > 16 || bytes >= mib << 20;
 }
 
-// Whether a gate/up pair of such matrices goes there: as one matrix, or two to
-// four tokens, which otherwise take two launches and a SiLU pass (M = 4: Q4_0
+// Whether a gate/up pair of such matrices goes there: as one matrix of both's rows,
+// or two to four tokens, which otherwise take two launches and a SiLU pass (M = 4: Q4_0
 // 5632 x 2048 18.4 -> 10.9 us, 18944 x 3584 52.4 -> 31.2; M = 2: 13.9 -> 10.8), but
 // not two on large matrices of the formats whose batch-1 kernel then reads at
 // nearly the rate of one token (M = 2: Q4_0 18944 x 3584 30.2 against 35.8, Q6_K
-// 37.6 against 44.3, Q8_0 14336 x 4096 33.8 against 34.5).
+// 37.6 against 44.3, Q8_0 14336 x 4096 33.8 against 34.5).  Two tokens of other formats
+// stay, also where two launches are faster (Q5_0 17408 x 2048 21.9 against 24.3): the
+// batch-1 kernel's limbs err by 1.4..1.9e-6 there, this one by 1.6e-7.
 bool thin_takes_pair(uint32_t dtype, int M, int64_t bytes) {
     if (!fq::mmqt_supported((int)dtype) || M < 2) return false;
     if (M == 2 && (dtype == FQ_DTYPE_Q4_0 || dtype == FQ_DTYPE_Q6_K || dtype == FQ_DTYPE_Q8_0))
         return bytes < 24 << 20;
-    return M <= 4 || thin_takes(dtype, M, bytes);
+    return M <= 4 || thin_takes(dtype, M, 2 * bytes);
 }
 
 // kNotTaken: another kernel runs the call (also where the workspace cannot grow
-// to this one's operands under capture).
+// to this one's operands under capture).  kSlower: estimated above limit_us.
+constexpr int kSlower = -2;
 int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, const float* bias,
              int bias_mode, int64_t bias_len, float* y, int M, int K, int N, int dev,
-             const DevInfo& di, hipStream_t st, uint8_t* fixed, size_t fixed_cap) {
+             const DevInfo& di, hipStream_t st, uint8_t* fixed, size_t fixed_cap, double limit_us) {
     if (!fq::mmqt_supported((int)dtype) || M < 2 || M > 32 || K <= 0 || K % 256 != 0) return kNotTaken;
     const bool q6k = dtype == FQ_DTYPE_Q6_K;
     const int64_t rb = (int64_t)(K / g.be) * g.bb;
@@ -616,6 +652,7 @@ int run_thin(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, 
     a.K = K;
     MmqtPlan pl = plan_mmqt(a, dtype, di.cus);
     if (pl.rows == 0) return kNotTaken;
+    if (thin_us(pl, a, dtype) > limit_us) return kSlower;
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     std::unique_ptr<StreamScratch::Lease> lease;
     uint8_t* buf = fixed;
@@ -752,6 +789,28 @@ int band_tiles(uint32_t dtype, int K, int N, int cus) {
     return tiles;
 }
 
+// Rows per band (a pair: gate rows, as many up rows) and K-splits of a band call.
+struct BandPlan {
+    int tiles, rpw, splits;
+};
+BandPlan band_plan(uint32_t dtype, int K, int N, bool pair, int cus) {
+    BandPlan p{band_tiles(dtype, K, N, cus), 0, 1};
+    if (pair) p.tiles = p.tiles >= 4 ? 4 : 2;
+    p.splits = mmqs_plan(pair ? 2 * N : N, K, cus, &p.rpw, p.tiles);
+    if (pair) p.rpw = 16 * ((p.rpw / 16 + 1) / 2);
+    return p;
+}
+// Its estimated time: rounds of work-groups, each its super-blocks of its tiles, a
+// K split's slab sum and the weight bytes (SmallUs).
+double band_us(uint32_t dtype, const Geometry& g, int K, int N, bool pair, int cus) {
+    const BandPlan p = band_plan(dtype, K, N, pair, cus);
+    const int nsb = K / 256, sb = (nsb + p.splits - 1) / p.splits;
+    const long wgs = ((long)N + p.rpw - 1) / p.rpw * p.splits, rounds = (wgs + cus - 1) / cus;
+    const double mats = pair ? 2.0 : 1.0, tiles = mats * (p.rpw / 16);
+    return 5.9 + 1.74 * (rounds - 1.0) + (double)rounds * sb * (small_us(dtype).band * tiles + 0.037) +
+           (p.splits > 1 ? 1.75 : 0.0) + 0.071e-6 * mats * N * ((double)(K / g.be) * g.bb);
+}
+
 // 2..16 tokens (by format and shape): token operands, then one pass over the
 // weights on the fp16 matrix cores, one band of rows per work-group (Q4_K at
 // 14336 x 4096: 19.2-19.7 us for every M in 4..16, against 21-30 us on the
@@ -765,12 +824,9 @@ int run_band(uint32_t dtype, const Geometry& g, const float* x, const Mats& ms, 
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     hipError_t e = hipSuccess;
     const bool pair = ms.mm == fq::MM_PAIR;
-    int tiles = band_tiles(dtype, K, N, di.cus);
-    if (pair) tiles = tiles >= 4 ? 4 : 2;
-    int rpw = 0;
-    const int splits = mmqs_plan(pair ? 2 * N : N, K, di.cus, &rpw, tiles);
-    if (pair) rpw = 16 * ((rpw / 16 + 1) / 2);  // gate rows of a band, as many up rows
-    const size_t need = mmqs_need(M, K, N, di.cus, tiles);
+    const BandPlan bp = band_plan(dtype, K, N, pair, di.cus);
+    const int rpw = bp.rpw, splits = bp.splits;
+    const size_t need = mmqs_need(M, K, N, di.cus, bp.tiles);
     std::unique_ptr<StreamScratch::Lease> lease;
     uint8_t* buf = fixed;
     if (fixed) {
@@ -891,9 +947,25 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
         if (rc != FQ_ERR_SHAPE) return rc;
     }
 
+    const BandRule rule = band_rule(dtype, g, M, K, N, w, di.cus);
     if (thin_takes(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {
-        const int rc = run_thin(dtype, g, x, Mats{fq::MM_ONE, {w}, {N}}, bias, bias_mode, bias_len, y, M,
-                                K, N, dev, di, st, fixed, fixed_cap);
+        // (where bands fill their rounds the band kernel is faster: at M = 8 Q5_0 12288
+        // x 4096 16.7 us there, 20.6 here, 14336 x 4096 20.5 and 20.9; Q4_0 12288 x 5632
+        // 19.6 and 23.1, 13824 x 5632 23.3 and 23.6, 17408 x 5632, two rounds, 33.4 and 25.7)
+        const double limit = M <= 16 && K < 32 * 256 && rule.takes
+                                 ? 1.04 * band_us(dtype, g, K, N, false, di.cus)
+                                 : HUGE_VAL;
+        const Mats ms{fq::MM_ONE, {w}, {N}};
+        int rc = run_thin(dtype, g, x, ms, bias, bias_mode, bias_len, y, M, K, N, dev, di, st, fixed,
+                          fixed_cap, limit);
+        if (rc == kSlower) {
+            rc = run_band(dtype, g, x, ms, bias, bias_mode, bias_len, y, M, K, N, dev, di, st, fixed,
+                          fixed_cap, x_ready);
+            if (rc == FQ_OK && band_x) *band_x = true;
+            if (rc == FQ_ERR_WORKSPACE)  // capture on a workspace that another call sized
+                rc = run_thin(dtype, g, x, ms, bias, bias_mode, bias_len, y, M, K, N, dev, di, st,
+                              fixed, fixed_cap, HUGE_VAL);
+        }
         if (rc != kNotTaken) return rc;
     }
 
@@ -917,7 +989,6 @@ int run_matmul(uint32_t dtype, const float* x, const void* w, const float* bias,
         return FQ_OK;
     }
 
-    const BandRule rule = band_rule(dtype, g, M, K, N, w, di.cus);
     if (M >= 2 && M <= 4 && !rule.block && K > 0 && packable(dtype) &&
         (dtype == FQ_DTYPE_Q6_K || (int64_t)N * (K / g.be) * g.bb >= (8 << 20))) {
         // two to four tokens: the same kernel dots each weight unit it reads
@@ -1525,7 +1596,7 @@ int fq_fused_qkv(uint32_t dtype, const float* x, const void* wq, const void* wk,
         if (M > 32)
             rc = run_prefill(dtype, g, x, ms, nullptr, 0, 0, y, M, K, Nt, dev, di, st, nullptr, 0);
         else if (thin_takes(dtype, M, 0))
-            rc = run_thin(dtype, g, x, ms, nullptr, 0, 0, y, M, K, Nt, dev, di, st, nullptr, 0);
+            rc = run_thin(dtype, g, x, ms, nullptr, 0, 0, y, M, K, Nt, dev, di, st, nullptr, 0, HUGE_VAL);
         if (rc != kNotTaken) return rc;
     }
     if (M >= 5 && M <= 16 && K < 32 * 256) {
@@ -1622,15 +1693,24 @@ int fq_ffn_up_fused(uint32_t dtype, const float* x, const void* w_gate, const vo
     }
     if (M > 1 && M <= 32) {  // gate and up rows in one launch
         const Mats ms{fq::MM_PAIR, {w_gate, w_up}, {N}};
-        int rc = kNotTaken;
-        if (!thin_takes_pair(dtype, M, (int64_t)N * (K / g.be) * g.bb) && M >= 5 && K < 32 * 256 &&
-            band_rule(dtype, g, M, K, N, w_gate, di.cus).takes &&
-            band_rule(dtype, g, M, K, N, w_up, di.cus).takes) {  // K unsplit
+        const int64_t bytes = (int64_t)N * (K / g.be) * g.bb;
+        const bool band = M >= 5 && M <= 16 && K < 32 * 256 &&  // K unsplit
+                          band_rule(dtype, g, M, K, N, w_gate, di.cus).takes &&
+                          band_rule(dtype, g, M, K, N, w_up, di.cus).takes;
+        // 5..16 tokens: the band kernel where it is estimated faster, for matrices that
+        // it takes one by one unless 10 % slower (M = 8: Q4_1 9472 x 5632 42.9 us there,
+        // 28.0 here, Q5_0 9472 x 4096 35.7 and 28.2); what it does not take here too
+        const bool thin = thin_takes_pair(dtype, M, bytes);
+        const double limit =
+            band ? (thin_takes(dtype, M, bytes) ? 1.04 : 0.9) * band_us(dtype, g, K, N, true, di.cus)
+                 : HUGE_VAL;
+        auto run = [&](double us) {
+            return run_thin(dtype, g, x, ms, nullptr, 0, 0, y, M, K, N, dev, di, st, nullptr, 0, us);
+        };
+        int rc = thin || (M >= 5 && !band) ? run(limit) : kNotTaken;
+        if (band && (rc == kSlower || rc == kNotTaken)) {
             rc = run_band(dtype, g, x, ms, nullptr, 0, 0, y, M, K, N, dev, di, st, nullptr, 0, false);
-            if (rc == FQ_ERR_WORKSPACE) rc = kNotTaken;
-        } else if (M >= 5 || thin_takes_pair(dtype, M, (int64_t)N * (K / g.be) * g.bb)) {
-            // (5..16 tokens that the band kernel does not take: here too)
-            rc = run_thin(dtype, g, x, ms, nullptr, 0, 0, y, M, K, N, dev, di, st, nullptr, 0);
+            if (rc == FQ_ERR_WORKSPACE) rc = run(HUGE_VAL);  // capture on what another call sized
         }
         if (rc != kNotTaken) return rc;
     }

@@ -140,3 +140,17 @@ def test_q6k_four_tokens_on_many_rows():
     W = dev_weight(F.Q6_K, synth.make_weights(F.Q6_K, N, K, 90), N, K)
     x = torch.from_numpy(synth.make_x(5, K, seed=91)).cuda()
     assert torch.equal(ops.matmul_transB(x[:4], W), ops.matmul_transB(x, W)[:4])
+
+
+# Sizes on both sides of the line between this kernel and the band kernel, whose
+# bands fill their rounds up to 16384 rows: one row more or less, other counts of tiles
+@pytest.mark.parametrize("dtype", ALL)
+@pytest.mark.parametrize("M,N,K", [(4, 12288, 4096), (8, 12289, 4096), (16, 16385, 2816), (5, 8200, 5632)])
+def test_band_or_shared_operands(dtype, M, N, K):
+    test_shapes(dtype, M, N, K)
+
+
+@pytest.mark.parametrize("dtype", ALL)
+@pytest.mark.parametrize("M,N,K", [(5, 1001, 256), (8, 6400, 2048), (16, 12289, 3584), (3, 16385, 1024)])
+def test_pair_band_or_shared_operands(dtype, M, N, K):
+    test_gate_up_pair(dtype, M, N, K)

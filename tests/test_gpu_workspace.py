@@ -247,3 +247,41 @@ def test_capture_of_fewer_tokens_than_warmed_up(op, dtype, Mw, M, K, ns):
         torch.cuda.synchronize()
     del g
     assert L.fq_release_workspace(side.cuda_stream) == 0
+
+
+# Calls whose kernel an estimate chooses (band or shared operands), first
+# under capture on a workspace that a call of other tokens sized: where the chosen
+# one does not fit, another runs.  Each within 1e-6 of the exact result.
+@pytest.mark.parametrize("op,dtype,Mw,M,K,ns", [
+    ("pair", F.Q4_0, 2, 8, 2048, (6400, 6400)), ("pair", F.Q6_K, 2, 5, 256, (4096, 4096)),
+    ("pair", F.Q5_0, 2, 8, 3584, (9472, 9472)), ("one", F.Q4_K, 17, 4, 4096, (11008,)),
+    ("one", F.Q4_0, 17, 8, 5632, (12288,)), ("one", F.Q5_0, 17, 4, 4096, (12288,))])
+def test_capture_where_estimates_choose(op, dtype, Mw, M, K, ns):
+    from forge_amd import ops
+    L = _lib.lib()
+    if op == "one":
+        W = ops.QWeight.from_numpy(synth.make_weights(dtype, ns[0], K, 140), dtype, ns[0], K, device="cuda")
+        run = lambda x: ops.matmul_transB(x, W)  # noqa: E731
+    else:
+        run = _fused(op, dtype, K, ns)
+    x = torch.from_numpy(synth.make_x(max(Mw, M), K, 141) * np.float32(1e-2)).cuda()
+    ref = run(x[:M])
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        run(x[:Mw])
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        y = run(x[:M])
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert float((y - ref).norm() / ref.norm()) < 2e-6
+        with torch.cuda.stream(side):
+            assert torch.equal(run(x[:M]), ref)
+        torch.cuda.synchronize()
+    del g
+    assert L.fq_release_workspace(side.cuda_stream) == 0
